@@ -697,7 +697,7 @@ extern "C" int qtts_gemm_q4(qtts_ctx *c, const qtts_w *w, const float *X, int64_
 {
     if (!c || !w || !X || !Y || rows < 0) return QTTS_ERR_INVALID;
     if (rows == 0) return QTTS_OK;
-    RCHK(ensure_io(c, std::max<int64_t>(rows * w->t.k, rows * w->t.npad)));
+    RCHK(ensure_io(c, rows * std::max({w->t.k, w->t.n, w->t.npad})));
     RCHK(stage_in(c, X, rows * w->t.k, c->d_io, flags));
     HIPCHK(c, hipMemsetAsync(c->d_io2, 0, rows * w->t.n * sizeof(float), c->stream));
     if (use_mfma(flags, rows) && gemm_supported(w->t)) {
