@@ -635,7 +635,8 @@ int qtts_time_decode(qtts_ctx *ctx, int64_t n_frames, int32_t iters,
  * measurement helper so a caller can see what the upload-time tables cost
  * against the weights they stand in for. */
 typedef struct {
-    int64_t talker_q4;            /* talker Q4 tiles: layers, codec head, text projection */
+    int64_t talker_q4;            /* talker Q4 tiles: layers, codec head, text projection (the prefill's
+                                     copy of the layers, as large again, shows in device_used) */
     int64_t predictor_q4;         /* predictor Q4 tiles: layers, lm heads, input projection */
     int64_t predictor_row_tables; /* projected code-embedding rows of steps 1..14 (f32), 0 if off */
     int64_t predictor_qkv_tables; /* their layer-0 q|k|v rows (f32), 0 if off */

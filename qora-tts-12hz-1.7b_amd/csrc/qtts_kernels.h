@@ -30,10 +30,42 @@ struct KvPaged {
     int32_t n_phys;
 };
 
+// A Q4 weight in the matrix cores' fragment order (layout in qtts_gemm.hip):
+// one record of `rec` bytes per (32-column group, 64 rows of k).
+struct Q4Frag {
+    const uint8_t *data;   // null: the weight takes the f32 matrix path
+    int32_t k, kc;         // rows, chunks of 64 rows
+    int32_t ng;            // 32-column groups
+    int32_t dual;          // 1: gate|up paired by 16 columns
+    int32_t rec, bshift;
+};
+
+// GEMM rows split into f16 hi + lo (layout in qtts_gemm.hip), and what undoes
+// their staging: a factor per row (rseg 0), per row and 256 or 64 columns
+// (rseg floats between the column slots), or one for all (rsc null).
+struct RowsSplit {
+    const uint8_t *p;
+    int32_t kc, M;
+    const float *rsc;
+    int32_t rseg;
+    float ufac;
+};
+
+// Partial sums of a projection: part i of element e at p[i * stride + e],
+// `per` consecutive parts make a slice (parts in order within a slice, then
+// slices in order).
+struct MmParts {
+    const float *p;
+    int32_t ld;            // floats per row
+    size_t stride;
+    int32_t n, per;
+};
+
 // One decoder layer on the device.  q|k|v and gate|up are fused along the
 // output dimension (columns [q | k | v], [gate | up]).
 struct LayerDev {
     Q4Tiled qkv, o, gate_up, down;
+    Q4Frag qkv_f, o_f, gate_up_f, down_f;   // talker layers: the prefill's copies
     const uint16_t *q_norm, *k_norm, *input_norm, *post_norm;
     // matrix-core prefill: the staging powers of two (shift = 14 -
     // ceil(log2(bound))) of the normed rows (bound sqrt(hidden) * max|gamma|
@@ -48,6 +80,7 @@ struct TalkerDev {
     int n_layers, hidden, text_hidden, n_heads, n_kv_heads, inter, vocab;
     const LayerDev *layers;              // host array [n_layers]
     Q4Tiled codec_head, text_fc1, text_fc2;
+    Q4Frag text_fc1_f, text_fc2_f;
     const float *text_fc1_bias, *text_fc2_bias;
     Q4Rows codec_rows, text_rows;        // embedding tables, reference layout
     const uint16_t *final_norm;
@@ -103,12 +136,13 @@ struct Workspace {
 // Buffers of the batched prefill, rows of one prompt chunk.
 struct PrefillWs {
     float *x;          // residual rows [cap_rows][hidden]
+    float *xs;         // the normed rows, split [cap_rows][hidden up to 64s]
     float *q;          // normed + roped q rows [cap_rows][16*128]
-    float *attn;       // attention rows [cap_rows][16*128]
-    float *h;          // silu(gate)*up rows [cap_rows][inter]
-    float *part;       // k-slice partial sums of a projection [cap_rows * prefill_part_floats]
-    float *inv;        // per-row 1/rms [cap_rows]
-    float *rmax;       // per-row largest |x| of a GEMM input by column slots [cap_rows][prefill_rmax_slots]
+    float *attn;       // attention rows [cap_rows][16*128], f32 or split
+    float *h;          // silu(gate)*up rows [cap_rows][inter up to 64s], f32 or split
+    float *part;       // partial sums of a projection (prefill_part_floats(cap_rows))
+    float *inv;        // per-row 1/rms [cap_rows] (f32 matrix path)
+    float *rsc;        // per-row factors of a split GEMM input by column slots [prefill_rsc_slots][cap_rows]
     int cap_rows;
 };
 
@@ -246,14 +280,29 @@ hipError_t enqueue_pred_row_tables(const PredictorDev &p, int n_tables, float *X
                                    hipStream_t s);
 bool pred_qkv_tables_supported(const PredictorDev &p);
 hipError_t enqueue_pred_qkv_tables(const PredictorDev &p, int n_tables, float *part, float *out, hipStream_t s);
-bool gemm_supported(const Q4Tiled &w);
-hipError_t enqueue_gemm_rows(const Q4Tiled &w, const float *X, int rows, float *Y, int ldy, float *rmax,
+bool frag_supported(const Q4Tiled &w);
+size_t frag_shape(const Q4Tiled &w, Q4Frag *f);
+hipError_t enqueue_frag_build(const Q4Tiled &w, const Q4Frag &f, uint8_t *out, hipStream_t s);
+hipError_t enqueue_split_rows(const float *X, int ld, int M, int K, int seg, uint8_t *out, int kc, float *rsc,
+                              int ldr, hipStream_t s);
+size_t mm_part_floats(const Q4Frag &w, int M, bool fp1);
+size_t mm_swiglu_part_floats(const Q4Frag &w, int M);
+hipError_t enqueue_mm_parts(const RowsSplit &a, const Q4Frag &w, bool fp1, float *part, MmParts *p, hipStream_t s);
+hipError_t enqueue_mm_swiglu(const RowsSplit &a, const Q4Frag &w, float *part, uint8_t *rows, int okc, float *rsc,
                              hipStream_t s);
-hipError_t enqueue_gemm_bias(const Q4Tiled &w, const float *X, int rows, const float *bias, bool silu, float *Y,
-                             int ldy, float *rmax, hipStream_t s);
+hipError_t enqueue_mm_rows(const Q4Frag &w, const float *X, int ld, int rows, const float *bias, bool silu, float *Y,
+                           int ldy, float *ws, size_t ws_floats, hipStream_t s);
+size_t mm_rows_ws_floats(const Q4Frag &w, int M);
+// The split-f16 contraction unless QTTS_GEMM_F32=1 (f32 matrix instructions).
+bool gemm_x3();
+bool gemm_supported(const Q4Tiled &w);
+hipError_t enqueue_gemm_rows(const Q4Tiled &w, const Q4Frag &f, const float *X, int rows, float *Y, int ldy, float *ws,
+                             size_t ws_floats, hipStream_t s);
+hipError_t enqueue_gemm_bias(const Q4Tiled &w, const Q4Frag &f, const float *X, int rows, const float *bias, bool silu,
+                             float *Y, int ldy, float *ws, size_t ws_floats, hipStream_t s);
 bool prefill_supported(const TalkerDev &m);
-int64_t prefill_part_floats(const TalkerDev &m);
-int64_t prefill_rmax_slots(const TalkerDev &m);
+int64_t prefill_part_floats(const TalkerDev &m, int rows);
+int64_t prefill_rsc_slots(const TalkerDev &m);
 int norm_shift(const uint16_t *gamma_host, int n);
 int bound_shift(double bound);
 int attn_shift(double bound);
@@ -264,7 +313,7 @@ hipError_t enqueue_codec_frame_rows(const Q4Rows &tcodec, const Q4Rows &pemb, in
 hipError_t enqueue_add_rows(const float *a, int lda, const float *b, int ldb, float *out, int ldo, int rows, int n,
                             hipStream_t s);
 hipError_t enqueue_fill_rows(float *x, int64_t n, uint32_t seed, hipStream_t s);
-hipError_t enqueue_row_inv(const float *X, int ld, int M, int K, float *inv, hipStream_t s);
+hipError_t enqueue_gateup_input(const TalkerDev &m, const PrefillWs &pw, int l, int M, hipStream_t s);
 hipError_t enqueue_gemm_gateup(const TalkerDev &m, const PrefillWs &pw, int l, int M, hipStream_t s);
 hipError_t enqueue_talker_prefill(const TalkerDev &m, const PrefillWs &pw, int M, int64_t start,
                                   float *hidden_out, hipStream_t s);

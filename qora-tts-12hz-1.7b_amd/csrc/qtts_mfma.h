@@ -137,6 +137,64 @@ __device__ __forceinline__ int range_shift(float mx)
     return max(-100, min(100, 15 - e));
 }
 
+// Sum of a projection's parts at element `at` (MmParts: parts in order within
+// a slice, then the slices in order).  NP > 0: exactly p.n parts, every load
+// issued before the first addition; 0: any count.
+template <int NP, class V>
+__device__ __forceinline__ V sum_parts_v(const MmParts &p, size_t at)
+{
+    if constexpr (NP > 0) {
+        V v[NP];
+#pragma unroll
+        for (int i = 0; i < NP; i++) v[i] = *(const V *)(p.p + (size_t)i * p.stride + at);
+        V tot = v[0], sv = v[0];
+        bool any = false;
+#pragma unroll
+        for (int i = 1; i < NP; i++) {
+            if (i % p.per == 0) {
+                tot = any ? tot + sv : sv;
+                any = true;
+                sv = v[i];
+            } else {
+                sv += v[i];
+            }
+        }
+        return any ? tot + sv : sv;
+    } else {
+        V tot{}, sv = *(const V *)(p.p + at);
+        bool any = false;
+        for (int i = 1; i < p.n; i++) {
+            const V x = *(const V *)(p.p + (size_t)i * p.stride + at);
+            if (i % p.per == 0) {
+                tot = any ? tot + sv : sv;
+                any = true;
+                sv = x;
+            } else {
+                sv += x;
+            }
+        }
+        return any ? tot + sv : sv;
+    }
+}
+template <int NP>
+__device__ __forceinline__ float sum_parts(const MmParts &p, size_t at) { return sum_parts_v<NP, float>(p, at); }
+template <int NP>
+__device__ __forceinline__ f32x4 sum_parts4(const MmParts &p, size_t at) { return sum_parts_v<NP, f32x4>(p, at); }
+
+// F<n>::go(args...) for a launch over n parts (0: the instance for any count).
+template <template <int> class F, class... A>
+static hipError_t by_parts(int n, const A &...args)
+{
+    switch (n) {
+    case 1: return F<1>::go(args...);
+    case 2: return F<2>::go(args...);
+    case 4: return F<4>::go(args...);
+    case 6: return F<6>::go(args...);
+    case 8: return F<8>::go(args...);
+    default: return F<0>::go(args...);
+    }
+}
+
 // The double-buffered schedule over nch >= 1 chunks.  fetch(f, c) issues
 // chunk c's global loads into register set f, stage(f, buf) writes a
 // register set into LDS buffer buf, mma(buf) runs the MFMAs of buffer buf.

@@ -1,28 +1,25 @@
 // qtts_prefill.hip — batched talker prefill for long prompts on the matrix
 // cores (prefill_talker_raw_from, talker.rs:379-482).
 //
-// A prompt of M rows runs layer by layer (k_row_inv first: 1/rms of every
-// input row, gemv.rs:445-454): per layer
-//   k_gemm_q4 (parts)    [M x 2048] x [2048 x 4096] q|k|v,   talker.rs:392-400
-//                        input norm fused, 3 k-slices
-//   k_prefill_qkv_post   slices summed, QK-norm, RoPE,       talker.rs:402-425
+// A prompt of M rows runs layer by layer (k_resid_norm first: the input rows
+// normed and split): per layer
+//   k_q4_gemm (parts)    [M x 2048] x [2048 x 4096] q|k|v    talker.rs:392-400
+//   k_prefill_qkv_post   parts summed, QK-norm, RoPE,        talker.rs:402-425
 //                        K/V append
-//   k_prefill_attn_mx    causal attention over the cache     talker.rs:427-458
-//   k_gemm_q4 (parts)    attn x o_proj, 6 k-slices           talker.rs:460
-//   k_resid_add_inv      x += slices; post-attention 1/rms   talker.rs:461-468
-//   k_gemm_q4 (swiglu)   silu(gate) * up, gate|up fused,     talker.rs:470-474
-//                        post-attention norm fused
-//   k_gemm_q4 (parts)    h x down_proj, 6 k-slices           talker.rs:475
-//   k_resid_add_inv      x += slices; next layer's 1/rms     talker.rs:476
+//   k_prefill_attn_mx    causal attention over the cache,    talker.rs:427-458
+//                        its rows split for the o-projection
+//   k_q4_gemm (parts)    attn x o_proj                       talker.rs:460
+//   k_resid_norm         x += parts; post-attention norm,    talker.rs:461-468
+//                        the normed rows split
+//   k_q4_gemm (swiglu)   silu(gate) * up, split              talker.rs:470-474
+//   k_q4_gemm (parts)    h x down_proj                       talker.rs:475
+//   k_resid_norm         x += parts; next layer's norm       talker.rs:476
 // then k_final_rms on the last row (talker.rs:477-481).
 //
-// k_gemm_q4 contracts f32 operands with f32 accumulation, the arithmetic
-// the reference's gemm_q4 (gemv.rs:349-412) does on the CPU: by default on
-// the f16 matrix cores with every operand split into f16 hi + lo (three
-// products, f32-accurate; see X3 below), or on v_mfma_f32_16x16x4_f32
-// (QTTS_GEMM_F32=1).  The weight is read from the same tiled Q4 layout the
-// decode GEMV streams (no second copy in HBM) and dequantised into LDS once
-// per row tile of the prompt.
+// k_q4_gemm (qtts_gemm.hip) contracts on the f16 matrix cores with split
+// operands, f32-accurate.  With QTTS_GEMM_F32=1, or for a layer weight whose
+// scales leave the split's range, the prompt runs on k_gemm_q4 below instead:
+// f32 rows, v_mfma_f32_16x16x4_f32, the decode GEMV's tiled weights.
 
 #include "qtts_device.h"
 #include "qtts_kernels.h"
@@ -35,32 +32,8 @@
 namespace qtts {
 
 // ---------------------------------------------------------------------------
-// per-row 1/rms (rms_norm_f16, gemv.rs:445-454): inv = 1 / sqrt(sum x^2 / K
-// + 1e-6).  One wave per row.
-// ---------------------------------------------------------------------------
-
-__global__ void __launch_bounds__(256)
-k_row_inv(const float *X, int ld, int M, int K, float *inv)
-{
-    const int lane = threadIdx.x & 63;
-    const int m = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (m >= M) return;
-    const float *x = X + (size_t)m * ld;
-    float s = 0.0f;
-    for (int k = lane * 4; k < K; k += 256) {
-        const f32x4 v = ld4(x + k);
-        s = fmaf(v.x, v.x, s);
-        s = fmaf(v.y, v.y, s);
-        s = fmaf(v.z, v.z, s);
-        s = fmaf(v.w, v.w, s);
-    }
-    s = wave_sum_dpp(s);
-    if (lane == 0) inv[m] = 1.0f / sqrtf(s / (float)K + 1e-6f);
-}
-
-// ---------------------------------------------------------------------------
-// Q4 GEMM on the matrix cores: Y[M][n] (op)= A'[M][K] x W[K][n], with
-// A' = A * inv[row] * gamma[k] when a norm is fused (the reference's
+// Q4 GEMM on the f32 matrix instructions: Y[M][n] (op)= A'[M][K] x W[K][n],
+// with A' = A * inv[row] * gamma[k] when a norm is fused (the reference's
 // x * inv_rms * gamma order) and W dequantised as (nibble - 8) * scale,
 // exact in f32.
 //
@@ -90,14 +63,6 @@ struct GemmA {
     const float *inv;        // per-row 1/rms, or null
     const uint16_t *gamma;   // [K] f16, or null
     int M;
-    // The range of the split-f16 staging (X3).  Rows without a norm: rmax
-    // [M][rslots] holds the largest |A| of each row over slots of rw columns
-    // (slot s: k in [s rw, (s+1) rw)), or is null (rows staged as they are).
-    // Rows with a norm: nshift, a power of two that takes the bound of
-    // |x * inv * gamma| (sqrt(K) * max|gamma|) into [2^13, 2^14].
-    const float *rmax;
-    int rslots, rw;
-    int nshift;
 };
 
 struct GemmOut {
@@ -105,85 +70,20 @@ struct GemmOut {
     int ldy, ncols;
     const float *bias;       // GEMM_BIAS*: [ncols]
     size_t slice_stride;     // GEMM_PART: floats between the slices' blocks
-    float *rmax;             // GEMM_SWIGLU: largest |output| per (row, 64-column tile) [rows][rslots], or null
-    int rslots;
 };
 
-// Address of the 16-byte word and the scale of (row k, group g) in the
-// tiled layout built by the runtime (qtts_device.h).
-__device__ __forceinline__ void tiled_word(const Q4Tiled &w, TileShape ts, int k, int g, const uint8_t *&word,
-                                           const uint16_t *&scale)
-{
-    const int P = ts.T / ts.GB;
-    const int s = k / w.KC, rr = k - s * w.KC, r = rr / P, pt = rr - r * P;
-    const int ct = g / ts.GB, gt = g - ct * ts.GB;
-    const bool wave_groups = (ts.T / 64) % ts.GB == 0;
-    const int t = wave_groups ? ((pt >> 6) * ts.GB + gt) * 64 + (pt & 63) : pt * ts.GB + gt;
-    const uint8_t *tile = w.data + (size_t)(s * w.CT + ct) * w.tile_bytes;
-    word = tile + ((size_t)r * ts.T + t) * 16;
-    scale = (const uint16_t *)(tile + (size_t)ts.R * ts.T * 16) + t * ts.R + r;
-}
-
-// X3: the contraction on v_mfma_f32_16x16x32_f16 in three products per
-// pair of operands.  Each staged value v is split into hi = f16(v) and
-// lo = f16(v - hi): hi + lo carries 22 bits of v's 24, and a dequantised
-// weight (a 4-bit integer times an f16 scale, 15 significant bits) is
-// exactly hi + lo.  acc += Ahi Bhi + Ahi Blo + Alo Bhi (f32 accumulation,
-// the products exact); the dropped Alo Blo is below 2^-22 of each term.
-// Per chunk of 32 that is 3 matrix instructions of 8192 multiply-adds
-// where the f32 path issues 8 of 1024.  The staged tiles are f16 rows of
-// HLD halves (80 bytes: a lane's 16-byte read of 8 halves at 16q bytes).
-constexpr int HLD = MFMA_HLD;
 // word 3 of a raw buffer descriptor on this GPU family (untyped dword
 // access, no swizzle, offsets checked against the record count in bytes)
 constexpr int BUF_RSRC_W3 = 0x00020000;
-// The B tile's 16-column blocks are BPAD halves apart beyond their rows, so
-// the four 8-column groups a wave writes at once (8 rows = 160 dwords apart
-// otherwise: the same banks two by two) start on banks 0, 32, 16, 48.
-constexpr int BPAD = 32;
 
-// (w & m) | o, kept opaque so the masked word is consumed as two f16 halves
-__device__ __forceinline__ uint32_t and_or_opaque(uint32_t w, uint32_t m, uint32_t o)
-{
-    uint32_t r;
-    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(w), "v"(m), "s"(o));   // one scalar operand (VOP3)
-    return r;
-}
-
-// x * g with g the low (HI = 0) or high f16 half of a register: one
-// v_fma_mix_f32 with a -0 addend, the product rounded once to f32 as a
-// multiply rounds it (sign of a zero product kept)
-template <int HI>
-__device__ __forceinline__ float mul_f16_half(uint32_t g, float x, float nz)
-{
-    float r;
-    if constexpr (HI)
-        asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(g), "v"(x), "v"(nz));
-    else
-        asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(g), "v"(x), "v"(nz));
-    return r;
-}
-
-template <int MB, int EPI, bool NORM, bool X3>
+template <int MB, int EPI, bool NORM>
 __global__ void __launch_bounds__(256, 2)
 k_gemm_q4(GemmA a, Q4Tiled w, GemmOut o, int tm, int S)
 {
     constexpr int BM = 16 * MB;
     constexpr int NA = (BM * GK / 4 + 255) / 256;   // 16-byte A slots per thread
-    constexpr int XSTRIDE = BM * HLD + GN * HLD + (GN / 16) * BPAD;   // halves per (buffer, half) on X3
-    constexpr int F32_BYTES = 2 * (BM + GN) * GLD * 4, X3_BYTES = 2 * 2 * XSTRIDE * 2;
-    constexpr int TILE_BYTES = X3 ? X3_BYTES : F32_BYTES;
-    // one LDS block: the staging tiles first (their bank layout assumes the
-    // block's base), then the per-row factors that undo the staging scales
-    // (X3) and the SwiGLU epilogue's per-wave row maxima
-    __shared__ __attribute__((aligned(16))) unsigned char lds[TILE_BYTES + BM * 4 + 4 * BM * 4];
-    float *rsc = (float *)(lds + TILE_BYTES);
-    float(*wmx)[BM] = (float(*)[BM])(lds + TILE_BYTES + BM * 4);
-    // f32: As[2][BM*GLD], Bs[2][GN*GLD]; X3: per buffer Ah, Al [BM*HLD] and Bh, Bl [GN*HLD]
-    float(*As)[BM * GLD] = (float(*)[BM * GLD])lds;
-    float(*Bs)[GN * GLD] = (float(*)[GN * GLD])(lds + 2 * BM * GLD * 4);
-    const auto xa = [&](int buf, int hl) { return (_Float16 *)lds + (size_t)(buf * 2 + hl) * XSTRIDE; };
-    const auto xb = [&](int buf, int hl) { return xa(buf, hl) + (size_t)BM * HLD; };
+    __shared__ __attribute__((aligned(16))) float As[2][BM * GLD];
+    __shared__ __attribute__((aligned(16))) float Bs[2][GN * GLD];
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
     // Workgroups are dealt round-robin to the 8 XCDs: give each XCD a
     // contiguous run of tiles (row blocks fastest) so the row blocks that
@@ -201,108 +101,45 @@ k_gemm_q4(GemmA a, Q4Tiled w, GemmOut o, int tm, int S)
 
     // A staging: slot i = t + 256 j (clamped: spare threads repeat the last
     // slot) covers row i / 8, floats 4 (i % 8)..+4 of the chunk.  Rows past
-    // M load row M-1 and stage zeros.  On X3 the rows of each 16-row block
-    // are taken in 4 x 4 transposed order, so the 4 rows of one 32-lane
-    // half of a write are 4 apart (80 dwords: disjoint bank ranges).
-    // aoffg: byte offset of the slot in A, unsigned 32 bits, so each load
-    // takes the chunk's wave-uniform base in scalar registers plus this
-    // X3 range: row r is staged times 2^sh(r), sh chosen so that the row's
-    // largest |value| over this slice's columns lies in [2^14, 2^15) (from
-    // rmax) or below the norm's static bound (nshift); the f16 halves then
-    // neither overflow nor go subnormal where the value is not tiny against
-    // the row.  The sums are scaled back by 2^-(sh + bshift) per row in the
-    // epilogue.  Both scalings are exact.  The loads the staging factors need
-    // (1/rms, the rows' slots) are issued here and used in `pre`, after the
-    // first chunk's loads are issued: waiting for them does not hold those
-    // back.
+    // M load row M-1 and stage zeros.
     uint32_t aoffg[NA];
-    int aoff[NA], akk[NA], arow[NA];
-    float amul[NA], ainv[NA];
-    float arv[NA][2];               // two of the row's slots over this slice (rows without a norm, X3)
-    const int s0 = a.rmax ? (c0 * GK) / a.rw : 0, s1 = a.rmax ? (c1 * GK - 1) / a.rw : 0;
-    // A row's 8 slots of a chunk sit in 8 consecutive lanes (8 | 256, and the
-    // clamped slots fill whole groups of 8): lane e8 of the group reads the
-    // row's slots s0 + 2 e8 and s0 + 2 e8 + 1 (the launcher checks that a
-    // slice spans at most 16), and the group takes their maximum by DPP
-    const int e8 = t & 7;
+    int aoff[NA], akk[NA];
+    float amul[NA];
 #pragma unroll
     for (int j = 0; j < NA; j++) {
         const int slot = min(t + 256 * j, BM * GK / 4 - 1);
-        const int rr = slot >> 3;
-        const int r = X3 ? (rr & ~15) | ((rr & 3) << 2) | ((rr >> 2) & 3) : rr, m = m0 + r;
+        const int r = slot >> 3, m = m0 + r;
         aoffg[j] = (uint32_t)(min(m, a.M - 1) * a.lda + 4 * (slot & 7)) * 4u;
         aoff[j] = r * GLD + 4 * (slot & 7);
         akk[j] = 4 * (slot & 7);
-        arow[j] = (slot & 7) == 0 ? r : -1;      // the thread that records the row's factor
-        ainv[j] = NORM ? a.inv[min(m, a.M - 1)] : 1.0f;
-        if constexpr (X3 && !NORM) {
-            if (a.rmax) {
-                const float *rp = a.rmax + (size_t)min(m, a.M - 1) * a.rslots;
-#pragma unroll
-                for (int u = 0; u < 2; u++) {
-                    const int sl = s0 + 2 * e8 + u;
-                    const float v = rp[min(sl, s1)];
-                    arv[j][u] = sl <= s1 ? v : 0.0f;
-                }
-            }
-        }
+        amul[j] = m < a.M ? (NORM ? a.inv[m] : 1.0f) : 0.0f;
     }
-    auto pre = [&]() {
-#pragma unroll
-        for (int j = 0; j < NA; j++) {
-            const int m = m0 + (aoff[j] / GLD);
-            int sh = 0;
-            if constexpr (X3) {
-                if (NORM) {
-                    sh = a.nshift;
-                } else if (a.rmax) {
-                    float mx = fmaxf(arv[j][0], arv[j][1]);
-                    mx = fmaxf(mx, dpp_mov<0xB1>(mx));    // lane ^ 1
-                    mx = fmaxf(mx, dpp_mov<0x4E>(mx));    // lane ^ 2
-                    mx = fmaxf(mx, dpp_mov<0x141>(mx));   // the other quad of the 8 (half-row mirror)
-                    sh = range_shift(mx);
-                }
-            }
-            const float p2 = __builtin_ldexpf(1.0f, sh);
-            amul[j] = m < a.M ? (NORM ? ainv[j] * p2 : p2) : 0.0f;
-            if (arow[j] >= 0) rsc[arow[j]] = __builtin_ldexpf(1.0f, -(sh + (X3 ? w.bshift : 0)));
-        }
-    };
-    // B staging: bytes 4*qw..+4 (8 columns) of the tiled rows; groups past
-    // G stage zeros.  f32: row kr of groups 4*nt + gi and + 2.  X3: rows kr
-    // and kr + 1 of group 4*nt + gi (one wave per group), so the two rows'
-    // values of a column leave as one 4-byte LDS write.
-    const int kr = X3 ? 2 * (t & 15) : (t & 31);
-    const int qw = X3 ? (t >> 4) & 3 : (t >> 5) & 3;
-    // gi is the same across a wave: read it as a scalar, so the tile
-    // addresses below come from the scalar unit
-    const int gi = __builtin_amdgcn_readfirstlane(X3 ? t >> 6 : t >> 7);
+    // B staging: bytes 4*qw..+4 (8 columns) of row kr of groups 4*nt + gi
+    // and + 2; groups past G stage zeros.  gi is the same across a wave: read
+    // as a scalar, so the tile addresses below come from the scalar unit.
+    const int kr = t & 31, qw = (t >> 5) & 3;
+    const int gi = __builtin_amdgcn_readfirstlane(t >> 7);
     int gt[2], gct[2];
     bool gok[2];
 #pragma unroll
     for (int h = 0; h < 2; h++) {
-        const int g = 4 * nt + gi + (X3 ? 0 : 2 * h);
+        const int g = 4 * nt + gi + 2 * h;
         gok[h] = g < w.G;
         const int gc = min(g, w.G - 1);
         gct[h] = gc / ts.GB;
         gt[h] = gc - gct[h] * ts.GB;
     }
-
-    // X3: the weights are staged times 2^bshift (their split's low half a
-    // normal f16) and the sums scaled back by 2^-bshift (both exact)
-    const float bscale = X3 ? __builtin_ldexpf(1.0f, w.bshift) : 1.0f;
-
     // tile position of (pt, group): one group per wave when wave_groups,
     // else groups interleaved by thread -- one formula for both
     const int tA = wave_groups ? 1 : ts.GB, tB = wave_groups ? 64 : 1;
     // With P >= 32 (every tile but 8 groups x 128 threads) a chunk's 32 rows
     // lie in one tile row r0 and one 64-position block (pt0 is a multiple of
-    // 32), so tt = ttu(k0) + (kr [+ h]) * tA + gt * tB: a wave-uniform part
-    // per chunk and this constant thread part.
+    // 32), so tt = ttu(k0) + kr * tA + gt * tB: a wave-uniform part per chunk
+    // and this constant thread part.
     uint32_t thr_w[2], thr_s[2];   // byte offsets of the word and the scale from the chunk's base
 #pragma unroll
     for (int h = 0; h < 2; h++) {
-        const uint32_t tt = (uint32_t)((kr + (X3 ? h : 0)) * tA + gt[h] * tB);
+        const uint32_t tt = (uint32_t)(kr * tA + gt[h] * tB);
         thr_w[h] = tt * 16u + 4u * (uint32_t)qw;
         thr_s[h] = tt * (uint32_t)ts.R * 2u;
     }
@@ -329,9 +166,8 @@ k_gemm_q4(GemmA a, Q4Tiled w, GemmOut o, int tm, int S)
                 f.rg[j][1] = gv.y;
             }
         }
-        // k = k0 + kr (+ h on X3): slice s, row r, position pt of the tiled
-        // layout; k0 is a multiple of 32, so only P = 16 splits a chunk over
-        // rows
+        // k = k0 + kr: slice s, row r, position pt of the tiled layout; k0 is
+        // a multiple of 32, so only P = 16 splits a chunk over rows
         const int s = k0 / w.KC, rr0 = k0 - s * w.KC, r0 = rr0 / P, pt0 = rr0 - r0 * P;
 #pragma unroll
         for (int h = 0; h < 2; h++) {
@@ -344,7 +180,7 @@ k_gemm_q4(GemmA a, Q4Tiled w, GemmOut o, int tm, int S)
                 sc = __builtin_amdgcn_raw_buffer_load_b16(rsW, thr_s[h], tb + ts.R * ts.T * 16 + (ttu * ts.R + r0) * 2, 0);
             } else {
                 const uint8_t *tile = w.data + (size_t)(s * w.CT + gct[h]) * w.tile_bytes;
-                const int ptk = pt0 + kr + (X3 ? h : 0);
+                const int ptk = pt0 + kr;
                 const int r = r0 + (ptk >> 4), pt = ptk & 15;
                 const int tt = (pt >> 6) * 64 * ts.GB + (pt & 63) * tA + gt[h] * tB;
                 word = *(const uint32_t *)(tile + ((size_t)r * ts.T + tt) * 16 + 4 * qw);
@@ -358,67 +194,22 @@ k_gemm_q4(GemmA a, Q4Tiled w, GemmOut o, int tm, int S)
 #pragma unroll
         for (int j = 0; j < NA; j++) {
             f32x4 x = f.ra[j] * amul[j];
-            if constexpr (X3) {
-                if (NORM) {
-                    // (x * inv) * gamma, gamma read as f16 from its register
-                    const float nz = -0.0f;
-                    x.x = mul_f16_half<0>(f.rg[j][0], x.x, nz);
-                    x.y = mul_f16_half<1>(f.rg[j][0], x.y, nz);
-                    x.z = mul_f16_half<0>(f.rg[j][1], x.z, nz);
-                    x.w = mul_f16_half<1>(f.rg[j][1], x.w, nz);
-                }
-                // row aoff / GLD, halves 4 (slot % 8)..+3
-                const int r = aoff[j] / GLD, kk = aoff[j] - r * GLD;
-                uint32_t h01, l01, h23, l23;
-                split_f16_pair(x.x, x.y, h01, l01);
-                split_f16_pair(x.z, x.w, h23, l23);
-                *(uint2 *)&xa(buf, 0)[r * HLD + kk] = uint2{h01, h23};
-                *(uint2 *)&xa(buf, 1)[r * HLD + kk] = uint2{l01, l23};
-            } else {
-                if (NORM) {
-                    x.x *= h2f(f.rg[j][0] & 0xFFFFu);
-                    x.y *= h2f(f.rg[j][0] >> 16);
-                    x.z *= h2f(f.rg[j][1] & 0xFFFFu);
-                    x.w *= h2f(f.rg[j][1] >> 16);
-                }
-                *(f32x4 *)&As[buf][aoff[j]] = x;
+            if (NORM) {
+                x.x *= h2f(f.rg[j][0] & 0xFFFFu);
+                x.y *= h2f(f.rg[j][0] >> 16);
+                x.z *= h2f(f.rg[j][1] & 0xFFFFu);
+                x.w *= h2f(f.rg[j][1] >> 16);
             }
+            *(f32x4 *)&As[buf][aoff[j]] = x;
         }
         // 8 columns 32*g + 8*qw + c, c = 0..7: byte c/2, low nibble even c
-        if constexpr (X3) {
-            // Rows kr, kr + 1 interleaved by bytes: p01 = [r0.b0, r0.b1,
-            // r1.b0, r1.b1], p23 likewise, so (p >> 4c') & 0x000F000F
-            // holds column c's nibble of both rows.  Two values per packed
-            // f16 operation: | 0x64006400 gives 1024 + nib, adding -1032
-            // leaves nib - 8 exactly; hi = f16(n8 * s) is the f16 rounding
-            // of the exact product (4 + 11 significant bits), as
-            // f16(f32(n8) * s) is, and lo = f16(n8 * s - hi) in one fused
-            // operation is the rounding of the exact remainder, as
-            // f16(f32 product - hi) is.
-            const uint32_t p01 = __builtin_amdgcn_perm(f.rb[1], f.rb[0], 0x05040100u);
-            const uint32_t p23 = __builtin_amdgcn_perm(f.rb[1], f.rb[0], 0x07060302u);
-            // the rows' scales times 2^bshift: exact (a power-of-two multiple)
-            const h16x2 sp = {(_Float16)(h2f(f.rs[0]) * bscale), (_Float16)(h2f(f.rs[1]) * bscale)};
-            const h16x2 off = {(_Float16)-1032.0f, (_Float16)-1032.0f};
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const float sc = h2f(f.rs[h]);
 #pragma unroll
             for (int c = 0; c < 8; c++) {
-                const uint32_t pw = (c < 4 ? p01 : p23) >> (4 * (c & 3));
-                const h16x2 n8 = __builtin_bit_cast(h16x2, and_or_opaque(pw, 0x000F000Fu, 0x64006400u)) + off;
-                const h16x2 hi = n8 * sp;
-                const h16x2 lo = __builtin_elementwise_fma(n8, sp, -hi);
-                const int col = 32 * gi + 8 * qw + c;
-                *(h16x2 *)&xb(buf, 0)[col * HLD + (col >> 4) * BPAD + kr] = hi;
-                *(h16x2 *)&xb(buf, 1)[col * HLD + (col >> 4) * BPAD + kr] = lo;
-            }
-        } else {
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const float sc = h2f(f.rs[h]);
-#pragma unroll
-                for (int c = 0; c < 8; c++) {
-                    const float v = (float)((int)((f.rb[h] >> (4 * c)) & 15u) - 8) * sc;
-                    Bs[buf][(32 * gi + 8 * qw + 64 * h + c) * GLD + kr] = v;
-                }
+                const float v = (float)((int)((f.rb[h] >> (4 * c)) & 15u) - 8) * sc;
+                Bs[buf][(32 * gi + 8 * qw + 64 * h + c) * GLD + kr] = v;
             }
         }
     };
@@ -433,58 +224,12 @@ k_gemm_q4(GemmA a, Q4Tiled w, GemmOut o, int tm, int S)
 #pragma unroll
         for (int j = 0; j < 2; j++) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     mfma_pipeline<Fetch>(
-        c1 - c0, [&](Fetch &f, int c) { fetch(f, (c0 + c) * GK); }, stage, pre, [&](int buf) {
-            if constexpr (X3)
-                mfma_chunk_x3<MB, BPAD>(acc, xa(buf, 0), xa(buf, 1), xb(buf, 0), xb(buf, 1), cb, lane);
-            else
-                mfma_chunk<MB>(acc, As[buf], Bs[buf], cb, lane);
-        });
+        c1 - c0, [&](Fetch &f, int c) { fetch(f, (c0 + c) * GK); }, stage,
+        [&](int buf) { mfma_chunk<MB>(acc, As[buf], Bs[buf], cb, lane); });
 
-    if constexpr (X3) {
-        // rsc was written before the pipeline's first barrier
-#pragma unroll
-        for (int i = 0; i < MB; i++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const float u = rsc[16 * i + 4 * q + e];
-#pragma unroll
-                for (int j = 0; j < 2; j++) acc[i][j][e] *= u;
-            }
-    }
     // epilogue: element e of acc[i][j] is row 16i + 4q + e of the tile,
     // column 128nt + 16(cb0 + 2j) + r16
     float *Y = o.Y + (EPI == GEMM_PART ? (size_t)sl * o.slice_stride : 0);
-    if constexpr (EPI == GEMM_SWIGLU) {
-        // groups (4nt, 4nt+1) and (4nt+2, 4nt+3) are (gate, up) pairs
-        const int col = 32 * (2 * nt + (wv >> 1)) + 16 * (wv & 1) + r16;
-        float vmax[MB][4];
-#pragma unroll
-        for (int i = 0; i < MB; i++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int m = m0 + 16 * i + 4 * q + e;
-                const float v = silu_f(acc[i][0][e]) * acc[i][1][e];
-                if (m < a.M && col < o.ncols) Y[(size_t)m * o.ldy + col] = v;
-                vmax[i][e] = col < o.ncols ? fabsf(v) : 0.0f;
-            }
-        // largest |silu(g) u| of each row over this tile's 64 output columns
-        // (the range of the down projection's staging): over a wave's 16
-        // columns by DPP, then over the four waves through LDS
-        if (o.rmax) {
-#pragma unroll
-            for (int i = 0; i < MB; i++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const float v = row_max16(vmax[i][e]);   // the 16 lanes r16 of this q form one DPP row
-                    if (r16 == 0) wmx[wv][16 * i + 4 * q + e] = v;
-                }
-            __syncthreads();
-            if (t < BM && m0 + t < a.M)
-                o.rmax[(size_t)(m0 + t) * o.rslots + nt] =
-                    fmaxf(fmaxf(wmx[0][t], wmx[1][t]), fmaxf(wmx[2][t], wmx[3][t]));
-        }
-        return;
-    }
 #pragma unroll
     for (int i = 0; i < MB; i++) {
 #pragma unroll
@@ -492,7 +237,11 @@ k_gemm_q4(GemmA a, Q4Tiled w, GemmOut o, int tm, int S)
             const int m = m0 + 16 * i + 4 * q + e;
             if (m >= a.M) continue;
             float *yr = Y + (size_t)m * o.ldy;
-            {
+            if constexpr (EPI == GEMM_SWIGLU) {
+                // groups (4nt, 4nt+1) and (4nt+2, 4nt+3) are (gate, up) pairs
+                const int col = 32 * (2 * nt + (wv >> 1)) + 16 * (wv & 1) + r16;
+                if (col < o.ncols) yr[col] = silu_f(acc[i][0][e]) * acc[i][1][e];
+            } else {
 #pragma unroll
                 for (int j = 0; j < 2; j++) {
                     const int col = GN * nt + 16 * (cb0 + 2 * j) + r16;
@@ -508,28 +257,23 @@ k_gemm_q4(GemmA a, Q4Tiled w, GemmOut o, int tm, int S)
 }
 
 // ---------------------------------------------------------------------------
-// q|k|v partial rows (S k-slices, added in slice order) -> QK-norm
-// (talker.rs:89-99), RoPE at start + row (rope.rs:79-92), q rows out, K
-// (normed, roped) and V (raw) appended to the paged cache at the same
-// position (talker.rs:419-425).  One wave per (row, head): heads 0..15 q,
-// 16..23 k, 24..31 v; lane holds dims (l, l+64).
+// q|k|v partial rows -> QK-norm (talker.rs:89-99), RoPE at start + row
+// (rope.rs:79-92), q rows out, K (normed, roped) and V (raw) appended to the
+// paged cache at the same position (talker.rs:419-425).  One wave per (row,
+// head): heads 0..15 q, 16..23 k, 24..31 v; lane holds dims (l, l+64).
 // ---------------------------------------------------------------------------
 
+template <int NP>
 __global__ void __launch_bounds__(256)
-k_prefill_qkv_post(const float *part, int S, size_t slice_stride, int ldp, int M, int64_t start,
-                   const uint16_t *qn_g, const uint16_t *kn_g, const float *rope_cos, const float *rope_sin,
-                   KvPaged kv, int layer, float *q, int ldq)
+k_prefill_qkv_post(MmParts p, int M, int64_t start, const uint16_t *qn_g, const uint16_t *kn_g,
+                   const float *rope_cos, const float *rope_sin, KvPaged kv, int layer, float *q, int ldq)
 {
     const int lane = threadIdx.x & 63;
     const int m = blockIdx.x, hh = blockIdx.y * 4 + (threadIdx.x >> 6);
     if (m >= M) return;
     const int64_t pos = start + m;
-    const float *row = part + (size_t)m * ldp + hh * HEAD_DIM;
-    float x0 = row[lane], x1 = row[lane + 64];
-    for (int s = 1; s < S; s++) {
-        x0 += row[s * slice_stride + lane];
-        x1 += row[s * slice_stride + lane + 64];
-    }
+    const size_t at = (size_t)m * p.ld + hh * HEAD_DIM;
+    const float x0 = sum_parts<NP>(p, at + lane), x1 = sum_parts<NP>(p, at + lane + 64);
     if (hh >= 24) {
         float *vp = kv_ptr(kv, layer, (int)pos, hh - 24, 1);
         vp[lane] = x0;
@@ -548,33 +292,63 @@ k_prefill_qkv_post(const float *part, int S, size_t slice_stride, int ldp, int M
 }
 
 // ---------------------------------------------------------------------------
-// Residual add of a projection's k-slice partials (x += sum over slices, in
-// slice order: talker.rs:461, 474) fused with the next RMSNorm's 1/rms of
-// the updated row (gemv.rs:445-454).  One workgroup per row.
+// Residual add of a projection's partial sums (x += parts: talker.rs:461,
+// 474; p.n = 0: nothing to add) fused with the next RMSNorm (gemv.rs:445-454):
+// 1/rms of the updated row, and with a gamma the normed row (x * inv) * gamma
+// split for the GEMM, staged times 2^nshift.  One workgroup per row of at
+// most 2048 columns, each thread's values in registers.
 // ---------------------------------------------------------------------------
 
+template <int NP>
 __global__ void __launch_bounds__(256)
-k_resid_add_inv(float *x, int ldx, const float *part, int S, size_t slice_stride, int ldp, int H, float *inv)
+k_resid_norm(float *x, int H, MmParts p, float *inv_out, const uint16_t *gamma, int nshift, uint8_t *split, int kc)
 {
     __shared__ float red[4];
     const int t = threadIdx.x, m = blockIdx.x;
-    float *xr = x + (size_t)m * ldx;
-    const float *pr = part + (size_t)m * ldp;
+    float *xr = x + (size_t)m * H;
+    f32x4 v[2];
+    uint2 g[2];
     float ss = 0.0f;
-    for (int j = 4 * t; j < H; j += 1024) {
-        f32x4 p = ld4(pr + j);
-        for (int s = 1; s < S; s++) p += ld4(pr + s * slice_stride + j);
-        const f32x4 v = ld4(xr + j) + p;
-        *(f32x4 *)(xr + j) = v;
-        ss = fmaf(v.x, v.x, ss);
-        ss = fmaf(v.y, v.y, ss);
-        ss = fmaf(v.z, v.z, ss);
-        ss = fmaf(v.w, v.w, ss);
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        const int j = 4 * t + 1024 * u;
+        v[u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        g[u] = uint2{0, 0};
+        if (j >= H) continue;
+        v[u] = ld4(xr + j);
+        if (gamma) g[u] = *(const uint2 *)(gamma + j);
+        if (p.n) {
+            v[u] += sum_parts4<NP>(p, (size_t)m * p.ld + j);
+            *(f32x4 *)(xr + j) = v[u];
+        }
+        ss = fmaf(v[u].x, v[u].x, ss);
+        ss = fmaf(v[u].y, v[u].y, ss);
+        ss = fmaf(v[u].z, v[u].z, ss);
+        ss = fmaf(v[u].w, v[u].w, ss);
     }
     ss = wave_sum_dpp(ss);
     if ((t & 63) == 0) red[t >> 6] = ss;
     __syncthreads();
-    if (t == 0) inv[m] = 1.0f / sqrtf(((red[0] + red[1]) + (red[2] + red[3])) / (float)H + 1e-6f);
+    const float inv = 1.0f / sqrtf(((red[0] + red[1]) + (red[2] + red[3])) / (float)H + 1e-6f);
+    if (inv_out && t == 0) inv_out[m] = inv;
+    if (!split) return;
+    const float mul = inv * __builtin_ldexpf(1.0f, nshift);
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        const int j = 4 * t + 1024 * u;
+        if (j >= 64 * kc) continue;
+        f32x4 y = v[u] * mul;
+        y.x *= h2f(g[u].x & 0xFFFFu);
+        y.y *= h2f(g[u].x >> 16);
+        y.z *= h2f(g[u].y & 0xFFFFu);
+        y.w *= h2f(g[u].y >> 16);
+        uint32_t h0, l0, h1, l1;
+        split_f16_pair<true>(y.x, y.y, h0, l0);
+        split_f16_pair<true>(y.z, y.w, h1, l1);
+        uint8_t *o = split + ((size_t)m * kc + (j >> 6)) * 256 + ((j >> 5) & 1) * 128 + (j & 31) * 2;
+        *(uint2 *)o = uint2{h0, h1};
+        *(uint2 *)(o + 64) = uint2{l0, l1};
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -768,7 +542,7 @@ __device__ __forceinline__ void split4(float a, float b, float c, float d, half4
 template <bool SC>
 __global__ void __launch_bounds__(256)
 k_prefill_attn_mx(const float *q, int ldq, int M, int64_t start, KvPaged kv, int layer, float *out, int ldo,
-                  float *rmax, int rslots, int sq, int sk, int sv)
+                  uint8_t *split, float *rsc, int ldr, int sq, int sk, int sv)
 {
     constexpr int QR = 8;
     __shared__ float smax[4][16], ssum[4][16];
@@ -898,54 +672,42 @@ k_prefill_attn_mx(const float *q, int ldq, int M, int64_t start, KvPaged kv, int
             l = fmaf(wgt[w], ssum[w][qi], l);
         }
         const float inv = 1.0f / l;
-        float *op = out + (size_t)(m0 + row) * ldo + (2 * h + (qi & 1)) * HEAD_DIM + d0;
+        const int col = (2 * h + (qi & 1)) * HEAD_DIM + d0;
         float mx = 0.0f;
+        f32x4 v[2];
         // (the sums of P V times 2^sv, merged, divided by l, scaled back)
 #pragma unroll
-        for (int j = 0; j < 8; j += 4) {
+        for (int j = 0; j < 2; j++) {
             f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int w = 0; w < 4; w++) acc += wgt[w] * *(const f32x4 *)&so[w][qi][d0 + j];
+            for (int w = 0; w < 4; w++) acc += wgt[w] * *(const f32x4 *)&so[w][qi][d0 + 4 * j];
             acc = SC ? (acc * inv) * uv : acc * inv;
-            *(f32x4 *)(op + j) = acc;
+            v[j] = acc;
             mx = fmaxf(mx, fmaxf(fmaxf(fabsf(acc.x), fabsf(acc.y)), fmaxf(fabsf(acc.z), fabsf(acc.w))));
         }
-        // the largest |output| of the row over its two heads (the range of
-        // the o-projection's staging): the row's 32 lanes are one half-wave
+        if (!split) {
+            float *op = out + (size_t)(m0 + row) * ldo + col;
+            *(f32x4 *)op = v[0];
+            *(f32x4 *)(op + 4) = v[1];
+            return;
+        }
+        // the row's two heads (256 columns, one K segment of the
+        // o-projection) staged by their largest |output|: the row's 32 lanes
+        // are one half-wave
         mx = fmaxf(mx, __shfl_xor(mx, 1));
         mx = fmaxf(mx, __shfl_xor(mx, 2));
         mx = fmaxf(mx, __shfl_xor(mx, 4));
         mx = fmaxf(mx, __shfl_xor(mx, 8));
         mx = fmaxf(mx, __shfl_xor(mx, 16));
-        if (rmax && (t & 31) == 0) rmax[(size_t)(m0 + row) * rslots + h] = mx;
+        const int sh = range_shift(mx);
+        const float p2 = __builtin_ldexpf(1.0f, sh);
+        half8 hi, lo;
+        split8(v[0] * p2, v[1] * p2, hi, lo);
+        uint8_t *sp = split + (size_t)(m0 + row) * (16 * HEAD_DIM * 4) + (col >> 5) * 128 + (col & 31) * 2;
+        *(half8 *)sp = hi;
+        *(half8 *)(sp + 64) = lo;
+        if ((t & 31) == 0) rsc[(size_t)h * ldr + m0 + row] = __builtin_ldexpf(1.0f, -sh);
     }
-}
-
-// ---------------------------------------------------------------------------
-// Largest |x| of each row over slots of rw columns: out[m][s] = max over k in
-// [s rw, min((s+1) rw, K)) of |X[m][k]|.  One wave per (row, slot).  The
-// range of the split-f16 staging for GEMM rows no kernel of the chain
-// measured on the way out.
-// ---------------------------------------------------------------------------
-
-__global__ void __launch_bounds__(256)
-k_row_absmax(const float *X, int ld, int M, int K, int rw, int rslots, float *out)
-{
-    const int lane = threadIdx.x & 63;
-    const int id = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (id >= M * rslots) return;
-    const int m = id / rslots, sl = id - m * rslots;
-    const float *x = X + (size_t)m * ld;
-    const int k1 = min((sl + 1) * rw, K);
-    float mx = 0.0f;
-    for (int k = sl * rw + lane; k < k1; k += 64) mx = fmaxf(mx, fabsf(x[k]));
-    mx = fmaxf(mx, __shfl_xor(mx, 1));
-    mx = fmaxf(mx, __shfl_xor(mx, 2));
-    mx = fmaxf(mx, __shfl_xor(mx, 4));
-    mx = fmaxf(mx, __shfl_xor(mx, 8));
-    mx = fmaxf(mx, __shfl_xor(mx, 16));
-    mx = fmaxf(mx, __shfl_xor(mx, 32));
-    if (lane == 0) out[(size_t)m * rslots + sl] = mx;
 }
 
 // the matrix-core attention unless QTTS_PREFILL_ATTN_VALU=1
@@ -1025,8 +787,7 @@ static int part_slices(const Q4Tiled &w)
     return S;
 }
 
-// The split-f16 contraction unless QTTS_GEMM_F32=1 (f32 matrix instructions).
-static bool gemm_x3()
+bool gemm_x3()
 {
     // read at every launch (a few hundred ns), so a caller or test can switch
     // paths between calls
@@ -1039,39 +800,17 @@ static hipError_t launch_gemm_mb(const GemmA &a, const Q4Tiled &w, const GemmOut
 {
     const int tm = (a.M + 16 * MB - 1) / (16 * MB), tn = (w.G * 32 + GN - 1) / GN;
     const dim3 grid(tm * tn * S);
-    if (gemm_x3() && w.bshift >= 0) {
-        if (a.inv)
-            hipLaunchKernelGGL((k_gemm_q4<MB, EPI, true, true>), grid, dim3(256), 0, s, a, w, o, tm, S);
-        else
-            hipLaunchKernelGGL((k_gemm_q4<MB, EPI, false, true>), grid, dim3(256), 0, s, a, w, o, tm, S);
-    } else {
-        if (a.inv)
-            hipLaunchKernelGGL((k_gemm_q4<MB, EPI, true, false>), grid, dim3(256), 0, s, a, w, o, tm, S);
-        else
-            hipLaunchKernelGGL((k_gemm_q4<MB, EPI, false, false>), grid, dim3(256), 0, s, a, w, o, tm, S);
-    }
+    if (a.inv)
+        hipLaunchKernelGGL((k_gemm_q4<MB, EPI, true>), grid, dim3(256), 0, s, a, w, o, tm, S);
+    else
+        hipLaunchKernelGGL((k_gemm_q4<MB, EPI, false>), grid, dim3(256), 0, s, a, w, o, tm, S);
     return hipGetLastError();
-}
-
-// The staging-range slots of every k-slice fit the GEMM's reads: at most 16
-// slots per slice (two per lane of a row's 8), all within the row.
-static bool rmax_fits(const GemmA &a, int K, int S)
-{
-    if (!a.rmax) return true;
-    if (a.rslots < 1 || a.rw < 1 || (int64_t)a.rslots * a.rw < K) return false;
-    const int nch = K / GK;
-    for (int sl = 0; sl < S; sl++) {
-        const int c0 = sl * nch / S, c1 = (sl + 1) * nch / S;
-        if ((c1 * GK - 1) / a.rw - (c0 * GK) / a.rw >= 16) return false;
-    }
-    return true;
 }
 
 template <int EPI>
 static hipError_t launch_gemm(const GemmA &a, const Q4Tiled &w, const GemmOut &o, int S, hipStream_t s)
 {
     if (!gemm_shape_ok(w, w.k) || a.M < 1 || a.lda % 4 || S < 1 || S > w.k / (2 * GK)) return hipErrorInvalidValue;
-    if (!rmax_fits(a, w.k, S) || (o.rmax && o.rslots < (w.G * 32 + GN - 1) / GN)) return hipErrorInvalidValue;
     if (EPI == GEMM_SWIGLU && (!w.interleave || w.G % 4)) return hipErrorInvalidValue;
     if ((EPI == GEMM_BIAS || EPI == GEMM_BIAS_SILU) && !o.bias) return hipErrorInvalidValue;
     if (EPI != GEMM_PART && S != 1) return hipErrorInvalidValue;
@@ -1090,37 +829,28 @@ bool gemm_supported(const Q4Tiled &w)
     return gemm_shape_ok(w, w.k);
 }
 
-static hipError_t row_absmax(const float *X, int ld, int M, int K, int rw, int rslots, float *out, hipStream_t s)
+// Rows of any magnitude (gemm_q4 takes any finite input, gemv.rs:349-412).
+// ws: the split path's workspace (enqueue_mm_rows).
+hipError_t enqueue_gemm_rows(const Q4Tiled &w, const Q4Frag &f, const float *X, int rows, float *Y, int ldy, float *ws,
+                             size_t ws_floats, hipStream_t s)
 {
-    const int n = M * rslots;
-    hipLaunchKernelGGL(k_row_absmax, dim3((n + 3) / 4), dim3(256), 0, s, X, ld, M, K, rw, rslots, out);
-    return hipGetLastError();
-}
-
-// Rows of any magnitude (gemm_q4 takes any finite input, gemv.rs:349-412):
-// each row's largest |x| first (rmax, rows floats), for the staging's range.
-hipError_t enqueue_gemm_rows(const Q4Tiled &w, const float *X, int rows, float *Y, int ldy, float *rmax,
-                             hipStream_t s)
-{
-    if (gemm_x3()) PCHK(row_absmax(X, w.k, rows, w.k, w.k, 1, rmax, s));
-    const GemmA a{X, w.k, nullptr, nullptr, rows, rmax, 1, w.k, 0};
-    return launch_gemm<GEMM_STORE>(a, w, GemmOut{Y, ldy, std::min(ldy, w.G * 32), nullptr, 0}, 1, s);
+    if (gemm_x3() && f.data && ws_floats >= (size_t)f.kc * 64 + 1)
+        return enqueue_mm_rows(f, X, w.k, rows, nullptr, false, Y, ldy, ws, ws_floats, s);
+    return launch_gemm<GEMM_STORE>(GemmA{X, w.k, nullptr, nullptr, rows}, w,
+                                   GemmOut{Y, ldy, std::min(ldy, w.G * 32), nullptr, 0}, 1, s);
 }
 
 // Y = X W + bias, optionally through SiLU (the text projection's fc1 / fc2,
-// talker.rs:105-116, over a batch of rows).  rmax: rows floats, as above.
-hipError_t enqueue_gemm_bias(const Q4Tiled &w, const float *X, int rows, const float *bias, bool silu, float *Y,
-                             int ldy, float *rmax, hipStream_t s)
+// talker.rs:105-116, over a batch of rows).
+hipError_t enqueue_gemm_bias(const Q4Tiled &w, const Q4Frag &f, const float *X, int rows, const float *bias, bool silu,
+                             float *Y, int ldy, float *ws, size_t ws_floats, hipStream_t s)
 {
-    if (gemm_x3()) PCHK(row_absmax(X, w.k, rows, w.k, w.k, 1, rmax, s));
-    const GemmA a{X, w.k, nullptr, nullptr, rows, rmax, 1, w.k, 0};
+    if (gemm_x3() && f.data && w.n % 32 == 0)
+        return enqueue_mm_rows(f, X, w.k, rows, bias, silu, Y, ldy, ws, ws_floats, s);
+    const GemmA a{X, w.k, nullptr, nullptr, rows};
     const GemmOut o{Y, ldy, std::min(ldy, w.n), bias, 0};
     return silu ? launch_gemm<GEMM_BIAS_SILU>(a, w, o, 1, s) : launch_gemm<GEMM_BIAS>(a, w, o, 1, s);
 }
-
-// Slots of the down projection's input range: one per 64 output columns of
-// the gate|up GEMM (one column tile).
-static int down_rslots(const TalkerDev &m) { return ((m.inter + 63) / 64 + 3) & ~3; }
 
 bool prefill_supported(const TalkerDev &m)
 {
@@ -1136,10 +866,10 @@ bool prefill_supported(const TalkerDev &m)
     return true;
 }
 
-// Column slots per prompt row of the staging-range buffer (PrefillWs.rmax):
-// 8 for the o-projection's input (one per kv head), one per 64 columns for
-// the down projection's.
-int64_t prefill_rmax_slots(const TalkerDev &m) { return std::max<int64_t>(8, down_rslots(m)); }
+// Column slots of the factors of a split GEMM input (PrefillWs.rsc): 8 for
+// the o-projection's (one per kv head), one per 64 columns for the down
+// projection's.
+int64_t prefill_rsc_slots(const TalkerDev &m) { return std::max<int64_t>(8, (m.inter + 63) / 64); }
 
 // The staging power of two of rows normed with this gamma (f16 bit
 // patterns, on the host): |x * inv * gamma| <= sqrt(n) * max|gamma|, since
@@ -1179,15 +909,22 @@ int norm_shift(const uint16_t *gamma_host, int n)
     return bound_shift(std::sqrt((double)n) * f16_max_abs(gamma_host, n));
 }
 
-// Floats per prompt row of the k-slice partials buffer.
-int64_t prefill_part_floats(const TalkerDev &m)
+// Floats of partial sums the prompt's projections need at up to `rows` rows.
+int64_t prefill_part_floats(const TalkerDev &m, int rows)
 {
     int64_t f = 0;
     for (int l = 0; l < m.n_layers; l++) {
         const LayerDev &L = m.layers[l];
-        f = std::max<int64_t>(f, (int64_t)part_slices(L.qkv) * L.qkv.G * 32);
-        f = std::max<int64_t>(f, (int64_t)part_slices(L.o) * L.o.G * 32);
-        f = std::max<int64_t>(f, (int64_t)part_slices(L.down) * L.down.G * 32);
+        for (const Q4Tiled *w : {&L.qkv, &L.o, &L.down}) f = std::max<int64_t>(f, (int64_t)rows * part_slices(*w) * w->G * 32);
+        if (!L.qkv_f.data) continue;
+        // a small batch may cut K finer than a large one
+        for (int r = rows;; r = std::min(64, rows)) {
+            f = std::max<int64_t>(f, (int64_t)mm_part_floats(L.qkv_f, r, false));
+            f = std::max<int64_t>(f, (int64_t)mm_part_floats(L.o_f, r, false));
+            f = std::max<int64_t>(f, (int64_t)mm_part_floats(L.down_f, r, true));
+            f = std::max<int64_t>(f, (int64_t)mm_swiglu_part_floats(L.gate_up_f, r));
+            if (r <= 64) break;
+        }
     }
     return f;
 }
@@ -1198,29 +935,67 @@ hipError_t enqueue_fill_rows(float *x, int64_t n, uint32_t seed, hipStream_t s)
     return hipGetLastError();
 }
 
-hipError_t enqueue_row_inv(const float *X, int ld, int M, int K, float *inv, hipStream_t s)
+static bool split_path(const TalkerDev &m)
 {
-    if (K % 4 || ld % 4) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_row_inv, dim3((M + 3) / 4), dim3(256), 0, s, X, ld, M, K, inv);
-    return hipGetLastError();
+    if (!gemm_x3() || m.hidden > 2048) return false;
+    for (int l = 0; l < m.n_layers; l++) {
+        const LayerDev &L = m.layers[l];
+        if (!L.qkv_f.data || !L.o_f.data || !L.gate_up_f.data || !L.down_f.data) return false;
+    }
+    return true;
 }
 
-// The prefill's gate|up GEMM of layer l alone (pw.x rows and pw.inv set).
+template <int NP>
+struct ResidNorm {
+    static hipError_t go(float *x, int H, int M, const MmParts &p, float *inv, const uint16_t *gamma, int nshift,
+                         uint8_t *split, hipStream_t s)
+    {
+        hipLaunchKernelGGL(k_resid_norm<NP>, dim3(M), dim3(256), 0, s, x, H, p, inv, gamma, nshift, split, (H + 63) / 64);
+        return hipGetLastError();
+    }
+};
+
+template <int NP>
+struct QkvPost {
+    static hipError_t go(const TalkerDev &m, const LayerDev &L, const PrefillWs &pw, const MmParts &p, int M, int64_t start,
+                         int l, hipStream_t s)
+    {
+        hipLaunchKernelGGL(k_prefill_qkv_post<NP>, dim3(M, 8), dim3(256), 0, s, p, M, start, L.q_norm, L.k_norm, m.rope_cos,
+                           m.rope_sin, m.kv, l, pw.q, 16 * HEAD_DIM);
+        return hipGetLastError();
+    }
+};
+
+// The prefill's gate|up GEMM of layer l alone (pw.xs rows; on the f32 path
+// pw.x rows and pw.inv).
 hipError_t enqueue_gemm_gateup(const TalkerDev &m, const PrefillWs &pw, int l, int M, hipStream_t s)
 {
     const LayerDev &L = m.layers[l];
-    return launch_gemm<GEMM_SWIGLU>(GemmA{pw.x, m.hidden, pw.inv, L.post_norm, M, nullptr, 0, 0, L.post_shift},
-                                    L.gate_up, GemmOut{pw.h, m.inter, m.inter, nullptr, 0, pw.rmax, down_rslots(m)},
-                                    1, s);
+    if (split_path(m)) {
+        const int kc = (m.hidden + 63) / 64;
+        return enqueue_mm_swiglu(RowsSplit{(const uint8_t *)pw.xs, kc, M, nullptr, 0, __builtin_ldexpf(1.0f, -L.post_shift)},
+                                 L.gate_up_f, pw.part, (uint8_t *)pw.h, (m.inter + 63) / 64, pw.rsc, s);
+    }
+    return launch_gemm<GEMM_SWIGLU>(GemmA{pw.x, m.hidden, pw.inv, L.post_norm, M}, L.gate_up,
+                                    GemmOut{pw.h, m.inter, m.inter, nullptr, 0}, 1, s);
 }
 
-// A projection into k-slice partials: slice s of row m at part[s * M * ld +
-// m * ld], ld = the weight's padded width.
-static hipError_t gemm_parts(const GemmA &a, const Q4Tiled &w, const PrefillWs &pw, int *S, int *ld, hipStream_t s)
+// What enqueue_gemm_gateup reads, from pw.x: the rows normed and split (for
+// layer l's staging), or their 1/rms.
+hipError_t enqueue_gateup_input(const TalkerDev &m, const PrefillWs &pw, int l, int M, hipStream_t s)
 {
-    *S = part_slices(w);
-    *ld = w.G * 32;
-    return launch_gemm<GEMM_PART>(a, w, GemmOut{pw.part, *ld, *ld, nullptr, (size_t)a.M * *ld}, *S, s);
+    const bool sp = split_path(m);
+    return ResidNorm<1>::go(pw.x, m.hidden, M, MmParts{}, pw.inv, sp ? m.layers[l].post_norm : nullptr,
+                            m.layers[l].post_shift, sp ? (uint8_t *)pw.xs : nullptr, s);
+}
+
+// A projection of the f32 path into k-slice partials: slice s of row m at
+// part[s * M * ld + m * ld], ld = the weight's padded width.
+static hipError_t gemm_parts(const GemmA &a, const Q4Tiled &w, const PrefillWs &pw, MmParts *p, hipStream_t s)
+{
+    const int S = part_slices(w), ld = w.G * 32;
+    *p = MmParts{pw.part, ld, (size_t)a.M * ld, S, 1};
+    return launch_gemm<GEMM_PART>(a, w, GemmOut{pw.part, ld, ld, nullptr, p->stride}, S, s);
 }
 
 // Rows pw.x[0..M) at positions start..start+M-1 through every layer; the
@@ -1229,46 +1004,57 @@ static hipError_t gemm_parts(const GemmA &a, const Q4Tiled &w, const PrefillWs &
 hipError_t enqueue_talker_prefill(const TalkerDev &m, const PrefillWs &pw, int M, int64_t start, float *hidden_out,
                                   hipStream_t s)
 {
-    if (M < 1 || M > pw.cap_rows) return hipErrorInvalidValue;
-    const int H = m.hidden, A = 16 * HEAD_DIM;
-    int S, ld;
-    PCHK(enqueue_row_inv(pw.x, H, M, H, pw.inv, s));
+    if (M < 1 || M > pw.cap_rows || m.hidden > 2048) return hipErrorInvalidValue;
+    const int H = m.hidden, A = 16 * HEAD_DIM, kh = (H + 63) / 64, ki = (m.inter + 63) / 64;
+    const bool sp = split_path(m);
+    uint8_t *xs = sp ? (uint8_t *)pw.xs : nullptr;
+    MmParts p{};
+    // x += parts, then the rows the next GEMM takes
+    const auto resid = [&](const uint16_t *gamma, int shift) {
+        return by_parts<ResidNorm>(p.n, pw.x, H, M, p, pw.inv, sp ? gamma : nullptr, shift, gamma ? xs : nullptr, s);
+    };
+    PCHK(resid(m.layers[0].input_norm, m.layers[0].in_shift));
     for (int l = 0; l < m.n_layers; l++) {
         const LayerDev &L = m.layers[l];
-        // q|k|v (input norm fused), QK-norm + RoPE + KV append, attention
-        PCHK(gemm_parts(GemmA{pw.x, H, pw.inv, L.input_norm, M, nullptr, 0, 0, L.in_shift}, L.qkv, pw, &S, &ld, s));
-        hipLaunchKernelGGL(k_prefill_qkv_post, dim3(M, 8), dim3(256), 0, s, pw.part, S, (size_t)M * ld, ld, M, start,
-                           L.q_norm, L.k_norm, m.rope_cos, m.rope_sin, m.kv, l, pw.q, A);
-        PCHK(hipGetLastError());
-        // attention rows, and each row's largest |value| per kv head's two
-        // q heads (the o-projection's staging range: 8 slots of 256)
+        // q|k|v, QK-norm + RoPE + KV append, attention
+        if (sp)
+            PCHK(enqueue_mm_parts(RowsSplit{xs, kh, M, nullptr, 0, __builtin_ldexpf(1.0f, -L.in_shift)}, L.qkv_f, false,
+                                  pw.part, &p, s));
+        else
+            PCHK(gemm_parts(GemmA{pw.x, H, pw.inv, L.input_norm, M}, L.qkv, pw, &p, s));
+        PCHK(by_parts<QkvPost>(p.n, m, L, pw, p, M, start, l, s));
+        uint8_t *as = sp ? (uint8_t *)pw.attn : nullptr;
         if (prefill_attn_mx()) {
             if (L.q_shift || L.k_shift || L.v_shift)
                 hipLaunchKernelGGL(k_prefill_attn_mx<true>, dim3((M + 7) / 8, 8), dim3(256), 0, s, pw.q, A, M, start,
-                                   m.kv, l, pw.attn, A, pw.rmax, 8, L.q_shift, L.k_shift, L.v_shift);
+                                   m.kv, l, pw.attn, A, as, pw.rsc, M, L.q_shift, L.k_shift, L.v_shift);
             else
                 hipLaunchKernelGGL(k_prefill_attn_mx<false>, dim3((M + 7) / 8, 8), dim3(256), 0, s, pw.q, A, M, start,
-                                   m.kv, l, pw.attn, A, pw.rmax, 8, 0, 0, 0);
-        } else {
-            hipLaunchKernelGGL(k_prefill_attn<PREFILL_ATTN_QB>, dim3((M + PREFILL_ATTN_QB - 1) / PREFILL_ATTN_QB, 8),
-                               dim3(256), 0, s, pw.q, A, M, start, m.kv, l, pw.attn, A);
+                                   m.kv, l, pw.attn, A, as, pw.rsc, M, 0, 0, 0);
             PCHK(hipGetLastError());
-            PCHK(row_absmax(pw.attn, A, M, A, 2 * HEAD_DIM, 8, pw.rmax, s));
+        } else {
+            // f32 rows over the q rows' own (pw.part holds at least M rows of
+            // them): split from there
+            float *out = sp ? pw.part : pw.attn;
+            hipLaunchKernelGGL(k_prefill_attn<PREFILL_ATTN_QB>, dim3((M + PREFILL_ATTN_QB - 1) / PREFILL_ATTN_QB, 8),
+                               dim3(256), 0, s, pw.q, A, M, start, m.kv, l, out, A);
+            PCHK(hipGetLastError());
+            if (sp) PCHK(enqueue_split_rows(out, A, M, A, 1, as, A / 64, pw.rsc, M, s));
         }
-        PCHK(hipGetLastError());
         // o-proj, residual, post-attention norm
-        PCHK(gemm_parts(GemmA{pw.attn, A, nullptr, nullptr, M, pw.rmax, 8, 2 * HEAD_DIM, 0}, L.o, pw, &S, &ld, s));
-        hipLaunchKernelGGL(k_resid_add_inv, dim3(M), dim3(256), 0, s, pw.x, H, pw.part, S, (size_t)M * ld, ld, H,
-                           pw.inv);
-        PCHK(hipGetLastError());
-        // gate|up with SwiGLU (and the down projection's staging range per
-        // 64 columns), down, residual, next layer's input norm
+        if (sp)
+            PCHK(enqueue_mm_parts(RowsSplit{as, A / 64, M, pw.rsc, M, 1.0f}, L.o_f, false, pw.part, &p, s));
+        else
+            PCHK(gemm_parts(GemmA{pw.attn, A, nullptr, nullptr, M}, L.o, pw, &p, s));
+        PCHK(resid(L.post_norm, L.post_shift));
+        // gate|up with SwiGLU, down, residual, next layer's input norm
         PCHK(enqueue_gemm_gateup(m, pw, l, M, s));
-        PCHK(gemm_parts(GemmA{pw.h, m.inter, nullptr, nullptr, M, pw.rmax, down_rslots(m), 64, 0}, L.down, pw, &S,
-                        &ld, s));
-        hipLaunchKernelGGL(k_resid_add_inv, dim3(M), dim3(256), 0, s, pw.x, H, pw.part, S, (size_t)M * ld, ld, H,
-                           pw.inv);
-        PCHK(hipGetLastError());
+        if (sp)
+            PCHK(enqueue_mm_parts(RowsSplit{(const uint8_t *)pw.h, ki, M, pw.rsc, M, 1.0f}, L.down_f, true, pw.part, &p, s));
+        else
+            PCHK(gemm_parts(GemmA{pw.h, m.inter, nullptr, nullptr, M}, L.down, pw, &p, s));
+        const bool last = l + 1 == m.n_layers;
+        PCHK(resid(last ? nullptr : m.layers[l + 1].input_norm, last ? 0 : m.layers[l + 1].in_shift));
     }
     hipLaunchKernelGGL(k_final_rms, dim3(1), dim3(256), 0, s, pw.x + (size_t)(M - 1) * H, m.final_norm, H,
                        hidden_out);

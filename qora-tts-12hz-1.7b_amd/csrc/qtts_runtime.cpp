@@ -23,6 +23,7 @@ using namespace qtts;
 
 struct qtts_w {
     Q4Tiled t;
+    Q4Frag f{};
     Q4Rows rows;
     float *x = nullptr, *y = nullptr, *part = nullptr;
     std::vector<void *> allocs;
@@ -63,8 +64,8 @@ struct qtts_ctx {
     float *d_io = nullptr;                           // API staging, 2 rows of max(hidden,vocab,4096)
     float *d_io2 = nullptr;
     int64_t io_floats = 0;
-    float *d_rmax = nullptr;                         // per-row largest |x| of a GEMM's rows (staging range)
-    int64_t rmax_rows = 0;
+    float *d_mm = nullptr;                           // workspace of the split GEMM's rows (enqueue_mm_rows)
+    size_t mm_floats = 0;
 
     hipGraphExec_t frame_exec[2] = {nullptr, nullptr};   // one and two attention pages per workgroup
     bool gen_started = false;
@@ -118,6 +119,7 @@ struct qtts_prefix {
 // row by row through the decode kernels.  Same for qtts_gemm_q4 rows.
 constexpr int64_t MFMA_MIN_ROWS = 16;
 constexpr int PREFILL_MAX_ROWS = 1024;   // rows per prefill chunk
+constexpr int TEXT_BATCH_ROWS = 256;     // text rows whose partial sums are held at once
 
 // special ids of the prompt layout (generate_new.rs:25-36)
 constexpr uint32_t TTS_PAD_ID = 151671, TTS_EOS_ID = 151673, CODEC_BOS_ID = 2149;
@@ -321,6 +323,23 @@ static int build_tiled(qtts_ctx *c, std::vector<void *> &allocs, const std::vect
     return QTTS_OK;
 }
 
+// The matrix cores' copy of a tiled weight, permuted on the device (the same
+// nibbles and scales; null where the split GEMM does not take the weight).
+static int build_frag(qtts_ctx *c, std::vector<void *> &allocs, const Q4Tiled &t, Q4Frag *out)
+{
+    *out = Q4Frag{};
+    if (!frag_supported(t)) return QTTS_OK;
+    Q4Frag f;
+    const size_t bytes = frag_shape(t, &f);
+    void *mem = nullptr;
+    HIPCHK(c, hipMalloc(&mem, bytes));
+    allocs.push_back(mem);
+    HIPCHK(c, enqueue_frag_build(t, f, (uint8_t *)mem, c->stream));
+    f.data = (const uint8_t *)mem;
+    *out = f;
+    return QTTS_OK;
+}
+
 static void parallel_for(int64_t n, const std::function<void(int64_t, int64_t)> &fn)
 {
     int nt = (int)std::min<int64_t>(std::max(1u, std::thread::hardware_concurrency()), 16);
@@ -409,6 +428,12 @@ static int upload_layer(qtts_ctx *c, const qtts_layer_host &L, int hidden, int h
                      &out->gate_up, nullptr, true));
     snprintf(name, sizeof name, "%sDOWN", pfx);
     RCHK(build_tiled(c, A, {src_of(L.down_proj)}, role_cfg(name, L.down_proj.k), &out->down, nullptr));
+    if (!predictor) {
+        RCHK(build_frag(c, A, out->qkv, &out->qkv_f));
+        RCHK(build_frag(c, A, out->o, &out->o_f));
+        RCHK(build_frag(c, A, out->gate_up, &out->gate_up_f));
+        RCHK(build_frag(c, A, out->down, &out->down_f));
+    }
     RCHK(upload_vec(c, A, L.q_norm, head_dim, &out->q_norm));
     RCHK(upload_vec(c, A, L.k_norm, head_dim, &out->k_norm));
     RCHK(upload_vec(c, A, L.input_norm, hidden, &out->input_norm));
@@ -542,7 +567,7 @@ extern "C" void qtts_ctx_destroy(qtts_ctx *c)
     if (c->d_forced) hipFree(c->d_forced);
     if (c->d_io) hipFree(c->d_io);
     if (c->d_io2) hipFree(c->d_io2);
-    if (c->d_rmax) hipFree(c->d_rmax);
+    if (c->d_mm) hipFree(c->d_mm);
     if (c->d_copy) hipFree(c->d_copy);
     if (c->d_read) hipFree(c->d_read);
     if (c->d_sink) hipFree(c->d_sink);
@@ -583,16 +608,16 @@ static int ensure_io(qtts_ctx *c, int64_t floats)
     return QTTS_OK;
 }
 
-// One float per GEMM row for the rows' largest |x| (grown on demand).
-static int ensure_rmax(qtts_ctx *c, int64_t rows)
+// Workspace of the split GEMM over plain rows (grown on demand).
+static int ensure_mm(qtts_ctx *c, size_t floats)
 {
-    if (rows <= c->rmax_rows) return QTTS_OK;
+    if (floats <= c->mm_floats) return QTTS_OK;
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    if (c->d_rmax) hipFree(c->d_rmax);
-    c->d_rmax = nullptr;
-    c->rmax_rows = 0;
-    HIPCHK(c, hipMalloc(&c->d_rmax, (size_t)rows * sizeof(float)));
-    c->rmax_rows = rows;
+    if (c->d_mm) hipFree(c->d_mm);
+    c->d_mm = nullptr;
+    c->mm_floats = 0;
+    HIPCHK(c, hipMalloc(&c->d_mm, floats * sizeof(float)));
+    c->mm_floats = floats;
     return QTTS_OK;
 }
 
@@ -603,19 +628,20 @@ static int ensure_prefill(qtts_ctx *c, int rows)
     if (c->pf_mem) hipFree(c->pf_mem);
     c->pf_mem = nullptr;
     c->pf = PrefillWs{};
-    const int64_t H = c->tm.hidden, A = 16 * HEAD_DIM, I = c->tm.inter, P = prefill_part_floats(c->tm);
-    const int64_t RS = prefill_rmax_slots(c->tm);
-    const int64_t per_row = H + A + A + I + P + 1 + RS;
+    // split rows take whole chunks of 64 columns, as many bytes as f32 ones
+    const int64_t H = c->tm.hidden, A = 16 * HEAD_DIM, Hs = (H + 63) / 64 * 64, Is = (c->tm.inter + 63) / 64 * 64;
+    const int64_t P = (prefill_part_floats(c->tm, rows) + 3) & ~(int64_t)3, RS = prefill_rsc_slots(c->tm);
     float *base = nullptr;
-    HIPCHK(c, hipMalloc(&base, (size_t)rows * per_row * sizeof(float)));
+    HIPCHK(c, hipMalloc(&base, ((size_t)rows * (H + Hs + A + A + Is + RS + 1) + P) * sizeof(float)));
     c->pf_mem = base;
     c->pf.x = base;
-    c->pf.q = c->pf.x + rows * H;
+    c->pf.xs = c->pf.x + rows * H;
+    c->pf.q = c->pf.xs + rows * Hs;
     c->pf.attn = c->pf.q + rows * A;
     c->pf.h = c->pf.attn + rows * A;
-    c->pf.part = c->pf.h + rows * I;
-    c->pf.rmax = c->pf.part + rows * P;   // 16-byte aligned: every width before it is a multiple of 4
-    c->pf.inv = c->pf.rmax + rows * RS;
+    c->pf.part = c->pf.h + rows * Is;     // every width before it is a multiple of 32
+    c->pf.rsc = c->pf.part + P;
+    c->pf.inv = c->pf.rsc + rows * RS;
     c->pf.cap_rows = rows;
     return QTTS_OK;
 }
@@ -657,6 +683,7 @@ extern "C" int qtts_q4_upload(qtts_ctx *c, const qtts_q4_host *w, qtts_w **out)
     const int64_t G = w->n / 32;
     (void)G;
     int r = build_tiled(c, h->allocs, {src_of(*w)}, role_cfg("GEMV", w->k), &h->t, nullptr);
+    if (r == QTTS_OK) r = build_frag(c, h->allocs, h->t, &h->f);
     if (r == QTTS_OK) r = upload_rows(c, h->allocs, {*w}, &h->rows);
     if (r == QTTS_OK) r = dev_alloc(c, h->allocs, &h->x, (size_t)w->k * 2);
     if (r == QTTS_OK) r = dev_alloc(c, h->allocs, &h->y, (size_t)std::max<int64_t>(w->n, h->t.npad) * 2);
@@ -701,8 +728,9 @@ extern "C" int qtts_gemm_q4(qtts_ctx *c, const qtts_w *w, const float *X, int64_
     RCHK(stage_in(c, X, rows * w->t.k, c->d_io, flags));
     HIPCHK(c, hipMemsetAsync(c->d_io2, 0, rows * w->t.n * sizeof(float), c->stream));
     if (use_mfma(flags, rows) && gemm_supported(w->t)) {
-        RCHK(ensure_rmax(c, rows));
-        HIPCHK(c, enqueue_gemm_rows(w->t, c->d_io, (int)rows, c->d_io2, w->t.n, c->d_rmax, c->stream));
+        // the bound of qtts_gemm_q4_noalloc's scratch, so both run the same launches
+        RCHK(ensure_mm(c, SCRATCH_FLOATS));
+        HIPCHK(c, enqueue_gemm_rows(w->t, w->f, c->d_io, (int)rows, c->d_io2, w->t.n, c->d_mm, SCRATCH_FLOATS, c->stream));
     }
     else
         HIPCHK(c, enqueue_gemv_rows(w->t, c->d_io, (int)rows, c->d_io2, w->part, c->stream));
@@ -724,15 +752,14 @@ extern "C" int qtts_gemm_q4_noalloc(qtts_ctx *c, const qtts_w *w, const float *X
     if (rows == 0) return QTTS_OK;
     // 2^20 rows keep every launch's grid within the device's limits (the
     // matrix-core GEMM's row tiles x column tiles x 256 threads below 2^32)
-    static_assert((size_t)1 << 20 <= SCRATCH_FLOATS, "one float of scratch per row for the rows' ranges");
     if (rows > (1 << 20)) return fail(c, QTTS_ERR_CAPACITY, "at most %d rows", 1 << 20);
     if (!c->scratch) return fail(c, QTTS_ERR_STATE, "no scratch address for device %d", c->device);
     hipSetDevice(c->device);
     const Q4Tiled &t = w->t;
     if (use_mfma(flags, rows) && gemm_supported(t)) {
-        // the rows' largest |x| (the staging range) in the scratch array:
-        // rows <= 2^20 = its size
-        HIPCHK(c, enqueue_gemm_rows(t, X, (int)rows, Y, t.n, c->scratch, c->stream));
+        // the split rows, their factors and partial sums in the scratch array
+        // (more rows than fit go in batches)
+        HIPCHK(c, enqueue_gemm_rows(t, w->f, X, (int)rows, Y, t.n, c->scratch, SCRATCH_FLOATS, c->stream));
     } else {
         const size_t need = (size_t)t.S * 2 * t.npad;
         if (need > SCRATCH_FLOATS)
@@ -866,6 +893,8 @@ static int upload_model(qtts_ctx *c, const qtts_talker_host *t, const qtts_predi
     RCHK(build_tiled(c, A, {src_of(t->codec_head)}, role_cfg("HEAD", t->hidden), &m.codec_head, nullptr));
     RCHK(build_tiled(c, A, {src_of(t->text_fc1)}, role_cfg("TEXT", t->text_fc1.k), &m.text_fc1, nullptr));
     RCHK(build_tiled(c, A, {src_of(t->text_fc2)}, role_cfg("TEXT", t->text_fc2.k), &m.text_fc2, nullptr));
+    RCHK(build_frag(c, A, m.text_fc1, &m.text_fc1_f));
+    RCHK(build_frag(c, A, m.text_fc2, &m.text_fc2_f));
     RCHK(upload_vec(c, A, t->text_fc1_bias, t->text_fc1.n, &m.text_fc1_bias));
     RCHK(upload_vec(c, A, t->text_fc2_bias, t->text_fc2.n, &m.text_fc2_bias));
     RCHK(upload_rows(c, A, {t->codec_embedding}, &m.codec_rows));
@@ -1467,10 +1496,14 @@ static int text_rows(qtts_ctx *c, const uint32_t *d_ids, int n, float *out, floa
     Q4Rows e = m.text_rows;
     e.n = m.text_hidden;
     float *raw = scratch, *h1 = scratch + (size_t)n * m.text_hidden;
-    RCHK(ensure_rmax(c, n));
+    const int batch = std::min(n, TEXT_BATCH_ROWS);
+    const size_t ws = std::max(mm_rows_ws_floats(m.text_fc1_f, batch), mm_rows_ws_floats(m.text_fc2_f, batch));
+    RCHK(ensure_mm(c, ws));
     HIPCHK(c, enqueue_gather_rows(e, d_ids, n, raw, m.text_hidden, c->stream));
-    HIPCHK(c, enqueue_gemm_bias(m.text_fc1, raw, n, m.text_fc1_bias, true, h1, m.text_fc1.n, c->d_rmax, c->stream));
-    HIPCHK(c, enqueue_gemm_bias(m.text_fc2, h1, n, m.text_fc2_bias, false, out, m.hidden, c->d_rmax, c->stream));
+    HIPCHK(c, enqueue_gemm_bias(m.text_fc1, m.text_fc1_f, raw, n, m.text_fc1_bias, true, h1, m.text_fc1.n, c->d_mm, ws,
+                                c->stream));
+    HIPCHK(c, enqueue_gemm_bias(m.text_fc2, m.text_fc2_f, h1, n, m.text_fc2_bias, false, out, m.hidden, c->d_mm, ws,
+                                c->stream));
     return QTTS_OK;
 }
 
@@ -2767,7 +2800,7 @@ extern "C" int qtts_time_prefill(qtts_ctx *c, int64_t rows, int32_t what, int32_
     const int M = (int)rows, H = m.hidden;
     if (what == 0) {
         HIPCHK(c, enqueue_fill_rows(c->pf.x, (int64_t)M * H, 7u, c->stream));
-        HIPCHK(c, enqueue_row_inv(c->pf.x, H, M, H, c->pf.inv, c->stream));
+        HIPCHK(c, enqueue_gateup_input(m, c->pf, 0, M, c->stream));
         *flops = 2.0 * M * H * 2.0 * m.inter;
         return time_launches(c, iters, [&](int i) { return enqueue_gemm_gateup(m, c->pf, i % m.n_layers, M, c->stream); },
                              avg_us);

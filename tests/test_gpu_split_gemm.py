@@ -1,0 +1,82 @@
+"""The split-f16 Q4 GEMM (k_q4_gemm and the kernels around it) at the sizes
+where its tiles end: row blocks of 16, row tiles of up to 96, the rows where
+the K runs change, half chunks of 64 rows of K, K segments of 256, partial
+column tiles, widths that leave stores unaligned.
+
+Each element is held to its own bound against 64 bits.  Every staged value is
+within 2^-22 of the f32 it stands for (hi + lo, and lo lo dropped), and an
+element is at most 24 accumulations a segment (8 chunks of 32, three
+products) plus one per segment, each rounded to f32: |error| <= 2 (2^-22 +
+(24 + segments) 2^-24) sum_k |x_k w_k|, the factor 2 for the sums inside one
+matrix instruction.
+"""
+import numpy as np
+import pytest
+
+from qtts import synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx(ctx_factory):
+    return ctx_factory(256)
+
+
+def bits(a):
+    return np.ascontiguousarray(a, np.float32).view(np.uint32)
+
+
+def check(Y, X, w):
+    W, X = w.dequant().astype(np.float64), X.astype(np.float64)
+    bound = 2 * (2.0 ** -22 + (24 + -(-w.k // 256)) * 2.0 ** -24) * (np.abs(X) @ np.abs(W))
+    err = np.abs(Y.astype(np.float64) - X @ W)
+    assert (err <= bound).all(), f"largest error {np.max(err / np.maximum(bound, 1e-300)):.3g} of its bound"
+
+
+@pytest.mark.parametrize("k,n", [(64, 32), (96, 160), (256, 96), (288, 1500), (2048, 128), (2080, 1000), (6144, 64)])
+def test_rows_and_shapes(ctx, k, n):
+    rng = np.random.Generator(np.random.PCG64(k + n))
+    w = synth.q4_random(rng, k, n)
+    dw = ctx.upload(w)
+    X = rng.standard_normal((225, k)).astype(np.float32)
+    X *= np.exp2(rng.integers(-20, 20, (225, 1))).astype(np.float32)   # every row has its own range
+    whole = ctx.gemm(dw, X, path="mfma")
+    check(whole, X, w)
+    assert not whole[:, n // 32 * 32:].any()
+    for rows in (1, 2, 15, 16, 17, 31, 33, 48, 63, 64, 65, 80, 81, 96, 97, 161):
+        print(f"k={k} n={n} rows={rows}", flush=True)
+        Y = ctx.gemm(dw, X[:rows], path="mfma")
+        assert np.array_equal(bits(Y), bits(whole[:rows])), f"{rows} rows: not the bits of the same rows among 225"
+    dw.free()
+
+
+@pytest.mark.parametrize("k,n,rows", [(6144, 2048, 400), (2048, 12288, 600)])
+def test_rows_in_batches(ctx, k, n, rows):
+    """More rows than the workspace holds at once: the same bits as one by
+    one batch."""
+    rng = np.random.Generator(np.random.PCG64(rows))
+    w = synth.q4_random(rng, k, n)
+    dw = ctx.upload(w)
+    X = rng.standard_normal((rows, k)).astype(np.float32)
+    whole = ctx.gemm(dw, X, path="mfma")
+    at = [0, 15, 159, 160, 161, rows - 1]
+    check(whole[at], X[at], w)
+    for r0 in range(0, rows, 100):
+        assert np.array_equal(bits(ctx.gemm(dw, X[r0:r0 + 100], path="mfma")), bits(whole[r0:r0 + 100]))
+    dw.free()
+
+
+def test_zero_and_not_finite_rows(ctx):
+    """A zero row gives zeros; an inf or NaN stays in its own row."""
+    rng = np.random.Generator(np.random.PCG64(9))
+    w = synth.q4_random(rng, 512, 96)
+    dw = ctx.upload(w)
+    X = rng.standard_normal((40, 512)).astype(np.float32)
+    ref = ctx.gemm(dw, X, path="mfma")
+    X[3], X[5, 7], X[21, 300] = 0.0, np.inf, np.nan
+    Y = ctx.gemm(dw, X, path="mfma")
+    keep = [i for i in range(40) if i not in (3, 5, 21)]
+    assert np.array_equal(bits(Y[keep]), bits(ref[keep]))
+    assert not Y[3].any() and not np.isfinite(Y[5]).any() and not np.isfinite(Y[21]).any()
+    dw.free()
