@@ -41,7 +41,7 @@ extern "C" {
 
 #define QTTS_DEVICE_PTRS   1    /* flags: float buffers are device memory  */
 /* Path choice for qtts_gemm_q4 and qtts_talker_prefill (default: by row
- * count, the matrix cores from 16 rows up). */
+ * count, the matrix cores from 3 rows up). */
 #define QTTS_PATH_ROWWISE  2    /* flags: one GEMV pass per row            */
 #define QTTS_PATH_MFMA     4    /* flags: matrix-core GEMM at any row count */
 
@@ -224,8 +224,8 @@ int qtts_gemv_q4(qtts_ctx *ctx, const qtts_w *w, const float *x, float *y,
                  int flags);
 
 /* Y[rows][n] = X[rows][k] * W.  Replaces `gemm` (gemv.rs:157-162) ->
- * `gemm_q4` (gemv.rs:349-412).  From 16 rows (k a multiple of 32, at least
- * 64) an f32 matrix-core GEMM; fewer rows run the GEMV, two rows per pass
+ * `gemm_q4` (gemv.rs:349-412).  From 3 rows (k a multiple of 32, at least
+ * 64) an f32-accurate matrix-core GEMM; fewer rows run the GEMV, two rows per pass
  * over W.  flags may force either path (QTTS_PATH_*). */
 int qtts_gemm_q4(qtts_ctx *ctx, const qtts_w *w, const float *X, int64_t rows,
                  float *Y, int flags);
@@ -233,13 +233,14 @@ int qtts_gemm_q4(qtts_ctx *ctx, const qtts_w *w, const float *X, int64_t rows,
 /* qtts_gemm_q4 on DEVICE pointers X [rows][k] and Y [rows][n] that
  * allocates nothing: no reference counterpart.  For callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving
- * loops).  The GEMV passes' split-K partial sums use a 4 MiB device array
- * held by the library on each GPU until the process ends; a weight whose
- * passes need more (S * 2 * npad floats, S = ceil(k / 2048) for the
- * default tile) is refused with QTTS_ERR_CAPACITY.  Only enqueues on the
+ * loops).  The GEMV passes' split-K partial sums and the matrix cores' staged
+ * rows use 4 MiB of device memory that the context holds (rows that do not
+ * fit go in batches); a weight whose GEMV passes need more (S * 2 * npad
+ * floats, S = ceil(k / 2048) for the default tile) is refused with
+ * QTTS_ERR_CAPACITY.  Only enqueues on the
  * context stream (no synchronisation; qtts_sync or the stream from
- * qtts_stream orders the results).  Calls that overlap on one GPU share
- * that array and race.  At most 2^20 rows per call (QTTS_ERR_CAPACITY
+ * qtts_stream orders the results; launches captured from it and replayed on
+ * another stream share the context's 4 MiB with its later calls).  At most 2^20 rows per call (QTTS_ERR_CAPACITY
  * beyond).  flags: QTTS_PATH_* as for qtts_gemm_q4. */
 int qtts_gemm_q4_noalloc(qtts_ctx *ctx, const qtts_w *w, const float *X,
                          int64_t rows, float *Y, int flags);
@@ -311,7 +312,7 @@ int qtts_talker_decode_token(qtts_ctx *ctx, uint32_t token, int is_text,
  * start_pos..start_pos+seq-1 on top of the cached prefix:
  * `prefill_talker_raw_from` (talker.rs:379-482).  Requires
  * kv_len == start_pos.  Writes the last row's final-normed hidden.  From
- * 16 rows the layers run as batched matrix-core GEMMs (chunks of up to
+ * 3 rows the layers run as batched matrix-core GEMMs (chunks of up to
  * 1024 rows); fewer rows go one by one through the decode kernels.  flags
  * may force either path (QTTS_PATH_*). */
 int qtts_talker_prefill(qtts_ctx *ctx, const float *X, int64_t seq,

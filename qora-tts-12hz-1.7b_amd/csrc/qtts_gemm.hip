@@ -600,8 +600,15 @@ hipError_t enqueue_mm_rows(const Q4Frag &w, const float *X, int ld, int rows, co
 {
     const size_t per_row = (size_t)w.kc * 64 + 1, ncols = (size_t)w.ng * 32;
     const int tn = (w.ng + 3) / 4, nseg = mm_segments(w);
-    // bias and SiLU are applied where the partial sums are added
-    size_t cap = ws_floats / (per_row + (bias || silu ? (size_t)nseg * ncols : 0));
+    // One workgroup per (tile, K segment) and partial sums where tiles alone
+    // would leave CUs idle: 24 x 6144 x 2048 takes 38 us so (two batches that
+    // fit the workspace), 58 us as 16 long K loops; past two batches the long
+    // loops have the rows to fill the chip.  Bias and SiLU are applied where
+    // partial sums are added.
+    const size_t cap_parts = ws_floats / (per_row + (size_t)nseg * ncols);
+    const bool parts = bias || silu ||
+                       ((int64_t)((rows + 79) / 80) * tn < 192 && (size_t)rows <= 2 * (cap_parts & ~(size_t)15));
+    size_t cap = parts ? cap_parts : ws_floats / per_row;
     if (cap < 1) return hipErrorInvalidValue;
     if (cap >= 16) cap &= ~(size_t)15;
     for (int r0 = 0; r0 < rows; r0 += (int)cap) {
@@ -609,8 +616,6 @@ hipError_t enqueue_mm_rows(const Q4Frag &w, const float *X, int ld, int rows, co
         // split rows first (16-byte aligned), then the parts, then the factors
         uint8_t *sp = (uint8_t *)ws;
         float *part = ws + (size_t)M * w.kc * 64;
-        const bool fits = per_row * M + (size_t)nseg * M * ncols <= ws_floats;
-        const bool parts = bias || silu || (fits && (int64_t)((M + 79) / 80) * tn < 192);
         float *rsc = part + (parts ? (size_t)nseg * M * ncols : 0);
         GCHK(enqueue_split_rows(X + (size_t)r0 * ld, ld, M, w.k, 0, sp, w.kc, rsc, 0, s));
         const RowsSplit a{sp, w.kc, M, rsc, 0, 1.0f};

@@ -14,7 +14,6 @@
 #include <cstdlib>
 #include <cstring>
 #include <functional>
-#include <mutex>
 #include <string>
 #include <thread>
 #include <vector>
@@ -71,7 +70,7 @@ struct qtts_ctx {
     bool gen_started = false;
     bool force_sync_err = false;                     // qtts_debug_force_sync_err: armed for the next call
 
-    float *scratch = nullptr;                        // this device's copy of `scratch` (qtts_gemm_q4_noalloc)
+    float *scratch = nullptr;                        // qtts_gemm_q4_noalloc's workspace, SCRATCH_FLOATS
 
     float *d_copy = nullptr;                         // copy-calibration buffers, 2 x copy_floats
     int64_t copy_floats = 0;
@@ -116,8 +115,12 @@ struct qtts_prefix {
 };
 
 // Prompts at least this long take the matrix-core prefill; shorter ones run
-// row by row through the decode kernels.  Same for qtts_gemm_q4 rows.
-constexpr int64_t MFMA_MIN_ROWS = 16;
+// row by row through the decode kernels.  Same for qtts_gemm_q4 rows.  The
+// 28-layer prefill of 2 / 3 / 10 rows takes 1.51 / 1.5 / 1.56 ms on the
+// matrix cores and 1.3 / 1.9 / 6.4 ms row by row; 2048 x 4096 over 2 / 3 / 8
+// rows 9.6 / 11 / 12 us and 7.0 / 13 / 27 us.  Both are as far from 64 bits
+// (2e-7 of a product, 1.3e-7 of the prefill's hidden).
+constexpr int64_t MFMA_MIN_ROWS = 3;
 constexpr int PREFILL_MAX_ROWS = 1024;   // rows per prefill chunk
 constexpr int TEXT_BATCH_ROWS = 256;     // text rows whose partial sums are held at once
 
@@ -469,34 +472,11 @@ static void drop_graph(qtts_ctx *c)
     }
 }
 
-// ---------------------------------------------------------------------------
-// scratch of the allocation-free entry point (qtts_gemm_q4_noalloc): the
-// split-K partial sums of its GEMV passes live in this file-scope device
-// array, one copy per GPU, held until the process ends.  Host code never
-// passes the array's name to a kernel (on the host it is only a stand-in):
-// its device address is looked up once per device, with that device
-// current, when the first context on the device is created.
-// ---------------------------------------------------------------------------
-
+// Workspace of the allocation-free entry point (qtts_gemm_q4_noalloc): the
+// split-K partial sums of its GEMV passes, the matrix cores' split rows,
+// factors and partial sums.  One per context, allocated with it, so that
+// calls of different contexts (threads, streams) do not share it.
 constexpr size_t SCRATCH_FLOATS = (size_t)1 << 20;    // 4 MiB
-constexpr int SCRATCH_MAX_DEVICES = 64;
-static __device__ __align__(256) float scratch[SCRATCH_FLOATS];
-static std::mutex g_scratch_mu;
-static float *g_scratch_dev[SCRATCH_MAX_DEVICES];      // device address of `scratch` per device
-
-static hipError_t scratch_address(int device, float **out)
-{
-    std::lock_guard<std::mutex> lock(g_scratch_mu);
-    if (device < 0 || device >= SCRATCH_MAX_DEVICES) return hipErrorInvalidDevice;
-    if (!g_scratch_dev[device]) {
-        void *p = nullptr;
-        const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-        if (e != hipSuccess) return e;
-        g_scratch_dev[device] = (float *)p;
-    }
-    *out = g_scratch_dev[device];
-    return hipSuccess;
-}
 
 extern "C" int qtts_ctx_create(int device, int64_t kv_capacity, qtts_ctx **out)
 {
@@ -518,12 +498,8 @@ extern "C" int qtts_ctx_create(int device, int64_t kv_capacity, qtts_ctx **out)
         delete c;
         return QTTS_ERR_HIP;
     }
-    if (scratch_address(device, &c->scratch) != hipSuccess) {
-        hipStreamDestroy(c->stream);
-        delete c;
-        return QTTS_ERR_HIP;
-    }
-    bool ok = hipMalloc(&c->st_gen, sizeof(DevState)) == hipSuccess &&
+    bool ok = hipMalloc(&c->scratch, SCRATCH_FLOATS * sizeof(float)) == hipSuccess &&
+              hipMalloc(&c->st_gen, sizeof(DevState)) == hipSuccess &&
               hipMalloc(&c->st_api, sizeof(DevState)) == hipSuccess &&
               hipHostMalloc(&c->h_st, sizeof(DevState), hipHostMallocDefault) == hipSuccess &&
               hipHostMalloc(&c->h_ring, sizeof(uint32_t) * RING_FRAMES * 16 * 2, hipHostMallocDefault) == hipSuccess &&
@@ -568,6 +544,7 @@ extern "C" void qtts_ctx_destroy(qtts_ctx *c)
     if (c->d_io) hipFree(c->d_io);
     if (c->d_io2) hipFree(c->d_io2);
     if (c->d_mm) hipFree(c->d_mm);
+    if (c->scratch) hipFree(c->scratch);
     if (c->d_copy) hipFree(c->d_copy);
     if (c->d_read) hipFree(c->d_read);
     if (c->d_sink) hipFree(c->d_sink);
@@ -739,12 +716,10 @@ extern "C" int qtts_gemm_q4(qtts_ctx *c, const qtts_w *w, const float *X, int64_
     return QTTS_OK;
 }
 
-// qtts_gemm_q4 on device rows, allocating nothing: the GEMV passes' partial
-// sums go to this device's `scratch` (its address looked up when the
-// context was created), the ragged columns are cleared by a fill kernel,
-// and nothing is staged, so the call only enqueues kernels on the context
-// stream and returns.  Calls that overlap on one GPU (other contexts,
-// other host threads) share the array and race.
+// qtts_gemm_q4 on device rows, allocating nothing: the context's `scratch`
+// holds what the launches hand to each other, the ragged columns are cleared
+// by a fill kernel, and nothing is staged, so the call only enqueues kernels
+// on the context stream and returns.
 extern "C" int qtts_gemm_q4_noalloc(qtts_ctx *c, const qtts_w *w, const float *X, int64_t rows, float *Y,
                                     int flags)
 {
@@ -753,12 +728,10 @@ extern "C" int qtts_gemm_q4_noalloc(qtts_ctx *c, const qtts_w *w, const float *X
     // 2^20 rows keep every launch's grid within the device's limits (the
     // matrix-core GEMM's row tiles x column tiles x 256 threads below 2^32)
     if (rows > (1 << 20)) return fail(c, QTTS_ERR_CAPACITY, "at most %d rows", 1 << 20);
-    if (!c->scratch) return fail(c, QTTS_ERR_STATE, "no scratch address for device %d", c->device);
     hipSetDevice(c->device);
     const Q4Tiled &t = w->t;
     if (use_mfma(flags, rows) && gemm_supported(t)) {
-        // the split rows, their factors and partial sums in the scratch array
-        // (more rows than fit go in batches)
+        // more rows than the scratch holds go in batches
         HIPCHK(c, enqueue_gemm_rows(t, w->f, X, (int)rows, Y, t.n, c->scratch, SCRATCH_FLOATS, c->stream));
     } else {
         const size_t need = (size_t)t.S * 2 * t.npad;
