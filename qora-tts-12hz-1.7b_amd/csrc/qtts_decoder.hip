@@ -1423,6 +1423,10 @@ hipError_t enqueue_decode(const DecoderDev &d, const DecoderWs &ws, const uint32
         DCHK(conv_gemm<CE_SCALE_RES>(U.pw2, U.ch, causal_in(ws.d, U.inner, L, 1, 1), po, L, ws, s));
         std::swap(sig, other);
     }
+    if (d.vocos_rows && !ws.f32 && dec_x3()) {
+        float *const bufs[4] = {ws.c, ws.d, ws.e, other};
+        return enqueue_vocos(d, ws, sig, bufs, L, cut, audio, dec_fuse_voc(), s);
+    }
     // 5. Vocos: init conv with the first block's pre-snake (or the final
     // snake) fused
     const float *na = d.n_voc ? d.voc[0].pre_alpha : d.final_alpha;

@@ -156,10 +156,14 @@ inline bool conv_tap_major(int ic, int k) { return k == 1 || ic % 32 == 0; }
 struct DecConv {
     const float *w, *b;      // w [oc][k][ic] when conv_tap_major(ic, k), else [oc][ic][k]
     int ic, oc, k, dil;
+    const uint8_t *pw;       // split weights in fragment order (qtts_dconv.hip), their rows' factors
+    const float *un;
 };
 struct DecConvT {            // kernel == stride (1 tap) or 2*stride (2 taps), padding 0
     const float *phases, *b; // [stride][oc] rows of ic x taps (tap-major as DecConv); 2 taps: x[i-1] (kernel tap r+stride), x[i] (tap r)
     int ic, oc, stride, taps;
+    const uint8_t *pw;       // as DecConv, rows [stride][oc]
+    const float *un;
 };
 struct DecLayer {
     const float *qkv;        // [3A][hidden] rows q, k, v
@@ -180,10 +184,11 @@ struct DecUpsample {
 };
 struct DecVocosRes {
     const float *a1_alpha, *a1_beta, *a2_alpha, *a2_beta;
+    const float *a1_par, *a2_par;   // [2][ch] e^alpha, e^-beta (qtts_dconv.hip)
     DecConv c1, c2;
 };
 struct DecVocos {
-    const float *pre_alpha, *pre_beta;
+    const float *pre_alpha, *pre_beta, *pre_par;
     DecConvT up;
     const DecVocosRes *res;  // host array
     int n_res;
@@ -203,12 +208,13 @@ struct DecoderDev {
     DecConv voc_init;
     const DecVocos *voc;                  // host array
     int n_voc;
-    const float *final_alpha, *final_beta;
+    const float *final_alpha, *final_beta, *final_par;
     const float *out_w;                   // [ch][k], one output channel
     float out_b;
     int out_k, out_dil;
     const float *rope_cos, *rope_sin;
     int64_t rope_rows;
+    bool vocos_rows;                      // the Vocos stages run position-major (qtts_dconv.hip)
     bool weights_f32;                     // a weight matrix outside the split-f16 range: f32 matrix path
 };
 struct DecoderWs {
@@ -319,6 +325,12 @@ hipError_t enqueue_talker_prefill(const TalkerDev &m, const PrefillWs &pw, int M
                                   float *hidden_out, hipStream_t s);
 hipError_t enqueue_decode(const DecoderDev &d, const DecoderWs &ws, const uint32_t *codes, int T, int64_t cut,
                           float *audio, hipStream_t s);
+bool vocos_fits(const DecoderDev &d);
+size_t dconv_weight_bytes(int rows, int ic, int kt);
+hipError_t enqueue_dconv_pack(const float *w, int rows, int ic, int kt, uint8_t *out, float *un, hipStream_t s);
+hipError_t enqueue_snake_par(const float *alpha, const float *beta, int n, float *out, hipStream_t s);
+hipError_t enqueue_vocos(const DecoderDev &d, const DecoderWs &ws, const float *sig, float *const bufs[4], int L, int64_t cut,
+                         float *audio, bool fuse, hipStream_t s);
 double decode_flops(const DecoderDev &d, int T);
 hipError_t enqueue_gateup_timing(const TalkerDev &m, const Workspace &ws, int l, hipStream_t s);
 hipError_t enqueue_attn_timing(const TalkerDev &m, const Workspace &ws, int l, int slot, int64_t pos,

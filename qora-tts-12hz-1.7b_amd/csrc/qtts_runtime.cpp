@@ -1805,6 +1805,48 @@ static int upload_convt(qtts_ctx *c, const qtts_convt1d_host &h, DecConvT *d)
     return upload_vec(c, c->dec_allocs, h.bias, (size_t)OC, &d->b);
 }
 
+// The position-major Vocos stages' copies: split weights in fragment order
+// and the snakes' exponentials, made on the device from what was uploaded
+// (the f32 weights stay for the f32 matrix path).
+static int pack_vocos(qtts_ctx *c)
+{
+    DecoderDev &d = c->dec;
+    d.vocos_rows = vocos_fits(d);
+    if (!d.vocos_rows) return QTTS_OK;
+    const auto conv = [&](const float *w, int rows, int ic, int kt, const uint8_t **pw, const float **un) {
+        uint8_t *p = nullptr;
+        float *u = nullptr;
+        RCHK(dev_alloc(c, c->dec_allocs, &p, dconv_weight_bytes(rows, ic, kt)));
+        RCHK(dev_alloc(c, c->dec_allocs, &u, rows));
+        HIPCHK(c, enqueue_dconv_pack(w, rows, ic, kt, p, u, c->stream));
+        *pw = p;
+        *un = u;
+        return QTTS_OK;
+    };
+    const auto snake = [&](const float *alpha, const float *beta, int n, const float **out) {
+        float *p = nullptr;
+        RCHK(dev_alloc(c, c->dec_allocs, &p, 2 * (size_t)n));
+        HIPCHK(c, enqueue_snake_par(alpha, beta, n, p, c->stream));
+        *out = p;
+        return QTTS_OK;
+    };
+    RCHK(conv(d.voc_init.w, d.voc_init.oc, d.voc_init.ic, d.voc_init.k, &d.voc_init.pw, &d.voc_init.un));
+    int ch = d.voc_init.oc;
+    for (int b = 0; b < d.n_voc; b++) {
+        DecVocos &B = c->dec_voc[b];
+        RCHK(snake(B.pre_alpha, B.pre_beta, ch, &B.pre_par));
+        ch = B.up.oc;
+        RCHK(conv(B.up.phases, B.up.stride * ch, B.up.ic, B.up.taps, &B.up.pw, &B.up.un));
+        for (DecVocosRes &R : c->dec_res[b]) {
+            RCHK(snake(R.a1_alpha, R.a1_beta, ch, &R.a1_par));
+            RCHK(snake(R.a2_alpha, R.a2_beta, ch, &R.a2_par));
+            RCHK(conv(R.c1.w, ch, ch, R.c1.k, &R.c1.pw, &R.c1.un));
+            RCHK(conv(R.c2.w, ch, ch, 1, &R.c2.pw, &R.c2.un));
+        }
+    }
+    return snake(d.final_alpha, d.final_beta, ch, &d.final_par);
+}
+
 static int upload_decoder(qtts_ctx *c, const qtts_decoder_host *h)
 {
     DecoderDev &d = c->dec;
@@ -1956,7 +1998,7 @@ static int upload_decoder(qtts_ctx *c, const qtts_decoder_host *h)
     RCHK(upload_vec(c, A, h->rope_sin, (size_t)h->rope_max_pos * (HD / 2), &d.rope_sin));
     d.rope_rows = h->rope_max_pos;
     c->dec_floats_per_frame = fpf;
-    return QTTS_OK;
+    return pack_vocos(c);
 }
 
 static void free_decoder(qtts_ctx *c)

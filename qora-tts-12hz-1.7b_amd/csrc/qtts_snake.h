@@ -22,7 +22,7 @@ namespace qtts {
 // a correctly rounded sin in f32 (1.2e-7 absolute); larger |t|, inf and NaN
 // take sinf.  No branch on the common path.
 #if defined(__HIPCC__)
-__host__ __device__ __attribute__((noinline))
+static __host__ __device__ __attribute__((noinline))
 #else
 static
 #endif
