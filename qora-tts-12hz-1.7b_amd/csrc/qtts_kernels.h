@@ -234,6 +234,15 @@ struct SampleArgsHost {
     int n_prev;
 };
 
+// 32-bit words copied by one launch (pinned host memory or device memory on
+// either side).
+constexpr int MOVE_SEGS = 4;
+struct MoveList {
+    struct { const void *src; void *dst; uint32_t words; } seg[MOVE_SEGS];
+};
+hipError_t enqueue_move(const MoveList &l, int n, hipStream_t s);
+hipError_t enqueue_page_copy(const KvPaged &kv, int n_layers, int src, int dst, hipStream_t s);
+
 hipError_t enqueue_gemv_plain(const Q4Tiled &w, const float *x, int NB, int ld, float *part, hipStream_t st);
 hipError_t enqueue_gemv_store(const Q4Tiled &w, const float *x, float *y, const float *bias, float *part,
                               hipStream_t st);

@@ -15,6 +15,8 @@
 #include "qtts_kernels.h"
 #include "qtts_devutil.h"
 
+#include <algorithm>
+
 namespace qtts {
 
 // out[i][j] = row ids[i] of e, j < e.n.  Grid (column blocks, rows).
@@ -74,6 +76,44 @@ hipError_t enqueue_add_rows(const float *a, int lda, const float *b, int ldb, fl
 {
     if (rows < 1) return hipSuccess;
     hipLaunchKernelGGL(k_add_rows, dim3((n + 255) / 256, rows), dim3(256), 0, s, a, lda, b, ldb, out, ldo, n);
+    return hipGetLastError();
+}
+
+// Words between pinned host memory and the device (or either side alone): a
+// kernel on the stream costs about 3 us and keeps the host free; small copies
+// through the runtime took 6 to 10 with their hand-over between engines.
+__global__ void __launch_bounds__(256)
+k_move(MoveList l)
+{
+    const uint32_t *src = (const uint32_t *)l.seg[blockIdx.y].src;
+    uint32_t *dst = (uint32_t *)l.seg[blockIdx.y].dst;
+    const uint32_t n = l.seg[blockIdx.y].words;
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) dst[i] = src[i];
+}
+
+hipError_t enqueue_move(const MoveList &l, int n, hipStream_t s)
+{
+    if (n < 1 || n > MOVE_SEGS) return hipErrorInvalidValue;
+    uint32_t most = 1;
+    for (int i = 0; i < n; i++) most = std::max(most, l.seg[i].words);
+    hipLaunchKernelGGL(k_move, dim3(std::min<uint32_t>((most + 255) / 256, 128), n), dim3(256), 0, s, l);
+    return hipGetLastError();
+}
+
+// One physical KV page to another in every layer: 512 KB a layer, eight
+// workgroups each (28 layers in one launch, 28 copies otherwise).
+__global__ void __launch_bounds__(256)
+k_page_copy(KvPaged kv, int src, int dst)
+{
+    constexpr int N = 2 * 8 * KV_PAGE * HEAD_DIM;
+    float *b = kv.base + (size_t)blockIdx.y * kv.n_phys * N;
+    for (int i = 4 * (blockIdx.x * 256 + threadIdx.x); i < N; i += 4 * 256 * 8)
+        *(f32x4 *)(b + (size_t)dst * N + i) = ld4(b + (size_t)src * N + i);
+}
+
+hipError_t enqueue_page_copy(const KvPaged &kv, int n_layers, int src, int dst, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_page_copy, dim3(8, n_layers), dim3(256), 0, s, kv, src, dst);
     return hipGetLastError();
 }
 

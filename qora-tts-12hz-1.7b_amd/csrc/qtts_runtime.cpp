@@ -60,6 +60,16 @@ struct qtts_ctx {
     float *leg_buf = nullptr;                        // side row + logits
     int *d_status = nullptr;
     int64_t lkv_len = 0;
+    // small host arguments and results go through pinned memory that a copy
+    // kernel reads and writes on the context stream (stage_in, finish)
+    uint8_t *h_pin = nullptr;                        // PIN_BYTES
+    size_t pin_top = 0;                              // taken since the last synchronisation
+    struct OutCopy { const void *dev; uint8_t *pin; void *host; size_t bytes; };
+    std::vector<OutCopy> outs;                       // results to hand over at the next finish()
+    int32_t *h_err = nullptr;                        // pinned copy of sync_err
+
+    uint8_t *arena = nullptr;                        // DevScratch of the prompt calls (ARENA_BYTES), a stack
+    size_t arena_top = 0;
     float *d_io = nullptr;                           // API staging, 2 rows of max(hidden,vocab,4096)
     float *d_io2 = nullptr;
     int64_t io_floats = 0;
@@ -122,6 +132,9 @@ struct qtts_prefix {
 // (2e-7 of a product, 1.3e-7 of the prefill's hidden).
 constexpr int64_t MFMA_MIN_ROWS = 3;
 constexpr int PREFILL_MAX_ROWS = 1024;   // rows per prefill chunk
+constexpr size_t PIN_BYTES = (size_t)1 << 20;    // pinned staging per context
+constexpr size_t PIN_MAX = (size_t)128 << 10;    // larger arguments are copied by the runtime
+constexpr size_t ARENA_BYTES = (size_t)64 << 20;
 constexpr int TEXT_BATCH_ROWS = 256;     // text rows whose partial sums are held at once
 
 // special ids of the prompt layout (generate_new.rs:25-36)
@@ -142,6 +155,7 @@ static int fail(qtts_ctx *c, int code, const char *fmt, ...)
         vsnprintf(buf, sizeof buf, fmt, ap);
         va_end(ap);
         c->err = buf;
+        c->outs.clear();     // a failed call hands over nothing
     }
     return code;
 }
@@ -499,6 +513,8 @@ extern "C" int qtts_ctx_create(int device, int64_t kv_capacity, qtts_ctx **out)
         return QTTS_ERR_HIP;
     }
     bool ok = hipMalloc(&c->scratch, SCRATCH_FLOATS * sizeof(float)) == hipSuccess &&
+              hipHostMalloc(&c->h_pin, PIN_BYTES, hipHostMallocDefault) == hipSuccess &&
+              hipHostMalloc(&c->h_err, sizeof(int32_t), hipHostMallocDefault) == hipSuccess &&
               hipMalloc(&c->st_gen, sizeof(DevState)) == hipSuccess &&
               hipMalloc(&c->st_api, sizeof(DevState)) == hipSuccess &&
               hipHostMalloc(&c->h_st, sizeof(DevState), hipHostMallocDefault) == hipSuccess &&
@@ -545,6 +561,9 @@ extern "C" void qtts_ctx_destroy(qtts_ctx *c)
     if (c->d_io2) hipFree(c->d_io2);
     if (c->d_mm) hipFree(c->d_mm);
     if (c->scratch) hipFree(c->scratch);
+    if (c->arena) hipFree(c->arena);
+    if (c->h_pin) hipHostFree(c->h_pin);
+    if (c->h_err) hipHostFree(c->h_err);
     if (c->d_copy) hipFree(c->d_copy);
     if (c->d_read) hipFree(c->d_read);
     if (c->d_sink) hipFree(c->d_sink);
@@ -629,22 +648,90 @@ static bool use_mfma(int flags, int64_t rows)
     return (flags & QTTS_PATH_MFMA) || rows >= MFMA_MIN_ROWS;
 }
 
-// Copy n floats in (host or device source) to a device buffer.
+// A slot of the pinned staging buffer, or null (full, or too large for it).
+static uint8_t *pin_take(qtts_ctx *c, size_t bytes)
+{
+    if (bytes > PIN_MAX || c->pin_top + bytes > PIN_BYTES) return nullptr;
+    uint8_t *p = c->h_pin + c->pin_top;
+    c->pin_top += (bytes + 255) & ~(size_t)255;
+    return p;
+}
+
+// Copy n floats in (host or device source) to a device buffer.  A small host
+// array goes through pinned memory and a copy kernel: 3 us on the stream and
+// no wait on the host, where a copy of pageable memory blocks it for about 8.
 static int stage_in(qtts_ctx *c, const float *src, int64_t n, float *dst, int flags)
 {
-    HIPCHK(c, hipMemcpyAsync(dst, src, n * sizeof(float),
+    const size_t bytes = (size_t)n * sizeof(float);
+    uint8_t *pin = flags & QTTS_DEVICE_PTRS ? nullptr : pin_take(c, bytes);
+    if (pin) {
+        memcpy(pin, src, bytes);
+        HIPCHK(c, enqueue_move(MoveList{{{pin, dst, (uint32_t)n}}}, 1, c->stream));
+        return QTTS_OK;
+    }
+    HIPCHK(c, hipMemcpyAsync(dst, src, bytes,
                              (flags & QTTS_DEVICE_PTRS) ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice,
                              c->stream));
     return QTTS_OK;
 }
 
+static int stage_ids(qtts_ctx *c, const uint32_t *src, int64_t n, uint32_t *dst)
+{
+    return stage_in(c, (const float *)src, n, (float *)dst, 0);
+}
+
+// n floats of a result to the caller's buffer.  A small host result is handed
+// over by the next finish(): src keeps its value until then.
 static int stage_out(qtts_ctx *c, const float *src, int64_t n, float *dst, int flags)
 {
     if (!dst) return QTTS_OK;
-    HIPCHK(c, hipMemcpyAsync(dst, src, n * sizeof(float),
+    const size_t bytes = (size_t)n * sizeof(float);
+    uint8_t *pin = flags & QTTS_DEVICE_PTRS ? nullptr : pin_take(c, bytes);
+    if (pin) {
+        c->outs.push_back({src, pin, dst, bytes});
+        return QTTS_OK;
+    }
+    HIPCHK(c, hipMemcpyAsync(dst, src, bytes,
                              (flags & QTTS_DEVICE_PTRS) ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost,
                              c->stream));
     return QTTS_OK;
+}
+
+// The end of a call: results to pinned memory in one launch, the wait, and
+// the results to the caller's buffers.  err: sync_err comes along in h_err.
+static int finish(qtts_ctx *c, bool err = false)
+{
+    MoveList l{};
+    int n = 0;
+    if (err) l.seg[n++] = {&c->st_gen->sync_err, c->h_err, 1};
+    for (const auto &o : c->outs) {
+        if (o.dev != o.pin) l.seg[n++] = {o.dev, o.pin, (uint32_t)(o.bytes / sizeof(float))};
+        if (n == MOVE_SEGS) {
+            HIPCHK(c, enqueue_move(l, n, c->stream));
+            n = 0;
+        }
+    }
+    if (n) HIPCHK(c, enqueue_move(l, n, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    for (const auto &o : c->outs) memcpy(o.host, o.pin, o.bytes);
+    c->outs.clear();
+    c->pin_top = 0;
+    return QTTS_OK;
+}
+
+// Where a kernel writes a result of n floats: the pinned slot itself (one
+// launch less), else `dev`; hand_over() after it, then finish().
+static float *out_buffer(qtts_ctx *c, int64_t n, float *dst, float *dev, int flags)
+{
+    uint8_t *pin = (flags & QTTS_DEVICE_PTRS) ? nullptr : pin_take(c, (size_t)n * sizeof(float));
+    if (!pin) return dev;
+    c->outs.push_back({pin, pin, dst, (size_t)n * sizeof(float)});
+    return (float *)pin;
+}
+
+static int hand_over(qtts_ctx *c, float *out, int64_t n, float *dst, float *dev, int flags)
+{
+    return out == dev ? stage_out(c, dev, n, dst, flags) : QTTS_OK;
 }
 
 // ---------------------------------------------------------------------------
@@ -687,14 +774,14 @@ extern "C" int qtts_gemv_q4(qtts_ctx *c, const qtts_w *w, const float *x, float 
 {
     if (!c || !w || !x || !y) return QTTS_ERR_INVALID;
     RCHK(stage_in(c, x, w->t.k, w->x, flags));
-    HIPCHK(c, enqueue_gemv_store(w->t, w->x, w->y, nullptr, w->part, c->stream));
+    const int64_t full = (int64_t)(w->t.n / 32) * 32;
+    float *out = out_buffer(c, w->t.n, y, w->y, flags);
+    HIPCHK(c, enqueue_gemv_store(w->t, w->x, out, nullptr, w->part, c->stream));
     // columns past the last full group stay zero (gemv.rs:255 starts from
     // vec![0.0; n] and only full groups are accumulated)
-    const int64_t full = (int64_t)(w->t.n / 32) * 32;
-    if (full < w->t.n) HIPCHK(c, hipMemsetAsync(w->y + full, 0, (w->t.n - full) * sizeof(float), c->stream));
-    RCHK(stage_out(c, w->y, w->t.n, y, flags));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return QTTS_OK;
+    if (full < w->t.n) HIPCHK(c, enqueue_zero_cols(out, 1, w->t.n, (int)full, w->t.n, c->stream));
+    RCHK(hand_over(c, out, w->t.n, y, w->y, flags));
+    return finish(c);
 }
 
 extern "C" int qtts_gemm_q4(qtts_ctx *c, const qtts_w *w, const float *X, int64_t rows, float *Y, int flags)
@@ -703,7 +790,6 @@ extern "C" int qtts_gemm_q4(qtts_ctx *c, const qtts_w *w, const float *X, int64_
     if (rows == 0) return QTTS_OK;
     RCHK(ensure_io(c, rows * std::max({w->t.k, w->t.n, w->t.npad})));
     RCHK(stage_in(c, X, rows * w->t.k, c->d_io, flags));
-    HIPCHK(c, hipMemsetAsync(c->d_io2, 0, rows * w->t.n * sizeof(float), c->stream));
     if (use_mfma(flags, rows) && gemm_supported(w->t)) {
         // the bound of qtts_gemm_q4_noalloc's scratch, so both run the same launches
         RCHK(ensure_mm(c, SCRATCH_FLOATS));
@@ -711,9 +797,10 @@ extern "C" int qtts_gemm_q4(qtts_ctx *c, const qtts_w *w, const float *X, int64_
     }
     else
         HIPCHK(c, enqueue_gemv_rows(w->t, c->d_io, (int)rows, c->d_io2, w->part, c->stream));
+    // columns past the last full group are zero (gemv.rs:255)
+    HIPCHK(c, enqueue_zero_cols(c->d_io2, (int)rows, w->t.n, (w->t.n / 32) * 32, w->t.n, c->stream));
     RCHK(stage_out(c, c->d_io2, rows * w->t.n, Y, flags));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return QTTS_OK;
+    return finish(c);
 }
 
 // qtts_gemm_q4 on device rows, allocating nothing: the context's `scratch`
@@ -755,8 +842,7 @@ extern "C" int qtts_embed_lookup_q4(qtts_ctx *c, const qtts_w *w, int64_t row, f
     e.n = e.G * 32;
     HIPCHK(c, enqueue_embed_row(e, nullptr, (uint32_t)row, w->y, c->stream));
     RCHK(stage_out(c, w->y, w->rows.n, out, flags));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return QTTS_OK;
+    return finish(c);
 }
 
 // ---------------------------------------------------------------------------
@@ -968,9 +1054,15 @@ static int build_pred_rows(qtts_ctx *c)
     return QTTS_OK;
 }
 
+static hipError_t push_state(qtts_ctx *c)
+{
+    static_assert(sizeof(DevState) % 4 == 0, "copied in words");
+    return enqueue_move(MoveList{{{c->h_st, c->st_gen, sizeof(DevState) / 4}}}, 1, c->stream);
+}
+
 static int write_state(qtts_ctx *c)
 {
-    HIPCHK(c, hipMemcpyAsync(c->st_gen, c->h_st, sizeof(DevState), hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, push_state(c));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return QTTS_OK;
 }
@@ -1005,12 +1097,7 @@ static void page_drop(qtts_ctx *c, int32_t page)
 // Copy one physical page (all layers, K and V) to another.
 static int page_copy(qtts_ctx *c, int32_t src, int32_t dst)
 {
-    const size_t blk = (size_t)2 * 8 * KV_PAGE * HEAD_DIM;
-    for (int l = 0; l < c->tm.n_layers; l++) {
-        float *b = c->tm.kv.base + (size_t)l * c->tm.kv.n_phys * blk;
-        HIPCHK(c, hipMemcpyAsync(b + (size_t)dst * blk, b + (size_t)src * blk, blk * sizeof(float),
-                                 hipMemcpyDeviceToDevice, c->stream));
-    }
+    HIPCHK(c, enqueue_page_copy(c->tm.kv, c->tm.n_layers, src, dst, c->stream));
     return QTTS_OK;
 }
 
@@ -1093,16 +1180,21 @@ extern "C" int qtts_model_dims(qtts_ctx *c, int32_t *th, int32_t *tv, int32_t *t
 // attention, gate|up + down) leaves sync_err set in the device state:
 // reported once, then cleared.  The launches after it skipped their waits,
 // so the outputs of the call are invalid.
-static int check_sync(qtts_ctx *c)
+static int sync_result(qtts_ctx *c, int32_t e)
 {
-    int32_t e = 0;
-    HIPCHK(c, hipMemcpyAsync(&e, &c->st_gen->sync_err, sizeof e, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
     if (!e) return QTTS_OK;
     const int32_t z = 0;
     HIPCHK(c, hipMemcpy(&c->st_gen->sync_err, &z, sizeof z, hipMemcpyHostToDevice));
     c->h_st->sync_err = 0;
     return fail(c, QTTS_ERR_HIP, "a cross-workgroup wait timed out (fused launch): outputs of this call are invalid");
+}
+
+static int check_sync(qtts_ctx *c)
+{
+    int32_t e = 0;
+    HIPCHK(c, hipMemcpyAsync(&e, &c->st_gen->sync_err, sizeof e, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    return sync_result(c, e);
 }
 
 // qtts_debug_force_sync_err armed: the state `st` of the call about to
@@ -1129,13 +1221,13 @@ static int step_pages(const qtts_ctx *c, int64_t kv) { return talker_fused_attn(
 static int talker_step_staged(qtts_ctx *c, int64_t position, float *hidden_out, float *logits_out, int flags)
 {
     c->h_st->position = position;
-    HIPCHK(c, hipMemcpyAsync(&c->st_gen->position, &c->h_st->position, sizeof(int64_t), hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, enqueue_move(MoveList{{{&c->h_st->position, &c->st_gen->position, 2}}}, 1, c->stream));
     RCHK(arm_sync_err(c, c->st_gen));
     HIPCHK(c, enqueue_talker_step(c->tm, c->ws, c->st_gen, 0, step_pages(c, c->h_st->kv_len), c->stream));
     RCHK(stage_out(c, c->ws.hidden, c->tm.hidden, hidden_out, flags));
     RCHK(stage_out(c, c->ws.logits, c->tm.vocab, logits_out, flags));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    const int rs = check_sync(c);
+    RCHK(finish(c, true));
+    const int rs = sync_result(c, *c->h_err);
     if (rs != QTTS_OK) {
         const std::string msg = c->err;
         RCHK(write_state(c));
@@ -1228,9 +1320,8 @@ extern "C" int qtts_talker_prefill(qtts_ctx *c, const float *X, int64_t seq, int
     RCHK(stage_out(c, c->ws.hid_work, H, hidden_out, flags));
     c->h_st->kv_len = (int32_t)(start_pos + seq);
     c->h_st->position = start_pos + seq;
-    HIPCHK(c, hipMemcpyAsync(c->st_gen, c->h_st, sizeof(DevState), hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return QTTS_OK;
+    HIPCHK(c, push_state(c));
+    return finish(c);
 }
 
 extern "C" int qtts_codec_head(qtts_ctx *c, const float *hidden, float *logits, int flags)
@@ -1240,8 +1331,7 @@ extern "C" int qtts_codec_head(qtts_ctx *c, const float *hidden, float *logits, 
     RCHK(stage_in(c, hidden, c->tm.hidden, c->d_io, flags));
     HIPCHK(c, enqueue_codec_head(c->tm, c->ws, c->d_io, c->d_io2, c->stream));
     RCHK(stage_out(c, c->d_io2, c->tm.vocab, logits, flags));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return QTTS_OK;
+    return finish(c);
 }
 
 extern "C" int qtts_embed_text_token(qtts_ctx *c, uint32_t token, float *out, int flags)
@@ -1250,8 +1340,7 @@ extern "C" int qtts_embed_text_token(qtts_ctx *c, uint32_t token, float *out, in
     if (!out) return QTTS_ERR_INVALID;
     RCHK(text_token_row(c, token, c->d_io2));
     RCHK(stage_out(c, c->d_io2, c->tm.text_fc2.n, out, flags));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return QTTS_OK;
+    return finish(c);
 }
 
 extern "C" int qtts_embed_codec_token(qtts_ctx *c, uint32_t token, float *out, int flags)
@@ -1261,8 +1350,7 @@ extern "C" int qtts_embed_codec_token(qtts_ctx *c, uint32_t token, float *out, i
     if ((int64_t)token >= c->tm.codec_rows.rows) return fail(c, QTTS_ERR_INVALID, "codec token %u out of range", token);
     HIPCHK(c, enqueue_embed_row(c->tm.codec_rows, nullptr, token, c->d_io, c->stream));
     RCHK(stage_out(c, c->d_io, c->tm.hidden, out, flags));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return QTTS_OK;
+    return finish(c);
 }
 
 // ---------------------------------------------------------------------------
@@ -1480,11 +1568,33 @@ static int text_rows(qtts_ctx *c, const uint32_t *d_ids, int n, float *out, floa
     return QTTS_OK;
 }
 
-// Device scratch for one prompt call, freed on every exit.
+// Device scratch for one prompt call, given back on every exit: from the context's arena, last in first out, or allocated
+// where it does not fit.
 struct DevScratch {
     void *p = nullptr;
-    ~DevScratch() { if (p) hipFree(p); }
+    qtts_ctx *from = nullptr;
+    size_t top = 0;
+    ~DevScratch()
+    {
+        if (!p) return;
+        if (from) from->arena_top = top;   // what takes it next is behind this call on the stream
+        else hipFree(p);
+    }
 };
+
+static int dev_scratch(qtts_ctx *c, DevScratch *b, size_t bytes)
+{
+    if (!c->arena) HIPCHK(c, hipMalloc(&c->arena, ARENA_BYTES));
+    if (c->arena_top + bytes <= ARENA_BYTES) {
+        b->p = c->arena + c->arena_top;
+        b->from = c;
+        b->top = c->arena_top;
+        c->arena_top += (bytes + 255) & ~(size_t)255;
+        return QTTS_OK;
+    }
+    HIPCHK(c, hipMalloc(&b->p, bytes));
+    return QTTS_OK;
+}
 
 extern "C" int qtts_embed_text_tokens(qtts_ctx *c, const uint32_t *ids, int64_t n, float *out, int flags)
 {
@@ -1496,14 +1606,13 @@ extern "C" int qtts_embed_text_tokens(qtts_ctx *c, const uint32_t *ids, int64_t 
         if ((int64_t)ids[i] >= m.text_rows.rows) return fail(c, QTTS_ERR_INVALID, "text token %u out of range", ids[i]);
     const size_t n_out = (size_t)n * m.hidden;
     DevScratch buf;
-    HIPCHK(c, hipMalloc(&buf.p, n * sizeof(uint32_t) + ((size_t)n * (m.text_hidden + m.text_fc1.n) + n_out) * sizeof(float)));
+    RCHK(dev_scratch(c, &buf, n * sizeof(uint32_t) + ((size_t)n * (m.text_hidden + m.text_fc1.n) + n_out) * sizeof(float)));
     float *rows = (float *)buf.p, *scratch = rows + n_out;
     uint32_t *d_ids = (uint32_t *)(scratch + (size_t)n * (m.text_hidden + m.text_fc1.n));
-    HIPCHK(c, hipMemcpyAsync(d_ids, ids, n * sizeof(uint32_t), hipMemcpyHostToDevice, c->stream));
+    RCHK(stage_ids(c, ids, n, d_ids));
     RCHK(text_rows(c, d_ids, (int)n, rows, scratch));
     RCHK(stage_out(c, rows, (int64_t)n_out, out, flags));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return QTTS_OK;
+    return finish(c);
 }
 
 extern "C" int qtts_build_icl_block(qtts_ctx *c, const uint32_t *ref_tokens, int64_t n_ref,
@@ -1537,14 +1646,14 @@ extern "C" int qtts_build_icl_block(qtts_ctx *c, const uint32_t *ref_tokens, int
     DevScratch buf;
     const size_t f_text = (size_t)nt * H, f_codec = (size_t)(n_frames + 1) * H, f_icl = (size_t)icl_len * H;
     const size_t f_scr = (size_t)nt * (m.text_hidden + m.text_fc1.n);
-    HIPCHK(c, hipMalloc(&buf.p, (f_text + f_codec + f_icl + f_scr) * sizeof(float) +
+    RCHK(dev_scratch(c, &buf, (f_text + f_codec + f_icl + f_scr) * sizeof(float) +
                                     (nt + 16 * n_frames + 1) * sizeof(uint32_t)));
     float *text = (float *)buf.p, *codec = text + f_text, *icl = codec + f_codec, *scr = icl + f_icl;
     uint32_t *d_ids = (uint32_t *)(scr + f_scr), *d_codes = d_ids + nt;
     const uint32_t bos = CODEC_BOS_ID;
-    HIPCHK(c, hipMemcpyAsync(d_ids, ids.data(), nt * sizeof(uint32_t), hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(d_codes, ref_codes, 16 * n_frames * sizeof(uint32_t), hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(d_codes + 16 * n_frames, &bos, sizeof(uint32_t), hipMemcpyHostToDevice, c->stream));
+    RCHK(stage_ids(c, ids.data(), nt, d_ids));
+    RCHK(stage_ids(c, ref_codes, 16 * n_frames, d_codes));
+    RCHK(stage_ids(c, &bos, 1, d_codes + 16 * n_frames));
     // text side: rows 0..text_len-1 (tts_eos last), row text_len = tts_pad
     RCHK(text_rows(c, d_ids, nt, text, scr));
     // codec side: codec_bos, then the per-frame sums (generate_new.rs:161-172)
@@ -1559,8 +1668,7 @@ extern "C" int qtts_build_icl_block(qtts_ctx *c, const uint32_t *ref_tokens, int
                                    (int)(icl_len - paired), (int)H, c->stream));
     RCHK(stage_out(c, icl, (int64_t)f_icl, icl_out, flags));
     if (rem_len) RCHK(stage_out(c, text + (size_t)icl_len * H, rem_len * (int64_t)H, remainder_out, flags));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return QTTS_OK;
+    return finish(c);
 }
 
 // Floats of device scratch text_rows needs for n text ids.
@@ -1592,11 +1700,11 @@ static int head_rows(qtts_ctx *c, uint32_t speaker_id, uint32_t language_id, con
     for (uint32_t t : cids)
         if ((int64_t)t >= m.codec_rows.rows) return fail(c, QTTS_ERR_INVALID, "codec token %u out of range", t);
     DevScratch buf;
-    HIPCHK(c, hipMalloc(&buf.p, (11 * H + text_scratch_floats(m, 5)) * sizeof(float) + 11 * sizeof(uint32_t)));
+    RCHK(dev_scratch(c, &buf, (11 * H + text_scratch_floats(m, 5)) * sizeof(float) + 11 * sizeof(uint32_t)));
     float *T = (float *)buf.p, *C = T + 5 * H, *scr = C + 6 * H;
     uint32_t *d_ids = (uint32_t *)(scr + text_scratch_floats(m, 5));
-    HIPCHK(c, hipMemcpyAsync(d_ids, tids, sizeof tids, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(d_ids + 5, cids, sizeof cids, hipMemcpyHostToDevice, c->stream));
+    RCHK(stage_ids(c, tids, 5, d_ids));
+    RCHK(stage_ids(c, cids, 6, d_ids + 5));
     RCHK(text_rows(c, d_ids, 5, T, scr));
     HIPCHK(c, enqueue_gather_rows(m.codec_rows, d_ids + 5, 6, C, (int)H, c->stream));
     const int64_t vm = voice ? std::min<int64_t>(voice_len, (int64_t)H) : 0;
@@ -1607,7 +1715,6 @@ static int head_rows(qtts_ctx *c, uint32_t speaker_id, uint32_t language_id, con
     HIPCHK(c, enqueue_add_rows(T + 3 * H, 0, C, (int)H, out + 3 * H, (int)H, 5, (int)H, c->stream));
     HIPCHK(c, enqueue_add_rows(T + 4 * H, 0, C + 5 * H, (int)H, out + 8 * H, (int)H, 1, (int)H, c->stream));
     if (voice) HIPCHK(c, enqueue_zero_cols(out + 7 * H, 1, (int)H, (int)vm, (int)H, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
     return QTTS_OK;
 }
 
@@ -1618,13 +1725,12 @@ extern "C" int qtts_build_prefill_head(qtts_ctx *c, uint32_t speaker_id, uint32_
     if (!out || voice_len < 0) return QTTS_ERR_INVALID;
     const size_t H = c->tm.hidden;
     DevScratch buf;
-    HIPCHK(c, hipMalloc(&buf.p, (9 * H + (voice ? (size_t)voice_len : 0) + 1) * sizeof(float)));
+    RCHK(dev_scratch(c, &buf, (9 * H + (voice ? (size_t)voice_len : 0) + 1) * sizeof(float)));
     float *rows = (float *)buf.p, *v = rows + 9 * H;
     if (voice && voice_len) RCHK(stage_in(c, voice, voice_len, v, flags));
     RCHK(head_rows(c, speaker_id, language_id, voice ? v : nullptr, voice_len, rows));
     RCHK(stage_out(c, rows, (int64_t)(9 * H), out, flags));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return QTTS_OK;
+    return finish(c);
 }
 
 extern "C" int qtts_build_icl_prefix(qtts_ctx *c, const uint32_t *ref_tokens, int64_t n_ref,
@@ -1646,14 +1752,14 @@ extern "C" int qtts_build_icl_prefix(qtts_ctx *c, const uint32_t *ref_tokens, in
     // CODEC_PAD for a ref token past the last frame
     const int64_t nf = std::min<int64_t>(n_ref - 1, n_frames), npad = n_ref - 1 - nf;
     DevScratch buf;
-    HIPCHK(c, hipMalloc(&buf.p, (3 * (size_t)n_ref * H + text_scratch_floats(m, n_ref)) * sizeof(float) +
+    RCHK(dev_scratch(c, &buf, (3 * (size_t)n_ref * H + text_scratch_floats(m, n_ref)) * sizeof(float) +
                                     (n_ref + 16 * n_frames + 2) * sizeof(uint32_t)));
     float *text = (float *)buf.p, *codec = text + n_ref * H, *rows = codec + n_ref * H, *scr = rows + n_ref * H;
     uint32_t *d_ids = (uint32_t *)(scr + text_scratch_floats(m, n_ref)), *d_codes = d_ids + n_ref;
     const uint32_t special[2] = {CODEC_BOS_ID, CODEC_PAD_ID};
-    HIPCHK(c, hipMemcpyAsync(d_ids, ref_tokens, n_ref * sizeof(uint32_t), hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(d_codes, ref_codes, 16 * n_frames * sizeof(uint32_t), hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(d_codes + 16 * n_frames, special, sizeof special, hipMemcpyHostToDevice, c->stream));
+    RCHK(stage_ids(c, ref_tokens, n_ref, d_ids));
+    RCHK(stage_ids(c, ref_codes, 16 * n_frames, d_codes));
+    RCHK(stage_ids(c, special, 2, d_codes + 16 * n_frames));
     RCHK(text_rows(c, d_ids, (int)n_ref, text, scr));
     HIPCHK(c, enqueue_gather_rows(m.codec_rows, d_codes + 16 * n_frames, 1, codec, (int)H, c->stream));
     if (nf > 0)
@@ -1664,8 +1770,7 @@ extern "C" int qtts_build_icl_prefix(qtts_ctx *c, const uint32_t *ref_tokens, in
                                       c->stream));
     HIPCHK(c, enqueue_add_rows(text, (int)H, codec, (int)H, rows, (int)H, (int)n_ref, (int)H, c->stream));
     RCHK(stage_out(c, rows, n_ref * (int64_t)H, out, flags));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return QTTS_OK;
+    return finish(c);
 }
 
 extern "C" int qtts_build_trailing_text(qtts_ctx *c, const uint32_t *tokens, int64_t n, float *out, int flags)
@@ -1696,7 +1801,7 @@ extern "C" int qtts_prefill_custom_voice(qtts_ctx *c, const uint32_t *text_token
     if (first && (int64_t)CODEC_BOS_ID >= m.codec_rows.rows) return fail(c, QTTS_ERR_INVALID, "no CODEC_BOS row");
     if (n > c->kv_cap) return fail(c, QTTS_ERR_CAPACITY, "prompt of %lld rows beyond the KV cache", (long long)n);
     DevScratch buf;
-    HIPCHK(c, hipMalloc(&buf.p, ((size_t)(n + 2) * H + (voice ? (size_t)voice_len : 0) + m.vocab +
+    RCHK(dev_scratch(c, &buf, ((size_t)(n + 2) * H + (voice ? (size_t)voice_len : 0) + m.vocab +
                                  text_scratch_floats(m, 1)) * sizeof(float) + 2 * sizeof(uint32_t)));
     float *X = (float *)buf.p, *row = X + (size_t)n * H, *v = row + 2 * H, *lg = v + (voice ? voice_len : 0);
     float *scr = lg + m.vocab;
@@ -1708,7 +1813,7 @@ extern "C" int qtts_prefill_custom_voice(qtts_ctx *c, const uint32_t *text_token
     } else if (first) {
         // CODEC_BOS + the first text token (generate_new.rs:423-431, 453-461)
         const uint32_t ids[2] = {text_tokens[0], CODEC_BOS_ID};
-        HIPCHK(c, hipMemcpyAsync(d_ids, ids, sizeof ids, hipMemcpyHostToDevice, c->stream));
+        RCHK(stage_ids(c, ids, 2, d_ids));
         RCHK(text_rows(c, d_ids, 1, row, scr));
         HIPCHK(c, enqueue_gather_rows(m.codec_rows, d_ids + 1, 1, row + H, (int)H, c->stream));
         HIPCHK(c, enqueue_add_rows(row + H, (int)H, row, (int)H, X + 9 * H, (int)H, 1, (int)H, c->stream));
@@ -1718,7 +1823,7 @@ extern "C" int qtts_prefill_custom_voice(qtts_ctx *c, const uint32_t *text_token
     HIPCHK(c, enqueue_codec_head(m, c->ws, row, lg, c->stream));
     RCHK(stage_out(c, row, (int64_t)H, hidden_out, flags));
     RCHK(stage_out(c, lg, m.vocab, logits_out, flags));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    RCHK(finish(c));
     *position_out = icl_rows ? 9 + n_icl : (n_text > 0 ? 10 : 9);
     return QTTS_OK;
 }
@@ -2106,30 +2211,33 @@ extern "C" int qtts_decode_to_audio(qtts_ctx *c, const uint32_t *codes, int64_t 
         if (n_warmup) memcpy(&all[(size_t)g * T], warmup + (size_t)g * n_warmup, n_warmup * sizeof(uint32_t));
         memcpy(&all[(size_t)g * T + n_warmup], codes + (size_t)g * n_frames, n_frames * sizeof(uint32_t));
     }
-    HIPCHK(c, hipMemcpyAsync(c->dws.codes, all.data(), all.size() * sizeof(uint32_t), hipMemcpyHostToDevice,
-                             c->stream));
-    float *out = audio;
-    if (!(flags & QTTS_DEVICE_PTRS)) {   // stage the samples in the context's I/O buffer
+    RCHK(stage_ids(c, all.data(), (int64_t)all.size(), c->dws.codes));
+    float *dev = audio, *out = audio;
+    if (!(flags & QTTS_DEVICE_PTRS)) {   // the samples go through the context's buffers
         RCHK(ensure_io(c, n));
-        out = c->d_io;
+        dev = c->d_io;
+        out = out_buffer(c, n, audio, dev, flags);
     }
     // on the split-f16 convolutions unless a weight matrix is outside their
     // range; inputs outside it (flagged by the convolutions) repeat the
     // decode on the f32 matrix path
     c->dws.f32 = d.weights_f32;
     HIPCHK(c, enqueue_decode(d, c->dws, c->dws.codes, (int)T, cut, out, c->stream));
-    int32_t range = 0;
-    HIPCHK(c, hipMemcpyAsync(&range, c->dws.range_flag, sizeof range, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, enqueue_move(MoveList{{{c->dws.range_flag, c->h_err, 1}}}, 1, c->stream));
+    // the samples come along with the flag; a decode that has to be repeated
+    // sends them again
+    if (out == dev && !(flags & QTTS_DEVICE_PTRS))
+        HIPCHK(c, hipMemcpyAsync(audio, out, (size_t)n * sizeof(float), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    if (range && !c->dws.f32) {
+    if (*c->h_err && !c->dws.f32) {
         c->dws.f32 = true;
         const hipError_t e = enqueue_decode(d, c->dws, c->dws.codes, (int)T, cut, out, c->stream);
         c->dws.f32 = false;
         HIPCHK(c, e);
+        if (out == dev && !(flags & QTTS_DEVICE_PTRS))
+            HIPCHK(c, hipMemcpyAsync(audio, out, (size_t)n * sizeof(float), hipMemcpyDeviceToHost, c->stream));
     }
-    if (!(flags & QTTS_DEVICE_PTRS))
-        HIPCHK(c, hipMemcpyAsync(audio, out, (size_t)n * sizeof(float), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    RCHK(finish(c));
     *n_samples = n;
     return QTTS_OK;
 }
@@ -2169,8 +2277,7 @@ extern "C" int qtts_acoustic_embed_sum(qtts_ctx *c, const uint32_t *codes, float
     HIPCHK(c, hipMemcpyAsync(c->d_codes_api, codes, sizeof(uint32_t) * c->pm.n_groups, hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, enqueue_embed_sum(c->pm.emb_rows, c->pm.n_groups, c->d_codes_api, c->d_io, c->stream));
     RCHK(stage_out(c, c->d_io, c->pm.emb_rows.n, out, flags));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return QTTS_OK;
+    return finish(c);
 }
 
 extern "C" int qtts_sample_token(qtts_ctx *c, const float *logits, int64_t n, const qtts_sample_params *p,
@@ -2291,8 +2398,8 @@ extern "C" int qtts_predict_codes(qtts_ctx *c, const float *talker_hidden, float
         HIPCHK(c, enqueue_codec_head(v, c->ws, side, out + (size_t)g * p.vocab, c->stream));
     }
     RCHK(stage_out(c, out, (int64_t)p.n_groups * p.vocab, logits, flags));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    RCHK(check_sync(c));   // a wait that ran out: the cache keeps its length
+    RCHK(finish(c, true));
+    RCHK(sync_result(c, *c->h_err));   // a wait that ran out: the cache keeps its length
     c->lkv_len = pos + 1;
     return QTTS_OK;
 }
@@ -2321,7 +2428,7 @@ extern "C" int qtts_prefill_tokens(qtts_ctx *c, const uint32_t *ids, const uint8
     const int64_t nt = (int64_t)tid.size(), nc = (int64_t)cid.size();
     DevScratch buf;
     const size_t rows_f = (size_t)(n + nt + nc + 1) * H, scr_f = (size_t)nt * (m.text_hidden + m.text_fc1.n);
-    HIPCHK(c, hipMalloc(&buf.p, (rows_f + scr_f) * sizeof(float) + (size_t)n * sizeof(uint32_t)));
+    RCHK(dev_scratch(c, &buf, (rows_f + scr_f) * sizeof(float) + (size_t)n * sizeof(uint32_t)));
     float *X = (float *)buf.p, *trows = X + (size_t)n * H, *crows = trows + (size_t)nt * H;
     float *hid = crows + (size_t)nc * H, *scratch = hid + H;
     uint32_t *d_tid = (uint32_t *)(scratch + scr_f), *d_cid = d_tid + nt;
@@ -2342,8 +2449,7 @@ extern "C" int qtts_prefill_tokens(qtts_ctx *c, const uint32_t *ids, const uint8
     RCHK(qtts_kv_reset(c));
     RCHK(qtts_talker_prefill(c, X, n, 0, hid, flags | QTTS_DEVICE_PTRS));
     RCHK(stage_out(c, hid, H, hidden_out, flags));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return QTTS_OK;
+    return finish(c);
 }
 
 // ---------------------------------------------------------------------------
@@ -2378,8 +2484,8 @@ extern "C" int qtts_gen_begin(qtts_ctx *c, const float *logits, const float *hid
 {
     NEED_MODEL(c);
     if (!logits || !hidden || !p || position < 0) return QTTS_ERR_INVALID;
-    HIPCHK(c, hipMemcpyAsync(c->ws.logits, logits, sizeof(float) * c->tm.vocab, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(c->ws.hidden, hidden, sizeof(float) * c->tm.hidden, hipMemcpyHostToDevice, c->stream));
+    RCHK(stage_in(c, logits, c->tm.vocab, c->ws.logits, 0));
+    RCHK(stage_in(c, hidden, c->tm.hidden, c->ws.hidden, 0));
     DevState &s = *c->h_st;
     const int32_t kv = s.kv_len;
     const int32_t n_text = s.n_text;
@@ -2396,7 +2502,8 @@ extern "C" int qtts_gen_begin(qtts_ctx *c, const float *logits, const float *hid
     s.eos_enabled = p->eos_enabled;
     s.onset_frames = p->onset_frames;
     s.onset_temperature = p->onset_temperature;
-    RCHK(write_state(c));
+    HIPCHK(c, push_state(c));
+    RCHK(finish(c));
     c->gen_started = true;
     return QTTS_OK;
 }
@@ -2549,8 +2656,9 @@ extern "C" int qtts_gen_state(qtts_ctx *c, float *logits, float *hidden, int64_t
 {
     NEED_MODEL(c);
     RCHK(read_state(c));
-    if (logits) HIPCHK(c, hipMemcpy(logits, c->ws.logits, sizeof(float) * c->tm.vocab, hipMemcpyDeviceToHost));
-    if (hidden) HIPCHK(c, hipMemcpy(hidden, c->ws.hidden, sizeof(float) * c->tm.hidden, hipMemcpyDeviceToHost));
+    RCHK(stage_out(c, c->ws.logits, c->tm.vocab, logits, 0));
+    RCHK(stage_out(c, c->ws.hidden, c->tm.hidden, hidden, 0));
+    RCHK(finish(c));
     if (position) *position = c->h_st->position;
     if (rng) *rng = c->h_st->rng;
     return QTTS_OK;
