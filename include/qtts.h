@@ -313,7 +313,7 @@ int qtts_talker_decode_token(qtts_ctx *ctx, uint32_t token, int is_text,
  * `prefill_talker_raw_from` (talker.rs:379-482).  Requires
  * kv_len == start_pos.  Writes the last row's final-normed hidden.  From
  * 3 rows the layers run as batched matrix-core GEMMs (chunks of up to
- * 1024 rows); fewer rows go one by one through the decode kernels.  flags
+ * 2048 rows); fewer rows go one by one through the decode kernels.  flags
  * may force either path (QTTS_PATH_*). */
 int qtts_talker_prefill(qtts_ctx *ctx, const float *X, int64_t seq,
                         int64_t start_pos, float *hidden_out, int flags);

@@ -33,7 +33,7 @@
 
 namespace qtts {
 
-constexpr int MM_MAX_MB = 6;   // row blocks of 16 per tile, at most
+constexpr int MM_MAX_MB = 5;   // row blocks of 16 per tile, at most
 
 // ---------------------------------------------------------------------------
 // Fragment order.  Record (group, 64-row chunk): 1024 B of nibbles, lane l's
@@ -233,10 +233,12 @@ k_q4_gemm(RowsSplit a, Q4Frag w, MmOut o, int tm, int nrun, int run_chunks)
     const int aw = (t & 15) * 256 + (((t >> 4) ^ (t & 15)) * 16);
     const uint8_t *wp = w.data + ((size_t)min(grp, w.ng - 1) * w.kc + c0) * w.rec;
 
-    constexpr int AS = MB >= 6 || (FP == 1 && MB >= 5) ? 1 : 2;   // register sets of rows (a tall tile's chunk covers the loads by itself)
+    // register sets of rows and of weights: a tall tile's chunk covers the
+    // loads by itself; short tiles run one segment, all of it in flight at once
+    constexpr int AS = MB <= 2 ? 4 : MB >= 6 || (FP == 1 && MB >= 5) ? 1 : 2, WS = MB <= 2 ? 4 : 2;
     u32x4 ra[AS][MB];
-    u32x4 rn[2];
-    half8 rs[2][DUAL ? 4 : 2];       // [set][half of the chunk (+ 2 block)]
+    u32x4 rn[WS];
+    half8 rs[WS][DUAL ? 4 : 2];       // [set][half of the chunk (+ 2 block)]
     const auto fetch_a = [&](int s, int c) {
 #pragma unroll
         for (int i = 0; i < MB; i++) ra[s][i] = *(const u32x4 *)(ap + (size_t)c * 256 + ao[i]);
@@ -256,43 +258,60 @@ k_q4_gemm(RowsSplit a, Q4Frag w, MmOut o, int tm, int nrun, int run_chunks)
         for (int i = 0; i < MB; i++) *(u32x4 *)(lds + buf * BUF + i * 4096 + aw) = ra[s][i];
     };
     const float ubs = __builtin_ldexpf(1.0f, -w.bshift);
-    f32x4 cur[MB][2], tot[MB][2];
+    f32x4 cur[MB][2], tot[MB][2], seg[FP == 1 ? MB : 1][2];   // seg, FP 1: the segment's 64-column sums
 #pragma unroll
     for (int i = 0; i < MB; i++)
 #pragma unroll
         for (int j = 0; j < 2; j++) tot[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    const auto compute = [&](int s, int buf, bool first) {
+    // [half][block]; half 0 is dequantised a chunk ahead (tall tiles: its
+    // arithmetic then fills the last products' issue slots, not the wait for
+    // the rows after the barrier: 128 / 400 / 1024 rows x 2048 x 12288 40.4 ->
+    // 34.9, 59.1 -> 56.7, 151 -> 144 us)
+    constexpr bool AHEAD = MB > 2;
+    half8 wh[2][2], wl[2][2];
+    const auto dequant = [&](int s, int h) {
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-            half8 wh[2], wl[2];
+        for (int j = 0; j < 2; j++) dequant8(rn[s][2 * j + h], rs[s][DUAL ? 2 * j + h : h], wh[h][j], wl[h][j]);
+    };
+    const auto mma = [&](int h, const half8 (&xh)[MB], const half8 (&xl)[MB], bool first) {
+        const f32x4 z = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int j = 0; j < 2; j++) dequant8(rn[s][2 * j + h], rs[s][DUAL ? 2 * j + h : h], wh[j], wl[j]);
-            half8 xh[MB], xl[MB];
-            const int ph = 8 * h + q, pl = ph + 4;
+        for (int i = 0; i < MB; i++)
 #pragma unroll
-            for (int i = 0; i < MB; i++) {
-                xh[i] = *(const half8 *)(lds + buf * BUF + i * 4096 + ph * 256 + ((r16 ^ ph) * 16));
-                xl[i] = *(const half8 *)(lds + buf * BUF + i * 4096 + pl * 256 + ((r16 ^ pl) * 16));
-            }
-            const f32x4 z = {0.0f, 0.0f, 0.0f, 0.0f};
+            for (int j = 0; j < 2; j++)
+                cur[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wl[h][j], xh[i], first ? z : cur[i][j], 0, 0, 0);
 #pragma unroll
-            for (int i = 0; i < MB; i++)
+        for (int i = 0; i < MB; i++)
 #pragma unroll
-                for (int j = 0; j < 2; j++)
-                    cur[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wl[j], xh[i], first && h == 0 ? z : cur[i][j], 0, 0, 0);
+            for (int j = 0; j < 2; j++)
+                cur[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wh[h][j], xl[i], cur[i][j], 0, 0, 0);
 #pragma unroll
-            for (int i = 0; i < MB; i++)
+        for (int i = 0; i < MB; i++)
 #pragma unroll
-                for (int j = 0; j < 2; j++)
-                    cur[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wh[j], xl[i], cur[i][j], 0, 0, 0);
+            for (int j = 0; j < 2; j++)
+                cur[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wh[h][j], xh[i], cur[i][j], 0, 0, 0);
+    };
+    const auto read_x = [&](int buf, int h, half8 (&xh)[MB], half8 (&xl)[MB]) {
+        const int ph = 8 * h + q, pl = ph + 4;
 #pragma unroll
-            for (int i = 0; i < MB; i++)
-#pragma unroll
-                for (int j = 0; j < 2; j++)
-                    cur[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wh[j], xh[i], cur[i][j], 0, 0, 0);
+        for (int i = 0; i < MB; i++) {
+            xh[i] = *(const half8 *)(lds + buf * BUF + i * 4096 + ph * 256 + ((r16 ^ ph) * 16));
+            xl[i] = *(const half8 *)(lds + buf * BUF + i * 4096 + pl * 256 + ((r16 ^ pl) * 16));
         }
     };
-    // tot += cur times the power of two that undoes the staging (exact)
+    // chunk in buf with weights of set s; sn: the next chunk's set
+    const auto compute = [&](int s, int sn, int buf, bool first) {
+        half8 xh[2][MB], xl[2][MB];
+        read_x(buf, 0, xh[0], xl[0]);
+        if (!AHEAD) dequant(s, 0);
+        dequant(s, 1);
+        mma(0, xh[0], xl[0], first);
+        read_x(buf, 1, xh[1], xl[1]);
+        mma(1, xh[1], xl[1], false);
+        if (AHEAD) dequant(sn, 0);
+    };
+    // sums times the power of two that undoes the staging (exact), into the
+    // running ones
     const auto fold = [&](const float (&f)[MB]) {
 #pragma unroll
         for (int i = 0; i < MB; i++) {
@@ -303,12 +322,24 @@ k_q4_gemm(RowsSplit a, Q4Frag w, MmOut o, int tm, int nrun, int run_chunks)
                 for (int e = 0; e < 4; e++) tot[i][j][e] = fmaf(cur[i][j][e], u, tot[i][j][e]);
         }
     };
+    const auto fold_seg = [&](const float (&f)[MB], bool first) {
+#pragma unroll
+        for (int i = 0; i < (FP == 1 ? MB : 0); i++) {
+            const float u = f[i] * ubs;
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) seg[i][j][e] = first ? cur[i][j][e] * u : fmaf(cur[i][j][e], u, seg[i][j][e]);
+        }
+    };
 
-    fetch_a(0, 0);
-    fetch_w(0, 0);
-    if (AS == 2) fetch_a(AS - 1, min(1, n - 1));
-    fetch_w(1, min(1, n - 1));
+#pragma unroll
+    for (int u = 0; u < WS; u++) {
+        if (u < AS) fetch_a(u, min(u, n - 1));
+        fetch_w(u, min(u, n - 1));
+    }
     stage(0, 0);
+    if (AHEAD) dequant(0, 0);
     __syncthreads();
     for (int c = 0; c < n; c += 4) {
         float f4[MB];
@@ -320,22 +351,29 @@ k_q4_gemm(RowsSplit a, Q4Frag w, MmOut o, int tm, int nrun, int run_chunks)
 #pragma unroll
         for (int u = 0; u < 4; u++) {
             if (c + u < n) {
-                const int s = u & 1;
-                fetch_a(AS == 2 ? s : 0, min(c + u + AS, n - 1));
+                const int s = u % WS, buf = u & 1;
+                if (MB > 2 || c + u + AS < n) fetch_a(u % AS, min(c + u + AS, n - 1));
                 float f1[MB];            // the chunk's factors, in flight behind its matrix work
                 if constexpr (FP == 1) {
 #pragma unroll
                     for (int i = 0; i < MB; i++)
                         f1[i] = a.rsc[(size_t)(c0 + c + u) * a.rseg + min(m0 + 16 * i + r16, a.M - 1)];
                 }
-                compute(s, s, FP == 1 || u == 0);
-                if constexpr (FP == 1) fold(f1);
-                fetch_w(s, min(c + u + 2, n - 1));
-                stage(AS == 2 ? s ^ 1 : 0, s ^ 1);
+                compute(s, (u + 1) % WS, buf, FP == 1 || u == 0);
+                if constexpr (FP == 1) fold_seg(f1, u == 0);
+                if (MB > 2 || c + u + WS < n) fetch_w(s, min(c + u + WS, n - 1));
+                stage((u + 1) % AS, buf ^ 1);
                 __syncthreads();
             }
         }
-        if constexpr (FP == 4) fold(f4);
+        if constexpr (FP == 4) {
+            fold(f4);
+        } else {
+#pragma unroll
+            for (int i = 0; i < MB; i++)
+#pragma unroll
+                for (int j = 0; j < 2; j++) tot[i][j] += seg[i][j];
+        }
     }
 
     if constexpr (EPI == MM_SWIGLU) {
@@ -529,16 +567,16 @@ hipError_t enqueue_split_rows(const float *X, int ld, int M, int K, int seg, uin
 // the chip idle behind long K loops, and the partial sums are still small.
 constexpr int MM_SEG_ROWS = 64;
 
-// With factors every 64 columns (fp1) a slice is one chain of 64-column
-// sums, so the cut into slices is the same at any row count.
-static int mm_run_chunks(const Q4Frag &w, int M, bool fp1)
+static int mm_run_chunks(const Q4Frag &w, int M)
 {
-    return M <= MM_SEG_ROWS && !fp1 ? 4 : 4 * (mm_segments(w) / mm_slices(w));
+    // (down's 24 segments: 24 partial sums are more to add than they save
+    // from 17 rows on)
+    return M <= (mm_segments(w) > 8 ? 16 : MM_SEG_ROWS) ? 4 : 4 * (mm_segments(w) / mm_slices(w));
 }
 
-size_t mm_part_floats(const Q4Frag &w, int M, bool fp1)
+size_t mm_part_floats(const Q4Frag &w, int M)
 {
-    const int rc = mm_run_chunks(w, M, fp1);
+    const int rc = mm_run_chunks(w, M);
     return (size_t)((w.kc + rc - 1) / rc) * M * w.ng * 32;
 }
 
@@ -546,12 +584,12 @@ size_t mm_part_floats(const Q4Frag &w, int M, bool fp1)
 // (fp1), every 256 (rsc with rseg) or not at all.
 hipError_t enqueue_mm_parts(const RowsSplit &a, const Q4Frag &w, bool fp1, float *part, MmParts *p, hipStream_t s)
 {
-    const int rc = mm_run_chunks(w, a.M, fp1), nseg = mm_segments(w);
+    const int rc = mm_run_chunks(w, a.M), nseg = mm_segments(w);
     p->p = part;
     p->ld = w.ng * 32;
     p->stride = (size_t)a.M * p->ld;
     p->n = (w.kc + rc - 1) / rc;
-    p->per = rc == 4 && !fp1 ? nseg / mm_slices(w) : 1;
+    p->per = rc == 4 && mm_slices(w) < nseg ? nseg / mm_slices(w) : 1;
     const MmOut o{part, p->ld, 1, nullptr, 0, nullptr};
     return fp1 ? launch_mm<1, MM_PART>(a, w, o, rc, s) : launch_mm<4, MM_PART>(a, w, o, rc, s);
 }

@@ -300,7 +300,7 @@ size_t frag_shape(const Q4Tiled &w, Q4Frag *f);
 hipError_t enqueue_frag_build(const Q4Tiled &w, const Q4Frag &f, uint8_t *out, hipStream_t s);
 hipError_t enqueue_split_rows(const float *X, int ld, int M, int K, int seg, uint8_t *out, int kc, float *rsc,
                               int ldr, hipStream_t s);
-size_t mm_part_floats(const Q4Frag &w, int M, bool fp1);
+size_t mm_part_floats(const Q4Frag &w, int M);
 size_t mm_swiglu_part_floats(const Q4Frag &w, int M);
 hipError_t enqueue_mm_parts(const RowsSplit &a, const Q4Frag &w, bool fp1, float *part, MmParts *p, hipStream_t s);
 hipError_t enqueue_mm_swiglu(const RowsSplit &a, const Q4Frag &w, float *part, uint8_t *rows, int okc, float *rsc,

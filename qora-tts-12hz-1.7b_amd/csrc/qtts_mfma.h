@@ -191,6 +191,7 @@ static hipError_t by_parts(int n, const A &...args)
     case 4: return F<4>::go(args...);
     case 6: return F<6>::go(args...);
     case 8: return F<8>::go(args...);
+    case 24: return F<24>::go(args...);
     default: return F<0>::go(args...);
     }
 }

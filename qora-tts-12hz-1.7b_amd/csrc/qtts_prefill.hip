@@ -918,12 +918,11 @@ int64_t prefill_part_floats(const TalkerDev &m, int rows)
         for (const Q4Tiled *w : {&L.qkv, &L.o, &L.down}) f = std::max<int64_t>(f, (int64_t)rows * part_slices(*w) * w->G * 32);
         if (!L.qkv_f.data) continue;
         // a small batch may cut K finer than a large one
-        for (int r = rows;; r = std::min(64, rows)) {
-            f = std::max<int64_t>(f, (int64_t)mm_part_floats(L.qkv_f, r, false));
-            f = std::max<int64_t>(f, (int64_t)mm_part_floats(L.o_f, r, false));
-            f = std::max<int64_t>(f, (int64_t)mm_part_floats(L.down_f, r, true));
+        for (int r : {rows, std::min(64, rows), std::min(16, rows)}) {
+            f = std::max<int64_t>(f, (int64_t)mm_part_floats(L.qkv_f, r));
+            f = std::max<int64_t>(f, (int64_t)mm_part_floats(L.o_f, r));
+            f = std::max<int64_t>(f, (int64_t)mm_part_floats(L.down_f, r));
             f = std::max<int64_t>(f, (int64_t)mm_swiglu_part_floats(L.gate_up_f, r));
-            if (r <= 64) break;
         }
     }
     return f;

@@ -131,7 +131,8 @@ struct qtts_prefix {
 // rows 9.6 / 11 / 12 us and 7.0 / 13 / 27 us.  Both are as far from 64 bits
 // (2e-7 of a product, 1.3e-7 of the prefill's hidden).
 constexpr int64_t MFMA_MIN_ROWS = 3;
-constexpr int PREFILL_MAX_ROWS = 1024;   // rows per prefill chunk
+constexpr int PREFILL_MAX_ROWS = 2048;   // rows per prefill chunk, longer prompts in equal chunks
+constexpr int TIME_PREFILL_ROWS = 1024;  // rows qtts_time_prefill takes
 constexpr size_t PIN_BYTES = (size_t)1 << 20;    // pinned staging per context
 constexpr size_t PIN_MAX = (size_t)128 << 10;    // larger arguments are copied by the runtime
 constexpr size_t ARENA_BYTES = (size_t)64 << 20;
@@ -1301,9 +1302,11 @@ extern "C" int qtts_talker_prefill(qtts_ctx *c, const float *X, int64_t seq, int
     c->gen_started = false;
     const int H = c->tm.hidden;
     if (use_mfma(flags, seq) && prefill_supported(c->tm)) {
-        RCHK(ensure_prefill(c, (int)std::min<int64_t>(seq, PREFILL_MAX_ROWS)));
-        for (int64_t r0 = 0; r0 < seq; r0 += c->pf.cap_rows) {
-            const int rows = (int)std::min<int64_t>(c->pf.cap_rows, seq - r0);
+        // equal chunks: 1024 + 85 rows took as long as 1400 in one
+        const int64_t nch = (seq + PREFILL_MAX_ROWS - 1) / PREFILL_MAX_ROWS, per = (seq + nch - 1) / nch;
+        RCHK(ensure_prefill(c, (int)per));
+        for (int64_t r0 = 0; r0 < seq; r0 += per) {
+            const int rows = (int)std::min<int64_t>(per, seq - r0);
             RCHK(stage_in(c, X + r0 * H, (int64_t)rows * H, c->pf.x, flags));
             HIPCHK(c, enqueue_talker_prefill(c->tm, c->pf, rows, start_pos + r0, c->ws.hid_work, c->stream));
         }
@@ -2914,7 +2917,7 @@ extern "C" int qtts_time_prefill(qtts_ctx *c, int64_t rows, int32_t what, int32_
     NEED_MODEL(c);
     const TalkerDev &m = c->tm;
     if (!prefill_supported(m)) return fail(c, QTTS_ERR_UNSUPPORTED, "model shapes outside the matrix-core prefill");
-    if (rows > PREFILL_MAX_ROWS) return fail(c, QTTS_ERR_CAPACITY, "at most %d rows per prefill chunk", PREFILL_MAX_ROWS);
+    if (rows > TIME_PREFILL_ROWS) return fail(c, QTTS_ERR_CAPACITY, "at most %d rows per prefill timing", TIME_PREFILL_ROWS);
     if (rows > c->kv_cap || rows > m.rope_rows) return fail(c, QTTS_ERR_CAPACITY, "rows beyond the KV cache");
     hipSetDevice(c->device);
     RCHK(ensure_prefill(c, (int)rows));
