@@ -92,7 +92,7 @@ __global__ void k_snake_par(const float *alpha, const float *beta, int n, float 
 // refilled for the next tap as soon as its products are issued.
 // ---------------------------------------------------------------------------
 
-enum { DC_SNAKE = 0, DC_X_SNAKE = 1 };
+enum { DC_SNAKE = 0, DC_X_SNAKE = 1, DC_RAW = 2 };   // RAW: the sums of the slices, for a consumer below
 
 struct DcIn {
     const uint8_t *x;        // split rows
@@ -301,7 +301,7 @@ k_dconv(DcIn in, const uint8_t *wts, DcOut o, DcGeo g, DcFuse fz)
     }
 
     const int nw = n0 + 16 * PE * wv + r16;          // position of p = 0
-    if (g.ks > 1) {
+    if (EPI == DC_RAW || g.ks > 1) {
         float *pp = g.part + (size_t)slice * in.L * g.nph * o.M;
 #pragma unroll
         for (int p = 0; p < PE; p++) {
@@ -320,7 +320,8 @@ k_dconv(DcIn in, const uint8_t *wts, DcOut o, DcGeo g, DcFuse fz)
         __syncthreads();
         if (t == 0 && dc_out_of_range(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])))) *o.flag = 1;
     };
-    if constexpr (!FUSE) {
+    if constexpr (EPI == DC_RAW) {
+    } else if constexpr (!FUSE) {
         float mx = 0.0f;
 #pragma unroll
         for (int b = 0; b < CB; b += 2) {
@@ -483,6 +484,156 @@ k_dconv_reduce(const float *part, int ks, int64_t rows, int nph, DcOut o)
     if (threadIdx.x == 0 && dc_out_of_range(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])))) *o.flag = 1;
 }
 
+// ---------------------------------------------------------------------------
+// The transformer between VQ and upsampling (decoder.rs:198-340) on the same
+// rows: its matrices are 1x1 convolutions whose slices' sums the kernels below
+// add, each with what follows in the reference.  A few positions and 512 to
+// 3072 channels: the launches are bound by the latency of a record's loads,
+// so a launch takes many slices of one record a wave, and the kernels that
+// add the slices issue all their loads before the first addition.  The 8
+// layers of 512 channels, whole decode, channel-first before and this: 1
+// frame 1.20 -> 1.01 ms, 21 frames 1.67 -> 1.48 ms, 160 frames 4.24 -> 4.10.
+// ---------------------------------------------------------------------------
+
+struct LinSum {
+    const float *part;       // [ks][rows][M]
+    const float *un, *bias;  // [M]; bias may be null
+    int ks, rows, M;
+};
+
+// four consecutive channels of a row (KS > 0: that many slices, every load
+// issued before the first addition)
+template <int KS>
+__device__ __forceinline__ f32x4 lin_sum(const LinSum &p, int row, int ch)
+{
+    const float *a = p.part + (size_t)row * p.M + ch;
+    const size_t st = (size_t)p.rows * p.M;
+    f32x4 v;
+    if constexpr (KS > 0) {
+        f32x4 x[KS];
+#pragma unroll
+        for (int s = 0; s < KS; s++) x[s] = ld4(a + s * st);
+        v = x[0];
+#pragma unroll
+        for (int s = 1; s < KS; s++) v += x[s];
+    } else {
+        v = ld4(a);
+        for (int s = 1; s < p.ks; s++) v += ld4(a + s * st);
+    }
+    v *= ld4(p.un + ch);
+    return p.bias ? v + ld4(p.bias + ch) : v;
+}
+
+// slot store of eight channels (record rec, lane group q) of a split row
+__device__ __forceinline__ void split_store8(uint8_t *ys, int row, int C, int rec, int q, const f32x4 &a, const f32x4 &b)
+{
+    DcOut o{};
+    o.ys = ys;
+    o.M = C;
+    dc_store8(o, row, rec, q, a, b);
+}
+
+// plain f32 rows
+template <int KS>
+__global__ void __launch_bounds__(256)
+k_lin_rows(LinSum p, float *y)
+{
+    const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x, n4 = p.M / 4;
+    if (id >= p.rows * n4) return;
+    const int row = (int)(id / n4), ch = 4 * (int)(id - row * n4);
+    *(f32x4 *)(y + (size_t)row * p.M + ch) = lin_sum<KS>(p, row, ch);
+}
+
+// channel-first [M][rows]: 64 rows x 32 channels through LDS
+template <int KS>
+__global__ void __launch_bounds__(256)
+k_lin_cf(LinSum p, float *y)
+{
+    __shared__ float tile[64][33];
+    const int t = threadIdx.x, r0 = blockIdx.x * 64, c0 = blockIdx.y * 32;
+    for (int i = t; i < 64 * 8; i += 256) {
+        const int r = i >> 3, c = 4 * (i & 7);
+        if (r0 + r < p.rows) {
+            const f32x4 v = lin_sum<KS>(p, r0 + r, c0 + c);
+            for (int e = 0; e < 4; e++) tile[r][c + e] = v[e];
+        }
+    }
+    __syncthreads();
+    for (int i = t; i < 64 * 32; i += 256) {
+        const int r = i & 63, c = i >> 6;
+        if (r0 + r < p.rows) y[(size_t)(c0 + c) * p.rows + r0 + r] = tile[r][c];
+    }
+}
+
+// silu(gate) up of interleaved rows (gate 2j, up 2j + 1) into split rows
+template <int KS>
+__global__ void __launch_bounds__(256)
+k_lin_swiglu(LinSum p, uint8_t *ys, int32_t *flag)
+{
+    __shared__ float red[4];
+    const int C = p.M / 2, n8 = C / 8;
+    const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    float mx = 0.0f;
+    if (id < (int64_t)p.rows * n8) {
+        const int row = (int)(id / n8), j8 = (int)(id - (int64_t)row * n8), rec = j8 >> 2, q = j8 & 3;
+        f32x4 y[2];
+        for (int j = 0; j < 2; j++) {
+            const int c = 2 * (32 * rec + 4 * q + 16 * j);
+            const f32x4 a = lin_sum<KS>(p, row, c), b = lin_sum<KS>(p, row, c + 4);
+            y[j] = f32x4{silu_f(a.x) * a.y, silu_f(a.z) * a.w, silu_f(b.x) * b.y, silu_f(b.z) * b.w};
+            mx = max4(mx, y[j]);
+        }
+        split_store8(ys, row, C, rec, q, y[0], y[1]);
+    }
+    mx = wave_max_dpp(mx);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
+    __syncthreads();
+    if (threadIdx.x == 0 && dc_out_of_range(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])))) *flag = 1;
+}
+
+// x (+)= scale * sum, then RMSNorm (eps 1e-5) into split rows; one wave a
+// row of at most 512 NV channels, in registers.  scale null: x = sum.
+template <int NV, int KS>
+__global__ void __launch_bounds__(256)
+k_lin_resid_rms(LinSum p, const float *scale, float *x, const float *gamma, uint8_t *ys, int32_t *flag)
+{
+    __shared__ float red[4];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, row = blockIdx.x * 4 + wv, H = p.M;
+    float mx = 0.0f;
+    if (row < p.rows) {
+        f32x4 v[NV][2];
+        float ss = 0.0f;
+#pragma unroll
+        for (int i = 0; i < NV; i++)
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const int j8 = lane + 64 * i, ch = 32 * (j8 >> 2) + 4 * (j8 & 3) + 16 * j;
+                v[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                if (8 * j8 >= H) continue;
+                f32x4 a = lin_sum<KS>(p, row, ch);
+                float *xr = x + (size_t)row * H + ch;
+                if (scale) a = ld4(xr) + ld4(scale + ch) * a;
+                *(f32x4 *)xr = a;
+                v[i][j] = a;
+                ss = fmaf(a.x, a.x, fmaf(a.y, a.y, fmaf(a.z, a.z, fmaf(a.w, a.w, ss))));
+            }
+        const float inv = 1.0f / sqrtf(wave_sum_dpp(ss) / (float)H + 1e-5f);
+#pragma unroll
+        for (int i = 0; i < NV; i++) {
+            const int j8 = lane + 64 * i, rec = j8 >> 2, q = j8 & 3;
+            if (8 * j8 >= H) continue;
+            const f32x4 a = v[i][0] * inv * ld4(gamma + 32 * rec + 4 * q);
+            const f32x4 b = v[i][1] * inv * ld4(gamma + 32 * rec + 4 * q + 16);
+            mx = max4(max4(mx, a), b);
+            split_store8(ys, row, H, rec, q, a, b);
+        }
+    }
+    mx = wave_max_dpp(mx);
+    if (lane == 0) red[wv] = mx;
+    __syncthreads();
+    if (threadIdx.x == 0 && dc_out_of_range(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])))) *flag = 1;
+}
+
 // Channel-first f32 [C][L] -> split rows: 64 positions x 32 channels through
 // LDS; lane = position.
 __global__ void __launch_bounds__(256)
@@ -557,7 +708,7 @@ k_out_rows(const float *x, int C, int L, const float *w, float bias, int dil, in
 
 #define VCHK(x) do { hipError_t e_ = (x); if (e_ != hipSuccess) return e_; } while (0)
 
-constexpr int DC_CB = 6;     // 96-channel tiles
+constexpr int DC_CB = DC_VOCOS_CB, DC_LIN_CB = DC_TF_CB;
 constexpr int DC_FUSE_PB = 2;   // position blocks a wave of the fused residual unit
 
 bool dconv_fits(int oc, int ic, int kt, int dil)
@@ -567,11 +718,11 @@ bool dconv_fits(int oc, int ic, int kt, int dil)
 
 size_t dconv_weight_bytes(int rows, int ic, int kt) { return (size_t)rows * ic * kt * 4; }
 
-hipError_t enqueue_dconv_pack(const float *w, int rows, int ic, int kt, uint8_t *out, float *un, hipStream_t s)
+hipError_t enqueue_dconv_pack(const float *w, int rows, int ic, int kt, int cb, uint8_t *out, float *un, hipStream_t s)
 {
     hipLaunchKernelGGL(k_dconv_row_scale, dim3((rows + 3) / 4), dim3(256), 0, s, w, rows, ic * kt, un);
     const int64_t n = (int64_t)(rows / 16) * (ic / 32) * kt;
-    hipLaunchKernelGGL(k_dconv_pack, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, s, w, un, rows, ic, kt, DC_CB, out);
+    hipLaunchKernelGGL(k_dconv_pack, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, s, w, un, rows, ic, kt, cb, out);
     return hipGetLastError();
 }
 
@@ -664,6 +815,108 @@ static hipError_t dconv(const DcIn &in, const uint8_t *w, const DcOut &o, int np
         hipLaunchKernelGGL(k_dconv_reduce<EPI>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, ws.part, ks, rows, nph, o);
     }
     return hipGetLastError();
+}
+
+// A linear layer over split rows into slice sums: 64-channel tiles, slices of
+// one to a few records a wave, as many as give about two workgroups a CU.
+static hipError_t linear(const uint8_t *x, int nc, int rows, const DecLin &w, int M, const float *bias, const DecoderWs &ws,
+                         LinSum *out, hipStream_t s)
+{
+    DcGeo g{};
+    g.tm = M / (16 * DC_LIN_CB);
+    g.tn = (rows + 63) / 64;
+    g.nph = 1;
+    int ks = std::max(1, std::min({nc / 4, 16, 512 / std::max(1, g.tm * g.tn)}));
+    while (ks > 1 && (size_t)ks * rows * M > ws.part_cap) ks--;
+    g.cps = (nc + ks - 1) / ks;
+    g.ks = (nc + g.cps - 1) / g.cps;
+    g.part = ws.part;
+    if ((size_t)g.ks * rows * M > ws.part_cap) return hipErrorInvalidValue;
+    DcOut o{};
+    o.M = M;
+    o.os = 1;
+    const int lds = std::max(4 * 2 * 64 * 128, 4 * 4 * DC_LIN_CB * 1024);
+    hipLaunchKernelGGL((k_dconv<DC_LIN_CB, 4, 1, DC_RAW, false, true>), dim3((unsigned)(g.tm * g.tn * g.ks)), dim3(256), lds,
+                       s, DcIn{x, nc, rows, 1}, w.w, o, g, DcFuse{});
+    *out = LinSum{ws.part, w.un, bias, g.ks, rows, M};
+    return hipGetLastError();
+}
+
+// the instance of a consumer of slice sums for p.ks slices
+#define LIN_BY_KS(KERNEL, GRID, ...)                                                             \
+    do {                                                                                         \
+        switch (p.ks) {                                                                          \
+        case 1: hipLaunchKernelGGL((KERNEL(1)), GRID, dim3(256), 0, s, __VA_ARGS__); break;      \
+        case 2: hipLaunchKernelGGL((KERNEL(2)), GRID, dim3(256), 0, s, __VA_ARGS__); break;      \
+        case 4: hipLaunchKernelGGL((KERNEL(4)), GRID, dim3(256), 0, s, __VA_ARGS__); break;      \
+        case 8: hipLaunchKernelGGL((KERNEL(8)), GRID, dim3(256), 0, s, __VA_ARGS__); break;      \
+        default: hipLaunchKernelGGL((KERNEL(0)), GRID, dim3(256), 0, s, __VA_ARGS__); break;     \
+        }                                                                                        \
+        VCHK(hipGetLastError());                                                                 \
+    } while (0)
+#define K_ROWS(KS) k_lin_rows<KS>
+#define K_CF(KS) k_lin_cf<KS>
+#define K_SWIGLU(KS) k_lin_swiglu<KS>
+#define K_RMS1(KS) k_lin_resid_rms<1, KS>
+#define K_RMS4(KS) k_lin_resid_rms<4, KS>
+
+static hipError_t resid_rms(const LinSum &p, const float *scale, float *x, const float *gamma, uint8_t *ys, int32_t *flag,
+                            hipStream_t s)
+{
+    const dim3 grid((p.rows + 3) / 4);
+    if (p.M <= 512) LIN_BY_KS(K_RMS1, grid, p, scale, x, gamma, ys, flag);
+    else LIN_BY_KS(K_RMS4, grid, p, scale, x, gamma, ys, flag);
+    return hipSuccess;
+}
+
+// The transformer over T positions: in [latent][T] channel-first f32 to out
+// likewise.  bufs: four buffers of the workspace other than those two.
+hipError_t enqueue_dec_tf(const DecoderDev &d, const DecoderWs &ws, const float *in, float *out, float *const bufs[4], int T,
+                          hipStream_t s)
+{
+    const int H = d.hidden, A = d.n_heads * d.head_dim, I = d.inter, LAT = d.latent;
+    uint8_t *xs = (uint8_t *)bufs[0], *hs = (uint8_t *)bufs[1];
+    float *x = bufs[2], *qkv = bufs[3];
+    LinSum p{};
+    hipLaunchKernelGGL(k_cf_split, dim3((T + 63) / 64, LAT / 32), dim3(256), 0, s, in, LAT, T, hs, ws.range_flag);
+    VCHK(hipGetLastError());
+    VCHK(linear(hs, LAT / 32, T, d.tf_in, H, d.tf_in_b, ws, &p, s));
+    VCHK(resid_rms(p, nullptr, x, d.tf[0].in_norm, xs, ws.range_flag, s));
+    for (int l = 0; l < d.n_tf; l++) {
+        const DecLayer &L = d.tf[l];
+        VCHK(linear(xs, H / 32, T, L.pqkv, 3 * A, nullptr, ws, &p, s));
+        LIN_BY_KS(K_ROWS, dim3((unsigned)(((int64_t)T * 3 * A / 4 + 255) / 256)), p, qkv);
+        VCHK(enqueue_dec_attn_rows(d, qkv, T, hs, ws.range_flag, s));
+        VCHK(linear(hs, A / 32, T, L.po, H, nullptr, ws, &p, s));
+        VCHK(resid_rms(p, L.attn_scale, x, L.post_norm, xs, ws.range_flag, s));
+        VCHK(linear(xs, H / 32, T, L.pgu, 2 * I, nullptr, ws, &p, s));
+        LIN_BY_KS(K_SWIGLU, dim3((unsigned)(((int64_t)T * I / 8 + 255) / 256)), p, hs, ws.range_flag);
+        VCHK(linear(hs, I / 32, T, L.pdown, H, nullptr, ws, &p, s));
+        VCHK(resid_rms(p, L.mlp_scale, x, l + 1 < d.n_tf ? d.tf[l + 1].in_norm : d.tf_norm, xs, ws.range_flag, s));
+    }
+    VCHK(linear(xs, H / 32, T, d.tf_out, LAT, d.tf_out_b, ws, &p, s));
+    LIN_BY_KS(K_CF, dim3((T + 63) / 64, LAT / 32), p, out);
+    return hipSuccess;
+}
+
+// Whether enqueue_dec_tf runs a decoder's shapes (its slice sums within
+// part_floats are checked per call).  It was the faster one at every length
+// timed (1 to 400 frames: 11% to 1% of the decode), so no length limits it;
+// the shapes are what its tiles need: whole 64-channel tiles, whole records,
+// heads of the tiled attention's 64, and a row of at most 2048 in a wave's
+// registers.
+bool dec_tf_fits(const DecoderDev &d)
+{
+    const int A = d.n_heads * d.head_dim;
+    return !d.weights_f32 && d.n_tf > 0 && d.hidden <= 2048 && d.hidden % 64 == 0 && A % 64 == 0 && d.inter % 32 == 0 &&
+           d.latent % 64 == 0 && d.head_dim == 64 && dec_attn_tiled(d);
+}
+
+// The most positions whose slice sums fit part_floats.
+int dec_tf_rows(const DecoderDev &d, size_t part_floats)
+{
+    const int widest = std::max({3 * d.n_heads * d.head_dim, 2 * d.inter, d.latent, d.hidden});
+    return (int)std::min<size_t>(part_floats / widest, 1 << 20);
 }
 
 // The Vocos stages and the output conv from the upsamplers' signal sig

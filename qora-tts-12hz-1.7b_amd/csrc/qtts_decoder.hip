@@ -808,10 +808,12 @@ static inline size_t attn_tile_lds(int hd, int W)
     return (size_t)(2 * nk * kp + ATT_QB * kp + ATT_QB * (nk + 1)) * sizeof(float);
 }
 
-template <int HD>
+// ROWS: q|k|v as f32 rows [T][3A] (whole rows of a head coalesced), the output
+// as split rows (qtts_dconv.hip) with their range check; else channel-first.
+template <int HD, bool ROWS>
 __global__ void __launch_bounds__(256)
 k_dec_attn_tile(const float *qkv, int heads, int T, int W, const float *cs, const float *sn, int64_t rope_rows,
-                float *out)
+                float *out, int32_t *flag)
 {
     static_assert(HD % 4 == 0 && HD / 4 <= 16, "a lane's p.v takes 4 consecutive dims of 16 groups");
     extern __shared__ float sm[];
@@ -820,8 +822,9 @@ k_dec_attn_tile(const float *qkv, int heads, int T, int W, const float *cs, cons
     const int h = blockIdx.y, t0 = blockIdx.x * ATT_QB, kb = t0 - (W - 1);
     const int tid = threadIdx.x;
     const size_t A = (size_t)heads * HD;
-    const float *q = qkv + (size_t)h * HD * T, *k = qkv + (A + (size_t)h * HD) * T,
-                *v = qkv + (2 * A + (size_t)h * HD) * T;
+    const size_t ch = ROWS ? 1 : T, ps = ROWS ? 3 * A : 1;     // floats between channels, positions
+    const float *q = qkv + (size_t)h * HD * ch, *k = qkv + (A + (size_t)h * HD) * ch,
+                *v = qkv + (2 * A + (size_t)h * HD) * ch;
     float *Ks = sm, *Vs = Ks + NK * KP, *Qs = Vs + NK * KP, *Ps = Qs + ATT_QB * KP;
     // Every global load of the tile first (K and V of the window, Q of the
     // block, the RoPE values of the pairs this thread rotates; clamped, so
@@ -836,15 +839,15 @@ k_dec_attn_tile(const float *qkv, int heads, int T, int W, const float *cs, cons
 #pragma unroll
     for (int u = 0; u < KE; u++) {
         const int i = min(tid + u * 256, HD * NK - 1);
-        const int d = i / NK, j = i - d * NK, pc = min(max(kb + j, 0), T - 1);
-        kraw[u] = k[(size_t)d * T + pc];
-        vraw[u] = v[(size_t)d * T + pc];
+        const int d = ROWS ? i % HD : i / NK, j = ROWS ? i / HD : i - d * NK, pc = min(max(kb + j, 0), T - 1);
+        kraw[u] = k[d * ch + pc * ps];
+        vraw[u] = v[d * ch + pc * ps];
     }
 #pragma unroll
     for (int u = 0; u < QE; u++) {
         const int i = min(tid + u * 256, HD * ATT_QB - 1);
-        const int d = i / ATT_QB, j = i - d * ATT_QB;
-        qraw[u] = q[(size_t)d * T + min(t0 + j, T - 1)];
+        const int d = ROWS ? i % HD : i / ATT_QB, j = ROWS ? i / HD : i - d * ATT_QB;
+        qraw[u] = q[d * ch + min(t0 + j, T - 1) * ps];
     }
     const int64_t rmax = rope_rows - 1;
 #pragma unroll
@@ -867,7 +870,7 @@ k_dec_attn_tile(const float *qkv, int heads, int T, int W, const float *cs, cons
     for (int u = 0; u < KE; u++) {
         const int i = tid + u * 256;
         if (i < HD * NK) {
-            const int d = i / NK, j = i - d * NK, p = kb + j;
+            const int d = ROWS ? i % HD : i / NK, j = ROWS ? i / HD : i - d * NK, p = kb + j;
             const bool ok = p >= 0 && p < T;
             Ks[j * KP + d] = ok ? kraw[u] : 0.0f;
             Vs[j * KP + d] = ok ? vraw[u] : 0.0f;
@@ -877,7 +880,7 @@ k_dec_attn_tile(const float *qkv, int heads, int T, int W, const float *cs, cons
     for (int u = 0; u < QE; u++) {
         const int i = tid + u * 256;
         if (i < HD * ATT_QB) {
-            const int d = i / ATT_QB, j = i - d * ATT_QB;
+            const int d = ROWS ? i % HD : i / ATT_QB, j = ROWS ? i / HD : i - d * ATT_QB;
             Qs[j * KP + d] = t0 + j < T ? qraw[u] : 0.0f;
         }
     }
@@ -953,7 +956,8 @@ k_dec_attn_tile(const float *qkv, int heads, int T, int W, const float *cs, cons
     }
     __syncthreads();
     const int t = t0 + qi;
-    if (4 * kl >= HD) return;
+    if (!ROWS && 4 * kl >= HD) return;
+    static_assert(!ROWS || HD == 64, "sixteen lanes hold a row of a head");
     f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
     const float *pr = Ps + qi * NKP + qi;
     const float *vr = Vs + qi * KP + 4 * kl;
@@ -964,6 +968,24 @@ k_dec_attn_tile(const float *qkv, int heads, int T, int W, const float *cs, cons
         o.y = fmaf(pv, v4.y, o.y);
         o.z = fmaf(pv, v4.z, o.z);
         o.w = fmaf(pv, v4.w, o.w);
+    }
+    if constexpr (ROWS) {
+        // channels 64h + 4kl..+3: record 2h + kl / 8, four slots of it
+        if (t < T) {
+            uint32_t h0, l0, h1, l1;
+            split_f16_pair<true>(o.x, o.y, h0, l0);
+            split_f16_pair<true>(o.z, o.w, h1, l1);
+            uint8_t *y = (uint8_t *)out + (size_t)t * (A * 4) + (2 * h + (kl >> 3)) * 128 + 16 * (kl & 3) + 8 * ((kl >> 2) & 1);
+            *(uint2 *)y = uint2{h0, h1};
+            *(uint2 *)(y + 64) = uint2{l0, l1};
+        }
+        float *red = Qs;                       // the queries are in registers
+        const float mx = wave_max_dpp(t < T ? fmaxf(fmaxf(fabsf(o.x), fabsf(o.y)), fmaxf(fabsf(o.z), fabsf(o.w))) : 0.0f);
+        if ((tid & 63) == 0) red[tid >> 6] = mx;
+        __syncthreads();
+        const float m4 = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+        if (tid == 0 && (!(m4 < 65504.0f) || (m4 > 0.0f && m4 < 0x1p-14f))) *flag = 1;
+        return;
     }
     if (t >= T) return;
     float *op = out + ((size_t)h * HD + 4 * kl) * T + t;
@@ -1341,29 +1363,29 @@ static void col_rms(const float *x, const float *gamma, int H, int T, float *out
         hipLaunchKernelGGL(k_col_rms, dim3((T + 15) / 16), dim3(16 * COLRMS_CG), 0, s, x, gamma, H, T, 1e-5f, out);
 }
 
-hipError_t enqueue_decode(const DecoderDev &d, const DecoderWs &ws, const uint32_t *codes, int T, int64_t cut,
-                          float *audio, hipStream_t s)
+// the tiled attention holds the window in LDS
+bool dec_attn_tiled(const DecoderDev &d)
 {
-    if (T < 1 || T > ws.cap_frames) return hipErrorInvalidValue;
-    if (ws.range_flag) DCHK(hipMemsetAsync(ws.range_flag, 0, sizeof(int32_t), s));
-    const int D = d.codebook_dim, V = d.vq_dim, H = d.hidden, A = d.n_heads * d.head_dim, I = d.inter;
-    const int LAT = d.latent;
-    // 1. VQ -> [V][T]
-    if (d.n_rest == 15)
-        hipLaunchKernelGGL(k_vq_gather<15>, dim3((T + 63) / 64, D), dim3(64), 0, s, d.first_codebook, d.rest_codebooks,
-                           d.n_rest, D, codes, T, d.codebook_size, ws.a);
-    else
-        hipLaunchKernelGGL(k_vq_gather<0>, dim3((T + 63) / 64, D), dim3(64), 0, s, d.first_codebook, d.rest_codebooks,
-                           d.n_rest, D, codes, T, d.codebook_size, ws.a);
-    DCHK(hipGetLastError());
-    DCHK(conv_gemm<CE_STORE>(d.vq_proj, V, causal_in(ws.a, 2 * D, T, 1, 1), plain_out(ws.b, T, nullptr), T, ws, s));
-    // 2. pre-conv -> [LAT][T]
-    DCHK(conv_gemm<CE_STORE>(d.pre_conv.w, d.pre_conv.oc, causal_in(ws.b, V, T, d.pre_conv.k, d.pre_conv.dil),
-                             plain_out(ws.a, T, d.pre_conv.b), T, ws, s));
-    // 3. transformer on [H][T]: x in ws.b, normed in ws.c, q|k|v in ws.d, attention in ws.e
+    return d.window + ATT_QB - 1 <= 16 * ATT_SLOTS && attn_tile_lds(d.head_dim, d.window) <= 65536;
+}
+
+hipError_t enqueue_dec_attn_rows(const DecoderDev &d, const float *qkv, int T, uint8_t *ys, int32_t *flag, hipStream_t s)
+{
+    hipLaunchKernelGGL((k_dec_attn_tile<64, true>), dim3((T + ATT_QB - 1) / ATT_QB, d.n_heads), dim3(256),
+                       attn_tile_lds(d.head_dim, d.window), s, qkv, d.n_heads, T, d.window, d.rope_cos, d.rope_sin,
+                       d.rope_rows, (float *)ys, flag);
+    return hipGetLastError();
+}
+
+// The transformer channel-first (shapes or ranges outside the position-major
+// one): [LAT][T] in ws.a, x in ws.b, normed in ws.c, q|k|v in ws.d, attention
+// in ws.e, back to ws.a.
+static hipError_t enqueue_dec_tf_cf(const DecoderDev &d, const DecoderWs &ws, int T, hipStream_t s)
+{
+    const int H = d.hidden, A = d.n_heads * d.head_dim, I = d.inter, LAT = d.latent;
     DCHK(conv_gemm<CE_STORE>(d.tf_in_w, H, causal_in(ws.a, LAT, T, 1, 1), plain_out(ws.b, T, d.tf_in_b), T, ws, s));
     const size_t att_lds = attn_tile_lds(d.head_dim, d.window);
-    const bool att_tile = d.window + ATT_QB - 1 <= 16 * ATT_SLOTS && att_lds <= 65536;
+    const bool att_tile = dec_attn_tiled(d);
     for (int l = 0; l < d.n_tf; l++) {
         const DecLayer &L = d.tf[l];
         col_rms(ws.b, L.in_norm, H, T, ws.c, s);
@@ -1376,11 +1398,11 @@ hipError_t enqueue_decode(const DecoderDev &d, const DecoderWs &ws, const uint32
         }
         const dim3 ag((T + ATT_QB - 1) / ATT_QB, d.n_heads);
         if (att_tile && d.head_dim == 64)
-            hipLaunchKernelGGL(k_dec_attn_tile<64>, ag, dim3(256), att_lds, s, ws.d, d.n_heads, T, d.window,
-                               d.rope_cos, d.rope_sin, d.rope_rows, ws.e);
+            hipLaunchKernelGGL((k_dec_attn_tile<64, false>), ag, dim3(256), att_lds, s, ws.d, d.n_heads, T, d.window,
+                               d.rope_cos, d.rope_sin, d.rope_rows, ws.e, nullptr);
         else if (att_tile)
-            hipLaunchKernelGGL(k_dec_attn_tile<16>, ag, dim3(256), att_lds, s, ws.d, d.n_heads, T, d.window,
-                               d.rope_cos, d.rope_sin, d.rope_rows, ws.e);
+            hipLaunchKernelGGL((k_dec_attn_tile<16, false>), ag, dim3(256), att_lds, s, ws.d, d.n_heads, T, d.window,
+                               d.rope_cos, d.rope_sin, d.rope_rows, ws.e, nullptr);
         else if (d.head_dim == 64)
             hipLaunchKernelGGL(k_dec_attn<64>, dim3((T + 63) / 64, d.n_heads), dim3(64), 0, s, ws.d, d.n_heads, T,
                                d.window, ws.e);
@@ -1401,6 +1423,34 @@ hipError_t enqueue_decode(const DecoderDev &d, const DecoderWs &ws, const uint32
     col_rms(ws.b, d.tf_norm, H, T, ws.c, s);
     DCHK(hipGetLastError());
     DCHK(conv_gemm<CE_STORE>(d.tf_out_w, LAT, causal_in(ws.c, H, T, 1, 1), plain_out(ws.a, T, d.tf_out_b), T, ws, s));
+    return hipSuccess;
+}
+
+hipError_t enqueue_decode(const DecoderDev &d, const DecoderWs &ws, const uint32_t *codes, int T, int64_t cut,
+                          float *audio, hipStream_t s)
+{
+    if (T < 1 || T > ws.cap_frames) return hipErrorInvalidValue;
+    if (ws.range_flag) DCHK(hipMemsetAsync(ws.range_flag, 0, sizeof(int32_t), s));
+    const int D = d.codebook_dim, V = d.vq_dim;
+    // 1. VQ -> [V][T]
+    if (d.n_rest == 15)
+        hipLaunchKernelGGL(k_vq_gather<15>, dim3((T + 63) / 64, D), dim3(64), 0, s, d.first_codebook, d.rest_codebooks,
+                           d.n_rest, D, codes, T, d.codebook_size, ws.a);
+    else
+        hipLaunchKernelGGL(k_vq_gather<0>, dim3((T + 63) / 64, D), dim3(64), 0, s, d.first_codebook, d.rest_codebooks,
+                           d.n_rest, D, codes, T, d.codebook_size, ws.a);
+    DCHK(hipGetLastError());
+    DCHK(conv_gemm<CE_STORE>(d.vq_proj, V, causal_in(ws.a, 2 * D, T, 1, 1), plain_out(ws.b, T, nullptr), T, ws, s));
+    // 2. pre-conv -> [LAT][T]
+    DCHK(conv_gemm<CE_STORE>(d.pre_conv.w, d.pre_conv.oc, causal_in(ws.b, V, T, d.pre_conv.k, d.pre_conv.dil),
+                             plain_out(ws.a, T, d.pre_conv.b), T, ws, s));
+    // 3. transformer: [LAT][T] in ws.a, back to ws.a
+    if (d.tf_rows && !ws.f32 && dec_x3() && T <= dec_tf_rows(d, ws.part_cap)) {
+        float *const bufs[4] = {ws.b, ws.c, ws.d, ws.e};
+        DCHK(enqueue_dec_tf(d, ws, ws.a, ws.a, bufs, T, s));
+    } else {
+        DCHK(enqueue_dec_tf_cf(d, ws, T, s));
+    }
     // 4. upsample stages: ConvT (phases) then ConvNeXt; the signal moves
     // between ws.a and ws.b
     int L = T;

@@ -165,7 +165,12 @@ struct DecConvT {            // kernel == stride (1 tap) or 2*stride (2 taps), p
     const uint8_t *pw;       // as DecConv, rows [stride][oc]
     const float *un;
 };
+struct DecLin {              // split weights of 64-channel tiles (qtts_dconv.hip), their rows' factors
+    const uint8_t *w;
+    const float *un;
+};
 struct DecLayer {
+    DecLin pqkv, po, pgu, pdown;
     const float *qkv;        // [3A][hidden] rows q, k, v
     const float *o;          // [hidden][A]
     const float *gate_up;    // [2 inter][hidden] rows gate_j, up_j interleaved
@@ -214,6 +219,8 @@ struct DecoderDev {
     int out_k, out_dil;
     const float *rope_cos, *rope_sin;
     int64_t rope_rows;
+    DecLin tf_in, tf_out;
+    bool tf_rows;                         // the transformer runs position-major (qtts_dconv.hip)
     bool vocos_rows;                      // the Vocos stages run position-major (qtts_dconv.hip)
     bool weights_f32;                     // a weight matrix outside the split-f16 range: f32 matrix path
 };
@@ -336,7 +343,14 @@ hipError_t enqueue_decode(const DecoderDev &d, const DecoderWs &ws, const uint32
                           float *audio, hipStream_t s);
 bool vocos_fits(const DecoderDev &d);
 size_t dconv_weight_bytes(int rows, int ic, int kt);
-hipError_t enqueue_dconv_pack(const float *w, int rows, int ic, int kt, uint8_t *out, float *un, hipStream_t s);
+constexpr int DC_VOCOS_CB = 6, DC_TF_CB = 4;   // 16-channel blocks a tile
+hipError_t enqueue_dconv_pack(const float *w, int rows, int ic, int kt, int cb, uint8_t *out, float *un, hipStream_t s);
+bool dec_tf_fits(const DecoderDev &d);
+int dec_tf_rows(const DecoderDev &d, size_t part_floats);
+hipError_t enqueue_dec_tf(const DecoderDev &d, const DecoderWs &ws, const float *in, float *out, float *const bufs[4], int T,
+                          hipStream_t s);
+bool dec_attn_tiled(const DecoderDev &d);
+hipError_t enqueue_dec_attn_rows(const DecoderDev &d, const float *qkv, int T, uint8_t *ys, int32_t *flag, hipStream_t s);
 hipError_t enqueue_snake_par(const float *alpha, const float *beta, int n, float *out, hipStream_t s);
 hipError_t enqueue_vocos(const DecoderDev &d, const DecoderWs &ws, const float *sig, float *const bufs[4], int L, int64_t cut,
                          float *audio, bool fuse, hipStream_t s);

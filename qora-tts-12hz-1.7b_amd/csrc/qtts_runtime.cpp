@@ -1913,23 +1913,41 @@ static int upload_convt(qtts_ctx *c, const qtts_convt1d_host &h, DecConvT *d)
     return upload_vec(c, c->dec_allocs, h.bias, (size_t)OC, &d->b);
 }
 
-// The position-major Vocos stages' copies: split weights in fragment order
+// The position-major stages' copies: split weights in fragment order
 // and the snakes' exponentials, made on the device from what was uploaded
 // (the f32 weights stay for the f32 matrix path).
-static int pack_vocos(qtts_ctx *c)
+static int pack_rows(qtts_ctx *c)
 {
     DecoderDev &d = c->dec;
-    d.vocos_rows = vocos_fits(d);
-    if (!d.vocos_rows) return QTTS_OK;
-    const auto conv = [&](const float *w, int rows, int ic, int kt, const uint8_t **pw, const float **un) {
+    const auto pack = [&](const float *w, int rows, int ic, int kt, int cb, const uint8_t **pw, const float **un) {
         uint8_t *p = nullptr;
         float *u = nullptr;
         RCHK(dev_alloc(c, c->dec_allocs, &p, dconv_weight_bytes(rows, ic, kt)));
         RCHK(dev_alloc(c, c->dec_allocs, &u, rows));
-        HIPCHK(c, enqueue_dconv_pack(w, rows, ic, kt, p, u, c->stream));
+        HIPCHK(c, enqueue_dconv_pack(w, rows, ic, kt, cb, p, u, c->stream));
         *pw = p;
         *un = u;
         return QTTS_OK;
+    };
+    d.tf_rows = dec_tf_fits(d);
+    if (d.tf_rows) {
+        const int H = d.hidden, A = d.n_heads * d.head_dim;
+        const auto lin = [&](const float *w, int rows, int ic, DecLin *o) {
+            return pack(w, rows, ic, 1, DC_TF_CB, &o->w, &o->un);
+        };
+        RCHK(lin(d.tf_in_w, H, d.latent, &d.tf_in));
+        for (DecLayer &L : c->dec_layers) {
+            RCHK(lin(L.qkv, 3 * A, H, &L.pqkv));
+            RCHK(lin(L.o, H, A, &L.po));
+            RCHK(lin(L.gate_up, 2 * d.inter, H, &L.pgu));
+            RCHK(lin(L.down, H, d.inter, &L.pdown));
+        }
+        RCHK(lin(d.tf_out_w, d.latent, H, &d.tf_out));
+    }
+    d.vocos_rows = vocos_fits(d);
+    if (!d.vocos_rows) return QTTS_OK;
+    const auto conv = [&](const float *w, int rows, int ic, int kt, const uint8_t **pw, const float **un) {
+        return pack(w, rows, ic, kt, DC_VOCOS_CB, pw, un);
     };
     const auto snake = [&](const float *alpha, const float *beta, int n, const float **out) {
         float *p = nullptr;
@@ -2106,7 +2124,7 @@ static int upload_decoder(qtts_ctx *c, const qtts_decoder_host *h)
     RCHK(upload_vec(c, A, h->rope_sin, (size_t)h->rope_max_pos * (HD / 2), &d.rope_sin));
     d.rope_rows = h->rope_max_pos;
     c->dec_floats_per_frame = fpf;
-    return pack_vocos(c);
+    return pack_rows(c);
 }
 
 static void free_decoder(qtts_ctx *c)
