@@ -171,7 +171,7 @@ __device__ __forceinline__ f32x4 dc_epi(const DcOut &o, f32x4 acc, const f32x4 &
 }
 
 template <int CB, int PB, int KT, int EPI, bool FUSE, bool SK>
-__global__ void __launch_bounds__(256, 2)
+__global__ void __launch_bounds__(256, SK && KT > 2 ? 1 : 2)
 k_dconv(DcIn in, const uint8_t *wts, DcOut o, DcGeo g, DcFuse fz)
 {
     // SK: the waves share the positions (16 PB) and take every fourth record
@@ -210,12 +210,21 @@ k_dconv(DcIn in, const uint8_t *wts, DcOut o, DcGeo g, DcFuse fz)
         if (r < R) *(u32x4 *)&lds[buf * lbuf + r * 128 + (((idx & 7) ^ ((r >> 1) & 7)) * 16)] = v;
     };
     const uint8_t *wb = wts + (((size_t)(ph * g.tm + ct) * in.nc + c0) * KT) * (CB * 2048) + 16 * lane;
-    half8 wr[CB][2];
-    // block b of tap `tap` of the wave's record i
-    const auto load_w = [&](int b, int i, int tap) {
+    // SK: one wave a SIMD (the staged rows fill the LDS) and nothing else to
+    // cover the L2's latency, so its weights come two steps ahead, in the
+    // registers that leaves: decode of 5 frames 1.12 -> 1.06 ms, of 21 frames
+    // 1.48 -> 1.40 ms, of 40 frames 2.04 -> 1.89 ms.  With one or two taps a
+    // wave has too few steps: the second set costs 1 frame 0.02 ms.
+    constexpr int WS = SK && KT > 2 ? 2 : 1;
+    half8 wr[WS][CB][2];
+    // block b of the wave's step st (record st / KT, tap st % KT) into set u
+    const int nst = nrec * KT;
+    const auto load_w = [&](int u, int b, int st) {
+        st = min(st, nst - 1);
+        const int i = st / KT, tap = st - i * KT;
         const uint8_t *p = wb + (size_t)(i * CS * KT + tap) * (CB * 2048) + b * 2048;
-        wr[b][0] = *(const half8 *)p;
-        wr[b][1] = *(const half8 *)(p + 1024);
+        wr[u][b][0] = *(const half8 *)p;
+        wr[u][b][1] = *(const half8 *)(p + 1024);
     };
     f32x4 acc[PB][CB];
 #pragma unroll
@@ -228,7 +237,9 @@ k_dconv(DcIn in, const uint8_t *wts, DcOut o, DcGeo g, DcFuse fz)
 #pragma unroll
         for (int i = 0; i < NP; i++) v[i] = piece(i, c0);
 #pragma unroll
-        for (int b = 0; b < CB; b++) load_w(b, 0, 0);
+        for (int u = 0; u < WS; u++)
+#pragma unroll
+            for (int b = 0; b < CB; b++) load_w(u, b, u);
 #pragma unroll
         for (int i = 0; i < NP; i++) put(i, 0, v[i]);
     }
@@ -254,23 +265,34 @@ k_dconv(DcIn in, const uint8_t *wts, DcOut o, DcGeo g, DcFuse fz)
                 xh[p] = *(const half8 *)&lds[buf * lbuf + r * 128 + ((q ^ z) * 16)];
                 xl[p] = *(const half8 *)&lds[buf * lbuf + r * 128 + (((q + 4) ^ z) * 16)];
             }
-            const int wn = tap + 1 < KT ? c : min(c + 1, nrec - 1), wt = tap + 1 < KT ? tap + 1 : 0;
+            const int u = tap % WS;
 #pragma unroll
             for (int b = 0; b < CB; b++) {
 #pragma unroll
                 for (int p = 0; p < PB; p++)
-                    acc[p][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wr[b][1], xh[p], acc[p][b], 0, 0, 0);
+                    acc[p][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wr[u][b][1], xh[p], acc[p][b], 0, 0, 0);
 #pragma unroll
                 for (int p = 0; p < PB; p++)
-                    acc[p][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wr[b][0], xl[p], acc[p][b], 0, 0, 0);
+                    acc[p][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wr[u][b][0], xl[p], acc[p][b], 0, 0, 0);
 #pragma unroll
                 for (int p = 0; p < PB; p++)
-                    acc[p][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wr[b][0], xh[p], acc[p][b], 0, 0, 0);
-                load_w(b, wn, wt);
+                    acc[p][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wr[u][b][0], xh[p], acc[p][b], 0, 0, 0);
+                load_w(u, b, c * KT + tap + WS);
             }
 #pragma unroll
             for (int i = 0; i < PPT; i++)
                 if (tap * PPT + i < NP) put(tap * PPT + i, buf ^ 1, v[i]);
+        }
+        if constexpr (WS == 2 && KT % 2) {
+            // an odd record ends on the other set
+#pragma unroll
+            for (int b = 0; b < CB; b++)
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    const half8 t = wr[0][b][j];
+                    wr[0][b][j] = wr[WS - 1][b][j];
+                    wr[WS - 1][b][j] = t;
+                }
         }
         if constexpr (SK) {
             // one wave's lanes hand each other rows through LDS
