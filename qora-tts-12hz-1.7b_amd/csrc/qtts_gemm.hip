@@ -174,6 +174,14 @@ k_split_rows(const float *X, int ld, int K, int seg, uint8_t *out, int kc, float
 // row ^ part: writes (16 lanes of one row, 16 parts) and reads (16 rows of
 // one part) both spread over all banks.  Two register sets hold the next two
 // chunks' rows and weights.
+//
+// Measured (a talker layer of a 400-row prompt, against a kernel that
+// converted both operands while staging them): gate|up 103 -> 57 us (1.06
+// PFLOP/s of f16 products, 87% of what a large matrix product reaches),
+// q|k|v 37 -> 26, o 22 -> 21, down 49 -> 47.  The last three make 640 tiles:
+// 2.5 rounds over the 256 CUs that run as 3.  More waves a SIMD (row blocks
+// of 4: 59 -> 70 us) and an interleave of the instruction groups asked of
+// the scheduler (it spills) were slower.
 // ---------------------------------------------------------------------------
 
 enum { MM_STORE = 0, MM_PART = 1, MM_PART_DUAL = 2, MM_SWIGLU = 3 };
@@ -235,7 +243,7 @@ k_q4_gemm(RowsSplit a, Q4Frag w, MmOut o, int tm, int nrun, int run_chunks)
 
     // register sets of rows and of weights: a tall tile's chunk covers the
     // loads by itself; short tiles run one segment, all of it in flight at once
-    constexpr int AS = MB <= 2 ? 4 : MB >= 6 || (FP == 1 && MB >= 5) ? 1 : 2, WS = MB <= 2 ? 4 : 2;
+    constexpr int AS = MB <= 2 ? 4 : FP == 1 && MB >= 5 ? 1 : 2, WS = MB <= 2 ? 4 : 2;
     u32x4 ra[AS][MB];
     u32x4 rn[WS];
     half8 rs[WS][DUAL ? 4 : 2];       // [set][half of the chunk (+ 2 block)]
@@ -502,8 +510,12 @@ hipError_t enqueue_frag_build(const Q4Tiled &w, const Q4Frag &f, uint8_t *out, h
 }
 
 // k-slices of a weight whose consumer adds partial sums: a divisor of its
-// segments, about 96 column tiles x slices per row tile.  A property of the
-// weight alone (a row's bits do not depend on the batch).
+// segments, at most 144 column tiles x slices per row tile (128 for the
+// talker's q|k|v, o and down).  A property of the weight alone (a row's bits
+// do not depend on the batch), so one count serves every row count: 128 is
+// half the CUs per row tile, which fills them from two row tiles on; 96 would
+// lie better at 400 rows (480 tiles, not 640) and worse at 1100 (6 rounds of
+// 4 segments against 7 of 3).
 int mm_slices(const Q4Frag &w)
 {
     const int tn = (w.ng + 3) / 4, nseg = (w.kc + 3) / 4;
@@ -517,7 +529,9 @@ static int mm_segments(const Q4Frag &w) { return (w.kc + 3) / 4; }
 
 // Row blocks per tile: the row tiles x columns x runs fill the 256 CUs in
 // whole rounds; a tile's time is its matrix work (MB) plus what does not
-// depend on the rows (the weight's dequantisation, ~1.5 row blocks).
+// depend on the rows (the weight's dequantisation, ~1.5 row blocks, fitted to
+// gate|up of 128, 400 and 1024 rows: 34.9, 56.7 and 144 us).  Six row blocks
+// spill with half a chunk's weights dequantised ahead.
 static int mm_mb(int M, int per_tile, int max_mb)
 {
     int best = 1;
@@ -548,9 +562,9 @@ static hipError_t launch_mm(const RowsSplit &a, const Q4Frag &w, const MmOut &o,
     switch (mb) {
 #define MM_CASE(B) \
     case B: hipLaunchKernelGGL((k_q4_gemm<B, FP, EPI>), grid, dim3(256), 0, s, a, w, o, tm, nrun, run_chunks); break;
-        MM_CASE(1) MM_CASE(2) MM_CASE(3) MM_CASE(4) MM_CASE(5)
+        MM_CASE(1) MM_CASE(2) MM_CASE(3) MM_CASE(4)
 #undef MM_CASE
-    default: hipLaunchKernelGGL((k_q4_gemm<6, FP, EPI>), grid, dim3(256), 0, s, a, w, o, tm, nrun, run_chunks); break;
+    default: hipLaunchKernelGGL((k_q4_gemm<MM_MAX_MB, FP, EPI>), grid, dim3(256), 0, s, a, w, o, tm, nrun, run_chunks); break;
     }
     return hipGetLastError();
 }
@@ -564,7 +578,8 @@ hipError_t enqueue_split_rows(const float *X, int ld, int M, int K, int seg, uin
 
 // Rows up to which a prompt's GEMMs run one workgroup per K segment (each
 // writes its own partial sums) instead of one per slice: few row tiles leave
-// the chip idle behind long K loops, and the partial sums are still small.
+// the chip idle behind long K loops, and the partial sums are still small:
+// 28 layers of 10 rows 1.56 -> 1.44 ms, of 3 rows 1.51 -> 1.38.
 constexpr int MM_SEG_ROWS = 64;
 
 static int mm_run_chunks(const Q4Frag &w, int M)
