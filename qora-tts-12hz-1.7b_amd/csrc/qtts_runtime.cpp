@@ -818,16 +818,17 @@ extern "C" int qtts_gemm_q4_noalloc(qtts_ctx *c, const qtts_w *w, const float *X
     if (rows > (1 << 20)) return fail(c, QTTS_ERR_CAPACITY, "at most %d rows", 1 << 20);
     hipSetDevice(c->device);
     const Q4Tiled &t = w->t;
-    if (use_mfma(flags, rows) && gemm_supported(t)) {
-        // more rows than the scratch holds go in batches
+    const bool mx = use_mfma(flags, rows) && gemm_supported(t);
+    // a weight whose GEMV passes do not fit is refused for any few rows, not
+    // only for the one or two that take them
+    const size_t need = (size_t)t.S * 2 * t.npad;
+    if (need > SCRATCH_FLOATS && (!mx || (rows < 16 && !(flags & QTTS_PATH_MFMA))))
+        return fail(c, QTTS_ERR_CAPACITY, "this weight's GEMV passes need %zu floats of scratch; the maximum is %zu", need,
+                    SCRATCH_FLOATS);
+    if (mx)   // more rows than the scratch holds go in batches
         HIPCHK(c, enqueue_gemm_rows(t, w->f, X, (int)rows, Y, t.n, c->scratch, SCRATCH_FLOATS, c->stream));
-    } else {
-        const size_t need = (size_t)t.S * 2 * t.npad;
-        if (need > SCRATCH_FLOATS)
-            return fail(c, QTTS_ERR_CAPACITY, "this weight's GEMV passes need %zu floats of scratch; the maximum is %zu",
-                        need, SCRATCH_FLOATS);
+    else
         HIPCHK(c, enqueue_gemv_rows(t, X, (int)rows, Y, c->scratch, c->stream));
-    }
     // columns past the last full group are zero (gemv.rs:255)
     const int full = (t.n / 32) * 32;
     HIPCHK(c, enqueue_zero_cols(Y, (int)rows, t.n, full, t.n, c->stream));

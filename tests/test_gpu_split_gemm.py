@@ -13,7 +13,9 @@ matrix instruction.
 import numpy as np
 import pytest
 
+import qtts
 from qtts import synth
+from test_zz_no_alloc import DevBuf, hip
 
 pytestmark = pytest.mark.gpu
 
@@ -80,3 +82,30 @@ def test_zero_and_not_finite_rows(ctx):
     assert np.array_equal(bits(Y[keep]), bits(ref[keep]))
     assert not Y[3].any() and not np.isfinite(Y[5]).any() and not np.isfinite(Y[21]).any()
     dw.free()
+
+
+def test_noalloc_refusal_does_not_depend_on_the_path(ctx_factory, monkeypatch):
+    """16 slices of 128 rows (tile G8_T128) x 33,792 columns: GEMV partial sums
+    beyond the workspace.  Refused at any few rows, also those that the matrix
+    cores take by themselves; asked for, the matrix cores run."""
+    monkeypatch.setenv("QTTS_TILE_GEMV", "1")
+    c = ctx_factory(256)
+    rng = np.random.Generator(np.random.PCG64(78))
+    dw = c.upload(synth.q4_random(rng, 2048, 33792))
+    x = rng.standard_normal((16, 2048)).astype(np.float32)
+    h = hip()
+    dx, dy = DevBuf(h, x.nbytes), DevBuf(h, 16 * 33792 * 4)
+    try:
+        dx.put(x)
+        for rows in (1, 3, 15):
+            with pytest.raises(qtts.QttsError) as e:
+                c.gemm_noalloc(dw, dx.ptr.value, rows, dy.ptr.value)
+            assert e.value.code == qtts.ERR_CAPACITY
+        for rows, path in ((3, "mfma"), (16, None)):
+            c.gemm_noalloc(dw, dx.ptr.value, rows, dy.ptr.value, path=path)
+            c.sync()
+            assert np.array_equal(bits(dy.get((rows, 33792))), bits(c.gemm(dw, x[:rows], path="mfma")))
+    finally:
+        dx.free()
+        dy.free()
+        dw.free()
