@@ -17,8 +17,8 @@
 // then k_final_rms on the last row (talker.rs:477-481).
 //
 // k_q4_gemm (qtts_gemm.hip) contracts on the f16 matrix cores with split
-// operands, f32-accurate.  With QTTS_GEMM_F32=1, or for a layer weight whose
-// scales leave the split's range, the prompt runs on k_gemm_q4 below instead:
+// operands, f32-accurate.  With QTTS_GEMM_F32=1, or in a layer with a weight
+// whose scales leave the split's range, the GEMMs run on k_gemm_q4 below instead:
 // f32 rows, v_mfma_f32_16x16x4_f32, the decode GEMV's tiled weights.
 
 #include "qtts_device.h"
@@ -909,6 +909,20 @@ int norm_shift(const uint16_t *gamma_host, int n)
     return bound_shift(std::sqrt((double)n) * f16_max_abs(gamma_host, n));
 }
 
+static bool layer_has_frags(const LayerDev &L)
+{
+    return L.qkv_f.data && L.o_f.data && L.gate_up_f.data && L.down_f.data;
+}
+
+// Whether a layer takes the split GEMM: all four matrices, since each hands
+// its successor rows in the form that one reads.  A layer with a matrix
+// outside the split's range (a scale of 4096 or more) runs on the f32
+// instructions, the others as before.
+static bool split_layer(const TalkerDev &m, int l)
+{
+    return gemm_x3() && layer_has_frags(m.layers[l]);
+}
+
 // Floats of partial sums the prompt's projections need at up to `rows` rows.
 int64_t prefill_part_floats(const TalkerDev &m, int rows)
 {
@@ -916,7 +930,7 @@ int64_t prefill_part_floats(const TalkerDev &m, int rows)
     for (int l = 0; l < m.n_layers; l++) {
         const LayerDev &L = m.layers[l];
         for (const Q4Tiled *w : {&L.qkv, &L.o, &L.down}) f = std::max<int64_t>(f, (int64_t)rows * part_slices(*w) * w->G * 32);
-        if (!L.qkv_f.data) continue;
+        if (!layer_has_frags(L)) continue;
         // a small batch may cut K finer than a large one
         for (int r : {rows, std::min(64, rows), std::min(16, rows)}) {
             f = std::max<int64_t>(f, (int64_t)mm_part_floats(L.qkv_f, r));
@@ -932,16 +946,6 @@ hipError_t enqueue_fill_rows(float *x, int64_t n, uint32_t seed, hipStream_t s)
 {
     hipLaunchKernelGGL(k_fill_rows, dim3(1024), dim3(256), 0, s, x, n, seed);
     return hipGetLastError();
-}
-
-static bool split_path(const TalkerDev &m)
-{
-    if (!gemm_x3() || m.hidden > 2048) return false;
-    for (int l = 0; l < m.n_layers; l++) {
-        const LayerDev &L = m.layers[l];
-        if (!L.qkv_f.data || !L.o_f.data || !L.gate_up_f.data || !L.down_f.data) return false;
-    }
-    return true;
 }
 
 template <int NP>
@@ -970,7 +974,7 @@ struct QkvPost {
 hipError_t enqueue_gemm_gateup(const TalkerDev &m, const PrefillWs &pw, int l, int M, hipStream_t s)
 {
     const LayerDev &L = m.layers[l];
-    if (split_path(m)) {
+    if (split_layer(m, l)) {
         const int kc = (m.hidden + 63) / 64;
         return enqueue_mm_swiglu(RowsSplit{(const uint8_t *)pw.xs, kc, M, nullptr, 0, __builtin_ldexpf(1.0f, -L.post_shift)},
                                  L.gate_up_f, pw.part, (uint8_t *)pw.h, (m.inter + 63) / 64, pw.rsc, s);
@@ -983,7 +987,7 @@ hipError_t enqueue_gemm_gateup(const TalkerDev &m, const PrefillWs &pw, int l, i
 // layer l's staging), or their 1/rms.
 hipError_t enqueue_gateup_input(const TalkerDev &m, const PrefillWs &pw, int l, int M, hipStream_t s)
 {
-    const bool sp = split_path(m);
+    const bool sp = split_layer(m, l);
     return ResidNorm<1>::go(pw.x, m.hidden, M, MmParts{}, pw.inv, sp ? m.layers[l].post_norm : nullptr,
                             m.layers[l].post_shift, sp ? (uint8_t *)pw.xs : nullptr, s);
 }
@@ -1005,16 +1009,17 @@ hipError_t enqueue_talker_prefill(const TalkerDev &m, const PrefillWs &pw, int M
 {
     if (M < 1 || M > pw.cap_rows || m.hidden > 2048) return hipErrorInvalidValue;
     const int H = m.hidden, A = 16 * HEAD_DIM, kh = (H + 63) / 64, ki = (m.inter + 63) / 64;
-    const bool sp = split_path(m);
-    uint8_t *xs = sp ? (uint8_t *)pw.xs : nullptr;
+    uint8_t *const xs = (uint8_t *)pw.xs;
     MmParts p{};
-    // x += parts, then the rows the next GEMM takes
-    const auto resid = [&](const uint16_t *gamma, int shift) {
-        return by_parts<ResidNorm>(p.n, pw.x, H, M, p, pw.inv, sp ? gamma : nullptr, shift, gamma ? xs : nullptr, s);
+    // x += parts, then the rows the next GEMM takes: normed and split, or
+    // their 1/rms for the f32 instructions
+    const auto resid = [&](bool split, const uint16_t *gamma, int shift) {
+        return by_parts<ResidNorm>(p.n, pw.x, H, M, p, pw.inv, split ? gamma : nullptr, shift, split ? xs : nullptr, s);
     };
-    PCHK(resid(m.layers[0].input_norm, m.layers[0].in_shift));
+    PCHK(resid(split_layer(m, 0), m.layers[0].input_norm, m.layers[0].in_shift));
     for (int l = 0; l < m.n_layers; l++) {
         const LayerDev &L = m.layers[l];
+        const bool sp = split_layer(m, l);
         // q|k|v, QK-norm + RoPE + KV append, attention
         if (sp)
             PCHK(enqueue_mm_parts(RowsSplit{xs, kh, M, nullptr, 0, __builtin_ldexpf(1.0f, -L.in_shift)}, L.qkv_f, false,
@@ -1032,8 +1037,8 @@ hipError_t enqueue_talker_prefill(const TalkerDev &m, const PrefillWs &pw, int M
                                    m.kv, l, pw.attn, A, as, pw.rsc, M, 0, 0, 0);
             PCHK(hipGetLastError());
         } else {
-            // f32 rows over the q rows' own (pw.part holds at least M rows of
-            // them): split from there
+            // f32 rows in pw.part (at least M rows of the q|k|v's sums, which
+            // have been read), split from there
             float *out = sp ? pw.part : pw.attn;
             hipLaunchKernelGGL(k_prefill_attn<PREFILL_ATTN_QB>, dim3((M + PREFILL_ATTN_QB - 1) / PREFILL_ATTN_QB, 8),
                                dim3(256), 0, s, pw.q, A, M, start, m.kv, l, out, A);
@@ -1045,15 +1050,17 @@ hipError_t enqueue_talker_prefill(const TalkerDev &m, const PrefillWs &pw, int M
             PCHK(enqueue_mm_parts(RowsSplit{as, A / 64, M, pw.rsc, M, 1.0f}, L.o_f, false, pw.part, &p, s));
         else
             PCHK(gemm_parts(GemmA{pw.attn, A, nullptr, nullptr, M}, L.o, pw, &p, s));
-        PCHK(resid(L.post_norm, L.post_shift));
+        PCHK(resid(sp, L.post_norm, L.post_shift));
         // gate|up with SwiGLU, down, residual, next layer's input norm
         PCHK(enqueue_gemm_gateup(m, pw, l, M, s));
         if (sp)
             PCHK(enqueue_mm_parts(RowsSplit{(const uint8_t *)pw.h, ki, M, pw.rsc, M, 1.0f}, L.down_f, true, pw.part, &p, s));
         else
             PCHK(gemm_parts(GemmA{pw.h, m.inter, nullptr, nullptr, M}, L.down, pw, &p, s));
-        const bool last = l + 1 == m.n_layers;
-        PCHK(resid(last ? nullptr : m.layers[l + 1].input_norm, last ? 0 : m.layers[l + 1].in_shift));
+        if (l + 1 < m.n_layers)
+            PCHK(resid(split_layer(m, l + 1), m.layers[l + 1].input_norm, m.layers[l + 1].in_shift));
+        else
+            PCHK(resid(false, nullptr, 0));
     }
     hipLaunchKernelGGL(k_final_rms, dim3(1), dim3(256), 0, s, pw.x + (size_t)(M - 1) * H, m.final_norm, H,
                        hidden_out);

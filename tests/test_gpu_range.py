@@ -190,6 +190,33 @@ def test_prefill_mfma_out_of_f16_range(ctx_factory, case):
     om.close()
 
 
+@pytest.mark.parametrize("matrix", ["q_proj", "o_proj", "up_proj", "down_proj"])
+def test_prefill_one_matrix_outside_the_split(ctx_factory, matrix):
+    """One matrix of the middle layer with a scale of 5000 (no split copy of
+    it): that layer on the f32 instructions between two split ones, hidden and
+    every layer's cache against the oracle.  101 rows (sums by slice), 7 (by K
+    segment)."""
+    t = synth.make_talker(seed=9450, n_layers=3, text_vocab=256, rope_max_pos=256)
+    w = getattr(t.layers[1], matrix)
+    w.scales[3, 1] = np.array(5000.0, np.float16).view(np.uint16)
+    c = ctx_factory(256)
+    c.upload_model(t, synth.make_predictor(seed=9451, n_layers=1))
+    om = O.Model(t, synth.make_predictor(seed=9451, n_layers=1), kv_cap=256)
+    X = np.random.Generator(np.random.PCG64(9452)).standard_normal((101, t.hidden)).astype(np.float32)
+    for rows in (101, 7):
+        print(f"{matrix} rows={rows}", flush=True)
+        c.kv_reset()
+        om.kv_reset()
+        ref = om.prefill(X[:rows], 0)
+        ok, e = close(c.prefill_talker_raw_from(X[:rows], 0, path="mfma"), ref)
+        assert ok, f"{matrix}, {rows} rows: hidden rel err {e}"
+        for l in range(3):
+            for got, want in zip(c.kv_gather(l), om.kv_layer(l)):
+                for pos in (0, rows // 2, rows - 1):
+                    assert close(got[pos], want[pos])[0], f"{matrix}, {rows} rows: layer {l} position {pos}"
+    om.close()
+
+
 @pytest.mark.parametrize("e", [17, -14])
 def test_text_projection_out_of_f16_range(ctx_factory, e):
     """The text projection on the matrix cores (fc1 + bias, SiLU, fc2 +
