@@ -343,6 +343,9 @@ static int build_tiled(qtts_ctx *c, std::vector<void *> &allocs, const std::vect
 
 // The matrix cores' copy of a tiled weight, permuted on the device (the same
 // nibbles and scales; null where the split GEMM does not take the weight).
+// Made on the null stream, as the tiles' copies are, and complete on return:
+// the context's stream may hold queued work, and other contexts' streams do
+// not wait for it.
 static int build_frag(qtts_ctx *c, std::vector<void *> &allocs, const Q4Tiled &t, Q4Frag *out)
 {
     *out = Q4Frag{};
@@ -352,7 +355,8 @@ static int build_frag(qtts_ctx *c, std::vector<void *> &allocs, const Q4Tiled &t
     void *mem = nullptr;
     HIPCHK(c, hipMalloc(&mem, bytes));
     allocs.push_back(mem);
-    HIPCHK(c, enqueue_frag_build(t, f, (uint8_t *)mem, c->stream));
+    HIPCHK(c, enqueue_frag_build(t, f, (uint8_t *)mem, nullptr));
+    HIPCHK(c, hipStreamSynchronize(nullptr));
     f.data = (const uint8_t *)mem;
     *out = f;
     return QTTS_OK;

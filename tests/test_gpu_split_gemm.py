@@ -109,3 +109,28 @@ def test_noalloc_refusal_does_not_depend_on_the_path(ctx_factory, monkeypatch):
         dx.free()
         dy.free()
         dw.free()
+
+
+def test_weight_uploaded_behind_queued_work(ctx_factory):
+    """An uploaded weight is complete on return: uploaded by a context that
+    still has GEMMs queued on its stream, used at once by another one."""
+    a, b = ctx_factory(256), ctx_factory(256)
+    rng = np.random.Generator(np.random.PCG64(80))
+    w0, w = synth.q4_random(rng, 6144, 2048), synth.q4_random(rng, 2048, 1024)
+    d0 = a.upload(w0)
+    h = hip()
+    rows = 2000
+    dx, dy = DevBuf(h, rows * 6144 * 4), DevBuf(h, rows * 2048 * 4)
+    X = rng.standard_normal((20, 2048)).astype(np.float32)
+    try:
+        dx.put(np.zeros((rows, 6144), np.float32))
+        for _ in range(50):
+            a.gemm_noalloc(d0, dx.ptr.value, rows, dy.ptr.value)
+        dw = a.upload(w)
+        check(b.gemm(dw, X, path="mfma"), X, w)
+        a.sync()
+        dw.free()
+    finally:
+        dx.free()
+        dy.free()
+        d0.free()
