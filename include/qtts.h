@@ -556,6 +556,11 @@ int qtts_gen_state(qtts_ctx *ctx, float *logits, float *hidden,
  * timeout. */
 int qtts_debug_force_sync_err(qtts_ctx *ctx);
 
+/* Test hook, no reference counterpart: a figure of the context's state after
+ * its last call.  QTTS_ERR_INVALID for another `what`. */
+#define QTTS_QUERY_STAGING 0    /* bytes of the host staging buffer still taken (0 between calls) */
+int qtts_debug_query(qtts_ctx *ctx, int32_t what, int64_t *value);
+
 /* ---- measurement ------------------------------------------------------ */
 
 /* Average device time (us) of one kernel launch: one HIP event pair around

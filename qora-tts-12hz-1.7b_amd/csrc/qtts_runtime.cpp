@@ -157,6 +157,10 @@ static int fail(qtts_ctx *c, int code, const char *fmt, ...)
         va_end(ap);
         c->err = buf;
         c->outs.clear();     // a failed call hands over nothing
+        if (c->pin_top) {    // and gives its staging slots back, once nothing reads them
+            hipStreamSynchronize(c->stream);
+            c->pin_top = 0;
+        }
     }
     return code;
 }
@@ -2288,7 +2292,7 @@ extern "C" int qtts_predictor_chain(qtts_ctx *c, const float *th, const float *s
                              c->stream));
     DevState back{};
     HIPCHK(c, hipMemcpyAsync(&back, c->st_api, sizeof(DevState), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    RCHK(finish(c));
     if (back.nan_flag) return fail(c, QTTS_ERR_NAN, "NaN logits in the predictor");
     if (back.sync_err) return fail(c, QTTS_ERR_HIP, "a cross-workgroup wait timed out (predictor q|k|v + attention launch)");
     return QTTS_OK;
@@ -2700,6 +2704,15 @@ extern "C" int qtts_debug_force_sync_err(qtts_ctx *c)
     NEED_MODEL(c);
     c->force_sync_err = true;
     return QTTS_OK;
+}
+
+extern "C" int qtts_debug_query(qtts_ctx *c, int32_t what, int64_t *value)
+{
+    if (!c || !value) return QTTS_ERR_INVALID;
+    switch (what) {
+    case QTTS_QUERY_STAGING: *value = (int64_t)c->pin_top; return QTTS_OK;
+    default: return QTTS_ERR_INVALID;
+    }
 }
 
 // ---------------------------------------------------------------------------

@@ -215,3 +215,27 @@ def test_codec_vocab_not_whole_groups_refused(ctx_factory):
     X = np.random.Generator(np.random.PCG64(705)).standard_normal((4, t.hidden)).astype(np.float32)
     lg = c.apply_codec_head(c.prefill_talker_raw_from(X, 0))
     assert lg.shape == (3072,) and np.isfinite(lg).all()
+
+
+def test_staging_slots_given_back(ctx_factory, model):
+    """Every call gives the host staging buffer's slots back, a refused one
+    too (an unknown speaker behind a staged voice vector): slots that stayed
+    taken would send all later calls to the runtime's blocking copies."""
+    t, p = model
+    c = ctx_factory(256)
+    c.upload_model(t, p)
+    rng = np.random.Generator(np.random.PCG64(7200))
+    th, sem = rng.standard_normal((2, t.hidden)).astype(np.float32)
+    first = c.generate_acoustic_codes(th, sem)
+    for _ in range(80):                            # 80 x 16 KB: more than the buffer
+        codes = c.generate_acoustic_codes(th, sem)
+        assert c.debug_query("staging") == 0
+    assert np.array_equal(codes, first)
+    with pytest.raises(qtts.QttsError) as e:
+        c.build_prefill_head(10 ** 6, 2055, voice=th)
+    assert e.value.code == qtts.ERR_INVALID
+    assert c.debug_query("staging") == 0
+    c.forward_with_embedding(th, 0)
+    c.apply_codec_head(th)
+    c.embed_codec_token(5)
+    assert c.debug_query("staging") == 0
