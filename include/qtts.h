@@ -234,14 +234,14 @@ int qtts_gemm_q4(qtts_ctx *ctx, const qtts_w *w, const float *X, int64_t rows,
  * allocates nothing: no reference counterpart.  For callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving
  * loops).  The GEMV passes' split-K partial sums and the matrix cores' staged
- * rows use 4 MiB of device memory that the context holds (rows that do not
- * fit go in batches); a weight whose GEMV passes need more (S * 2 * npad
- * floats, S = ceil(k / 2048) for the default tile) is refused with
- * QTTS_ERR_CAPACITY.  Only enqueues on the
- * context stream (no synchronisation; qtts_sync or the stream from
- * qtts_stream orders the results; launches captured from it and replayed on
- * another stream share the context's 4 MiB with its later calls).  At most 2^20 rows per call (QTTS_ERR_CAPACITY
- * beyond).  flags: QTTS_PATH_* as for qtts_gemm_q4. */
+ * rows use 64 MiB of device memory that the context holds (rows that do not
+ * fit go in batches).  A weight whose GEMV passes need more than 4 MiB (S * 2
+ * * npad floats, S = ceil(k / 2048) for the default tile) is refused with
+ * QTTS_ERR_CAPACITY below 16 rows unless QTTS_PATH_MFMA is asked for.  Only
+ * enqueues on the context stream (no synchronisation; qtts_sync or the stream
+ * from qtts_stream orders the results; launches captured from it and replayed
+ * on another stream share the context's 64 MiB with its later calls).  At most
+ * 2^20 rows per call (QTTS_ERR_CAPACITY beyond).  flags: QTTS_PATH_* as for qtts_gemm_q4. */
 int qtts_gemm_q4_noalloc(qtts_ctx *ctx, const qtts_w *w, const float *X,
                          int64_t rows, float *Y, int flags);
 

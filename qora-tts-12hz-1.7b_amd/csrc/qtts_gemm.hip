@@ -643,27 +643,38 @@ size_t mm_swiglu_part_floats(const Q4Frag &w, int M)
     return M <= MM_SEG_ROWS ? (size_t)mm_segments(w) * M * w.ng * 32 : 0;
 }
 
+// Whether plain rows run one workgroup per (tile, K segment) and add partial
+// sums, against one long K loop a tile: a segment saved is about 2.2 us while
+// the tiles alone do not fill the CUs, the second launch costs about 10, and
+// the partial sums go out and back at about 4.2 TB/s.  Loop / segments:
+// 6144 x 2048 16 rows 50 / 16 us, 400 rows 74 / 68, 500 rows 75 / 80;
+// 2048 x 4096 64 rows 21 / 18, 100 rows 22 / 24; 1024 deep 13 / 13 at 3 rows
+// (no gain at any count).
+static bool rows_by_segment(int rows, size_t ncols, int nseg)
+{
+    return 8.0 * rows * ncols * nseg < 4.2e6 * (2.2 * (nseg - 1) - 10);
+}
+
 // Plain rows: Y[M][ldy] columns 0..ng*32-1 = (silu)(X W (+ bias)), the rows
 // split into `ws` first.  ws_floats bounds what one batch of rows may use
 // (split rows, factors, partial sums); more rows run in batches.  The sums of
 // a weight are cut into the same segments at any batch size; whether they
-// are added in registers or from partial sums does not change a bit.
+// are added in registers or from partial sums does not change a bit.  Bias and
+// SiLU are applied where partial sums are added.
 hipError_t enqueue_mm_rows(const Q4Frag &w, const float *X, int ld, int rows, const float *bias, bool silu, float *Y,
                            int ldy, float *ws, size_t ws_floats, hipStream_t s)
 {
     const size_t per_row = (size_t)w.kc * 64 + 1, ncols = (size_t)w.ng * 32;
-    const int tn = (w.ng + 3) / 4, nseg = mm_segments(w);
-    // One workgroup per (tile, K segment) and partial sums where tiles alone
-    // would leave CUs idle: 24 x 6144 x 2048 takes 38 us so (two batches that
-    // fit the workspace), 58 us as 16 long K loops; past two batches the long
-    // loops have the rows to fill the chip.  Bias and SiLU are applied where
-    // partial sums are added.
+    const int nseg = mm_segments(w);
     const size_t cap_parts = ws_floats / (per_row + (size_t)nseg * ncols);
-    const bool parts = bias || silu ||
-                       ((int64_t)((rows + 79) / 80) * tn < 192 && (size_t)rows <= 2 * (cap_parts & ~(size_t)15));
+    const bool parts = bias || silu || ((size_t)rows <= cap_parts && rows_by_segment(rows, ncols, nseg));
     size_t cap = parts ? cap_parts : ws_floats / per_row;
     if (cap < 1) return hipErrorInvalidValue;
-    if (cap >= 16) cap &= ~(size_t)15;
+    if ((size_t)rows > cap) {
+        // equal batches of whole row blocks
+        const size_t nb = (rows + cap - 1) / cap, per = ((rows + nb - 1) / nb + 15) & ~(size_t)15;
+        cap = per <= cap ? per : cap >= 16 ? cap & ~(size_t)15 : cap;
+    }
     for (int r0 = 0; r0 < rows; r0 += (int)cap) {
         const int M = (int)std::min<size_t>(cap, rows - r0);
         // split rows first (16-byte aligned), then the parts, then the factors
@@ -685,10 +696,18 @@ hipError_t enqueue_mm_rows(const Q4Frag &w, const float *X, int ld, int rows, co
     return hipSuccess;
 }
 
-// Workspace of one batch of M rows with partial sums.
+// Workspace of one batch of M rows with partial sums (bias / SiLU), and what
+// plain rows take at once, up to a bound.
 size_t mm_rows_ws_floats(const Q4Frag &w, int M)
 {
     return (size_t)M * (w.kc * 64 + 1 + (size_t)mm_segments(w) * w.ng * 32);
+}
+
+size_t mm_plain_ws_floats(const Q4Frag &w, int64_t M, size_t most)
+{
+    const size_t nseg = mm_segments(w), ncols = (size_t)w.ng * 32;
+    const size_t loop = (size_t)M * (w.kc * 64 + 1), seg = loop + (size_t)M * nseg * ncols;
+    return std::min(most, seg <= most && rows_by_segment((int)M, ncols, (int)nseg) ? seg : loop);
 }
 
 }  // namespace qtts

@@ -315,6 +315,7 @@ hipError_t enqueue_mm_swiglu(const RowsSplit &a, const Q4Frag &w, float *part, u
 hipError_t enqueue_mm_rows(const Q4Frag &w, const float *X, int ld, int rows, const float *bias, bool silu, float *Y,
                            int ldy, float *ws, size_t ws_floats, hipStream_t s);
 size_t mm_rows_ws_floats(const Q4Frag &w, int M);
+size_t mm_plain_ws_floats(const Q4Frag &w, int64_t M, size_t most);
 // The split-f16 contraction unless QTTS_GEMM_F32=1 (f32 matrix instructions).
 bool gemm_x3();
 bool gemm_supported(const Q4Tiled &w);

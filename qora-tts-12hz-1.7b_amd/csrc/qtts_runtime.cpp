@@ -131,6 +131,7 @@ struct qtts_prefix {
 // rows 9.6 / 11 / 12 us and 7.0 / 13 / 27 us.  Both are as far from 64 bits
 // (2e-7 of a product, 1.3e-7 of the prefill's hidden).
 constexpr int64_t MFMA_MIN_ROWS = 3;
+constexpr int64_t F32_MIN_ROWS = 16;
 constexpr int PREFILL_MAX_ROWS = 2048;   // rows per prefill chunk, longer prompts in equal chunks
 constexpr int TIME_PREFILL_ROWS = 1024;  // rows qtts_time_prefill takes
 constexpr size_t PIN_BYTES = (size_t)1 << 20;    // pinned staging per context
@@ -498,8 +499,12 @@ static void drop_graph(qtts_ctx *c)
 // Workspace of the allocation-free entry point (qtts_gemm_q4_noalloc): the
 // split-K partial sums of its GEMV passes, the matrix cores' split rows,
 // factors and partial sums.  One per context, allocated with it, so that
-// calls of different contexts (threads, streams) do not share it.
-constexpr size_t SCRATCH_FLOATS = (size_t)1 << 20;    // 4 MiB
+// calls of different contexts (threads, streams) do not share it.  The size
+// holds 2730 rows of 6144 columns: with 4 MiB (160 of them) 2000 rows x 6144 x
+// 2048 ran as thirteen launches of half the CUs or less and took 745 us, at
+// once 161.  The GEMV passes keep their limit of 4 MiB.
+constexpr size_t SCRATCH_FLOATS = (size_t)1 << 24;          // 64 MiB
+constexpr size_t GEMV_SCRATCH_FLOATS = (size_t)1 << 20;     // 4 MiB
 
 extern "C" int qtts_ctx_create(int device, int64_t kv_capacity, qtts_ctx **out)
 {
@@ -800,9 +805,8 @@ extern "C" int qtts_gemm_q4(qtts_ctx *c, const qtts_w *w, const float *X, int64_
     RCHK(ensure_io(c, rows * std::max({w->t.k, w->t.n, w->t.npad})));
     RCHK(stage_in(c, X, rows * w->t.k, c->d_io, flags));
     if (use_mfma(flags, rows) && gemm_supported(w->t)) {
-        // the bound of qtts_gemm_q4_noalloc's scratch, so both run the same launches
-        RCHK(ensure_mm(c, SCRATCH_FLOATS));
-        HIPCHK(c, enqueue_gemm_rows(w->t, w->f, c->d_io, (int)rows, c->d_io2, w->t.n, c->d_mm, SCRATCH_FLOATS, c->stream));
+        RCHK(ensure_mm(c, mm_plain_ws_floats(w->f, rows, SCRATCH_FLOATS)));
+        HIPCHK(c, enqueue_gemm_rows(w->t, w->f, c->d_io, (int)rows, c->d_io2, w->t.n, c->d_mm, c->mm_floats, c->stream));
     }
     else
         HIPCHK(c, enqueue_gemv_rows(w->t, c->d_io, (int)rows, c->d_io2, w->part, c->stream));
@@ -828,11 +832,12 @@ extern "C" int qtts_gemm_q4_noalloc(qtts_ctx *c, const qtts_w *w, const float *X
     const Q4Tiled &t = w->t;
     const bool mx = use_mfma(flags, rows) && gemm_supported(t);
     // a weight whose GEMV passes do not fit is refused for any few rows, not
-    // only for the one or two that take them
+    // only for the ones that take them: which do is the library's choice and
+    // moves with its kernels
     const size_t need = (size_t)t.S * 2 * t.npad;
-    if (need > SCRATCH_FLOATS && (!mx || (rows < 16 && !(flags & QTTS_PATH_MFMA))))
+    if (need > GEMV_SCRATCH_FLOATS && (!mx || (rows < F32_MIN_ROWS && !(flags & QTTS_PATH_MFMA))))
         return fail(c, QTTS_ERR_CAPACITY, "this weight's GEMV passes need %zu floats of scratch; the maximum is %zu", need,
-                    SCRATCH_FLOATS);
+                    GEMV_SCRATCH_FLOATS);
     if (mx)   // more rows than the scratch holds go in batches
         HIPCHK(c, enqueue_gemm_rows(t, w->f, X, (int)rows, Y, t.n, c->scratch, SCRATCH_FLOATS, c->stream));
     else

@@ -53,19 +53,28 @@ def test_rows_and_shapes(ctx, k, n):
     dw.free()
 
 
-@pytest.mark.parametrize("k,n,rows", [(6144, 2048, 400), (2048, 12288, 600)])
+@pytest.mark.parametrize("k,n,rows", [(6144, 2048, 450), (2048, 12288, 600), (6144, 64, 2900)])
 def test_rows_in_batches(ctx, k, n, rows):
-    """More rows than the workspace holds at once: the same bits as one by
-    one batch."""
+    """More rows than run one workgroup per K segment, and more (2900 x 6144)
+    than the workspace holds at once: the same bits as in batches of 100, with
+    and without the call's own allocations."""
     rng = np.random.Generator(np.random.PCG64(rows))
     w = synth.q4_random(rng, k, n)
     dw = ctx.upload(w)
     X = rng.standard_normal((rows, k)).astype(np.float32)
     whole = ctx.gemm(dw, X, path="mfma")
-    at = [0, 15, 159, 160, 161, rows - 1]
+    at = [0, 15, rows // 2, rows - 17, rows - 1]
     check(whole[at], X[at], w)
     for r0 in range(0, rows, 100):
         assert np.array_equal(bits(ctx.gemm(dw, X[r0:r0 + 100], path="mfma")), bits(whole[r0:r0 + 100]))
+    h = hip()
+    dx, dy = DevBuf(h, X.nbytes), DevBuf(h, whole.nbytes)
+    dx.put(X)
+    ctx.gemm_noalloc(dw, dx.ptr.value, rows, dy.ptr.value, path="mfma")
+    ctx.sync()
+    assert np.array_equal(bits(dy.get(whole.shape)), bits(whole))
+    dx.free()
+    dy.free()
     dw.free()
 
 
