@@ -239,9 +239,11 @@ int qtts_gemm_q4(qtts_ctx *ctx, const qtts_w *w, const float *X, int64_t rows,
  * * npad floats, S = ceil(k / 2048) for the default tile) is refused with
  * QTTS_ERR_CAPACITY below 16 rows unless QTTS_PATH_MFMA is asked for.  Only
  * enqueues on the context stream (no synchronisation; qtts_sync or the stream
- * from qtts_stream orders the results; launches captured from it and replayed
- * on another stream share the context's 64 MiB with its later calls).  At most
- * 2^20 rows per call (QTTS_ERR_CAPACITY beyond).  flags: QTTS_PATH_* as for qtts_gemm_q4. */
+ * from qtts_stream orders the results).  The workspace lives as long as the
+ * context: launches captured from this call into a graph may be replayed
+ * until qtts_ctx_destroy, and one replayed on another stream shares the
+ * workspace with the context's later calls.  At most 2^20 rows per call
+ * (QTTS_ERR_CAPACITY beyond).  flags: QTTS_PATH_* as for qtts_gemm_q4. */
 int qtts_gemm_q4_noalloc(qtts_ctx *ctx, const qtts_w *w, const float *X,
                          int64_t rows, float *Y, int flags);
 
