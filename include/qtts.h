@@ -40,8 +40,8 @@ extern "C" {
 #define QTTS_ERR_UNSUPPORTED -8 /* format the device path does not run     */
 
 #define QTTS_DEVICE_PTRS   1    /* flags: float buffers are device memory  */
-/* Path choice for qtts_gemm_q4 and qtts_talker_prefill (default: by row
- * count, the matrix cores from 3 rows up). */
+/* Path choice for qtts_gemm_q4 and qtts_talker_prefill (default: the faster
+ * one; the matrix cores from 16 rows up, and from 3 where they win). */
 #define QTTS_PATH_ROWWISE  2    /* flags: one GEMV pass per row            */
 #define QTTS_PATH_MFMA     4    /* flags: matrix-core GEMM at any row count */
 
@@ -225,8 +225,8 @@ int qtts_gemv_q4(qtts_ctx *ctx, const qtts_w *w, const float *x, float *y,
 
 /* Y[rows][n] = X[rows][k] * W.  Replaces `gemm` (gemv.rs:157-162) ->
  * `gemm_q4` (gemv.rs:349-412).  From 3 rows (k a multiple of 32, at least
- * 64) an f32-accurate matrix-core GEMM; fewer rows run the GEMV, two rows per pass
- * over W.  flags may force either path (QTTS_PATH_*). */
+ * 64; from 16 rows for a weight with scales of 4096 or more) an f32-accurate
+ * matrix-core GEMM; fewer rows run the GEMV, two rows per pass over W.  flags may force either path (QTTS_PATH_*). */
 int qtts_gemm_q4(qtts_ctx *ctx, const qtts_w *w, const float *X, int64_t rows,
                  float *Y, int flags);
 
@@ -314,9 +314,10 @@ int qtts_talker_decode_token(qtts_ctx *ctx, uint32_t token, int is_text,
  * start_pos..start_pos+seq-1 on top of the cached prefix:
  * `prefill_talker_raw_from` (talker.rs:379-482).  Requires
  * kv_len == start_pos.  Writes the last row's final-normed hidden.  From
- * 3 rows the layers run as batched matrix-core GEMMs (chunks of up to
- * 2048 rows); fewer rows go one by one through the decode kernels.  flags
- * may force either path (QTTS_PATH_*). */
+ * 16 rows, and from 3 unless a long cached prefix makes it the slower way,
+ * the layers run as batched matrix-core GEMMs (chunks of up to 2048 rows);
+ * fewer rows go one by one through the decode kernels.  flags may force
+ * either path (QTTS_PATH_*). */
 int qtts_talker_prefill(qtts_ctx *ctx, const float *X, int64_t seq,
                         int64_t start_pos, float *hidden_out, int flags);
 

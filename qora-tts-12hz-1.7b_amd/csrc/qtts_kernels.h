@@ -324,6 +324,7 @@ hipError_t enqueue_gemm_rows(const Q4Tiled &w, const Q4Frag &f, const float *X, 
 hipError_t enqueue_gemm_bias(const Q4Tiled &w, const Q4Frag &f, const float *X, int rows, const float *bias, bool silu,
                              float *Y, int ldy, float *ws, size_t ws_floats, hipStream_t s);
 bool prefill_supported(const TalkerDev &m);
+int prefill_split_layers(const TalkerDev &m);
 int64_t prefill_part_floats(const TalkerDev &m, int rows);
 int64_t prefill_rsc_slots(const TalkerDev &m);
 int norm_shift(const uint16_t *gamma_host, int n);

@@ -923,6 +923,13 @@ static bool split_layer(const TalkerDev &m, int l)
     return gemm_x3() && layer_has_frags(m.layers[l]);
 }
 
+int prefill_split_layers(const TalkerDev &m)
+{
+    int n = 0;
+    for (int l = 0; l < m.n_layers; l++) n += split_layer(m, l);
+    return n;
+}
+
 // Floats of partial sums the prompt's projections need at up to `rows` rows.
 int64_t prefill_part_floats(const TalkerDev &m, int rows)
 {

@@ -124,12 +124,12 @@ struct qtts_prefix {
     std::vector<int32_t> pages;
 };
 
-// Prompts at least this long take the matrix-core prefill; shorter ones run
-// row by row through the decode kernels.  Same for qtts_gemm_q4 rows.  The
-// 28-layer prefill of 2 / 3 / 10 rows takes 1.51 / 1.5 / 1.56 ms on the
-// matrix cores and 1.3 / 1.9 / 6.4 ms row by row; 2048 x 4096 over 2 / 3 / 8
-// rows 9.6 / 11 / 12 us and 7.0 / 13 / 27 us.  Both are as far from 64 bits
-// (2e-7 of a product, 1.3e-7 of the prefill's hidden).
+// Rows from which a GEMM runs on the matrix cores instead of row by row: 2048
+// x 4096 over 2 / 3 / 8 rows 9.6 / 11 / 12 us there and 7.0 / 13 / 27 us row by
+// row.  Both are as far from 64 bits (2e-7 of a product).  On the f32
+// instructions (a weight without a split copy, QTTS_GEMM_F32=1) the GEMV passes
+// are faster to 15 rows: 2048 x 4096 over 3 / 15 rows 62 / 62 us there, 23 / 62
+// row by row, 6144 x 2048 160 / 160 and 24 / 65.
 constexpr int64_t MFMA_MIN_ROWS = 3;
 constexpr int64_t F32_MIN_ROWS = 16;
 constexpr int PREFILL_MAX_ROWS = 2048;   // rows per prefill chunk, longer prompts in equal chunks
@@ -656,10 +656,29 @@ static int ensure_prefill(qtts_ctx *c, int rows)
     return QTTS_OK;
 }
 
-static bool use_mfma(int flags, int64_t rows)
+static bool gemm_mfma(const qtts_w *w, int flags, int64_t rows)
 {
-    if (flags & QTTS_PATH_ROWWISE) return false;
-    return (flags & QTTS_PATH_MFMA) || rows >= MFMA_MIN_ROWS;
+    if (!gemm_supported(w->t) || (flags & QTTS_PATH_ROWWISE)) return false;
+    return (flags & QTTS_PATH_MFMA) || rows >= (gemm_x3() && w->f.data ? MFMA_MIN_ROWS : F32_MIN_ROWS);
+}
+
+// Whether a prompt of `rows` rows on `start` cached positions runs on the
+// matrix cores.  A layer costs 22.4 us a row through the decode kernels plus
+// 1.5 ns a cached position; on the matrix cores 50 us (155 on the f32
+// instructions) for up to 15 rows, plus 32 ns a cached position, which few
+// workgroups read one after the other.  28 layers, ms, row by row / matrix
+// cores: 3 rows on 0 / 500 / 1000 / 2000 positions 1.94 / 1.37, 1.94 / 1.82,
+// 1.96 / 2.29, 2.01 / 3.22; 4 and 5 rows on 2000 2.65 / 3.23 and 3.31 / 3.23; 6 and
+// 7 rows on 4000 4.61 / 5.03 and 5.38 / 5.03; 8 rows on 8000 7.63 / 8.69; all
+// layers on the f32 instructions, 6 and 8 rows on 0 3.82 / 4.34 and 5.08 / 4.35.
+static bool prompt_mfma(const TalkerDev &m, int flags, int64_t rows, int64_t start)
+{
+    if (!prefill_supported(m) || (flags & QTTS_PATH_ROWWISE)) return false;
+    if ((flags & QTTS_PATH_MFMA) || rows >= F32_MIN_ROWS) return true;
+    if (rows < MFMA_MIN_ROWS) return false;
+    const double split = prefill_split_layers(m), f32 = m.n_layers - split;
+    const double one = rows * (22.4 + 0.0015 * start) * m.n_layers;
+    return one > 50 * split + 155 * f32 + 0.032 * start * m.n_layers;
 }
 
 // A slot of the pinned staging buffer, or null (full, or too large for it).
@@ -804,7 +823,7 @@ extern "C" int qtts_gemm_q4(qtts_ctx *c, const qtts_w *w, const float *X, int64_
     if (rows == 0) return QTTS_OK;
     RCHK(ensure_io(c, rows * std::max({w->t.k, w->t.n, w->t.npad})));
     RCHK(stage_in(c, X, rows * w->t.k, c->d_io, flags));
-    if (use_mfma(flags, rows) && gemm_supported(w->t)) {
+    if (gemm_mfma(w, flags, rows)) {
         RCHK(ensure_mm(c, mm_plain_ws_floats(w->f, rows, SCRATCH_FLOATS)));
         HIPCHK(c, enqueue_gemm_rows(w->t, w->f, c->d_io, (int)rows, c->d_io2, w->t.n, c->d_mm, c->mm_floats, c->stream));
     }
@@ -830,7 +849,7 @@ extern "C" int qtts_gemm_q4_noalloc(qtts_ctx *c, const qtts_w *w, const float *X
     if (rows > (1 << 20)) return fail(c, QTTS_ERR_CAPACITY, "at most %d rows", 1 << 20);
     hipSetDevice(c->device);
     const Q4Tiled &t = w->t;
-    const bool mx = use_mfma(flags, rows) && gemm_supported(t);
+    const bool mx = gemm_mfma(w, flags, rows);
     // a weight whose GEMV passes do not fit is refused for any few rows, not
     // only for the ones that take them: which do is the library's choice and
     // moves with its kernels
@@ -1315,7 +1334,7 @@ extern "C" int qtts_talker_prefill(qtts_ctx *c, const float *X, int64_t seq, int
     RCHK(seq_unshare_from(c, start_pos));
     c->gen_started = false;
     const int H = c->tm.hidden;
-    if (use_mfma(flags, seq) && prefill_supported(c->tm)) {
+    if (prompt_mfma(c->tm, flags, seq, start_pos)) {
         // equal chunks: 1024 + 85 rows took as long as 1400 in one
         const int64_t nch = (seq + PREFILL_MAX_ROWS - 1) / PREFILL_MAX_ROWS, per = (seq + nch - 1) / nch;
         RCHK(ensure_prefill(c, (int)per));

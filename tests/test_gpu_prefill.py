@@ -216,6 +216,51 @@ def test_prefill_fallback_paths(loaded, env, monkeypatch):
     om.kv_reset()
 
 
+@pytest.mark.parametrize("start,rows,path", [(40, 3, "mfma"), (2000, 3, "rowwise"), (2000, 4, "rowwise"),
+                                             (2000, 9, "mfma"), (2040, 15, "mfma"), (2040, 2, "rowwise")])
+def test_short_suffix_on_a_prefix(ctx_factory, start, rows, path):
+    """3 to 15 rows behind a cached prefix: the path that is faster there (the
+    bits of the one expected), against the oracle."""
+    t = synth.make_talker(seed=415, n_layers=2, text_vocab=256, rope_max_pos=2304)
+    p = synth.make_predictor(seed=416, n_layers=1)
+    c = ctx_factory(2304)
+    c.upload_model(t, p)
+    om = O.Model(t, p, kv_cap=2304)
+    rng = np.random.Generator(np.random.PCG64(2510 + start + rows))
+    K, V = rng.standard_normal((2, 2, start, 8, 128)).astype(np.float32)
+    X = rng.standard_normal((rows, t.hidden)).astype(np.float32)
+    om.kv_load(K, V)
+    ref = om.prefill(X, start)
+    out = []
+    for q in (None, path):
+        c.kv_load(K, V)
+        out.append(c.prefill_talker_raw_from(X, start, path=q))
+    assert np.array_equal(out[0].view(np.uint32), out[1].view(np.uint32)), "not the path expected"
+    ok, e = close(out[0], ref)
+    assert ok, f"rel err {e}"
+    check_kv(c, om, 2, start + rows)
+    om.close()
+    c.close()
+
+
+@pytest.mark.parametrize("rows,path", [(3, "rowwise"), (15, "rowwise"), (16, "mfma")])
+def test_few_rows_without_a_split_copy(ctx_factory, rows, path):
+    """A weight outside the split's range (a scale of 5000): fewer than 16 rows
+    run row by row, as the f32 instructions are the slower way there."""
+    c = ctx_factory(256)
+    rng = np.random.Generator(np.random.PCG64(2530 + rows))
+    w = synth.q4_random(rng, 2048, 1024)
+    w.scales[5, 2] = np.array(5000.0, np.float16).view(np.uint16)
+    dw = c.upload(w)
+    X = rng.standard_normal((rows, 2048)).astype(np.float32)
+    Y = c.gemm(dw, X)
+    assert np.array_equal(Y.view(np.uint32), c.gemm(dw, X, path=path).view(np.uint32))
+    R = O.gemm(X, w)
+    for r in range(rows):
+        assert close(Y[r], R[r])[0]
+    dw.free()
+
+
 def test_prefill_chunked(ctx_factory):
     """More rows than one prefill chunk (1024): the second chunk attends to
     the first through the cache."""
