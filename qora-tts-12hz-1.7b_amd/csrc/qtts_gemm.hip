@@ -112,55 +112,36 @@ k_frag_build(Q4Tiled w, Q4Frag f, uint8_t *out)
 // 32 lo halves, then the same for the next 32 columns.
 // ---------------------------------------------------------------------------
 
-// Rows of f32 into split rows, staged times a power of two from the largest
-// |x| of the row (seg = 0) or of each 256 columns (seg = 1): the factors that
-// undo it go to rsc[m] or rsc[s * ldr + m].  One workgroup per row.
+// Rows of f32 into split rows, each 256 columns (a K segment) staged times the
+// power of two from their largest |x|: small values keep their bits beside an
+// outlier elsewhere in the row.  The factors that undo it go to rsc[s * ldr +
+// m].  One workgroup per row.
 __global__ void __launch_bounds__(256)
-k_split_rows(const float *X, int ld, int K, int seg, uint8_t *out, int kc, float *rsc, int ldr)
+k_split_rows(const float *X, int ld, int K, uint8_t *out, int kc, float *rsc, int ldr)
 {
-    __shared__ float red[4];
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6, m = blockIdx.x;
     const float *x = X + (size_t)m * ld;
     uint8_t *o = out + (size_t)m * kc * 256;
     // four columns a lane, so a wave covers 256 (a caller's rows need not be
     // 16-byte aligned)
     typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
-    const auto emit = [&](int k, f32x4 v, float p2) {
-        uint32_t h0, l0, h1, l1;
-        split_f16_pair<true>(v.x * p2, v.y * p2, h0, l0);
-        split_f16_pair<true>(v.z * p2, v.w * p2, h1, l1);
-        uint8_t *p = o + (k >> 5) * 128 + (k & 31) * 2;
-        *(uint2 *)p = uint2{h0, h1};
-        *(uint2 *)(p + 64) = uint2{l0, l1};
-    };
-    if (seg) {
-        for (int k0 = 256 * wv; k0 < 64 * kc; k0 += 1024) {
-            const int k = k0 + 4 * lane;
-            f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
-            if (k < K) v = *(const f32x4u *)(x + k);
-            const float mx = wave_max_dpp(fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
-            const int sh = range_shift(mx);
-            if (k < 64 * kc) emit(k, v, __builtin_ldexpf(1.0f, sh));
-            if (lane == 0) rsc[(size_t)(k0 >> 8) * ldr + m] = __builtin_ldexpf(1.0f, -sh);
-        }
-        return;
-    }
-    float mx = 0.0f;
-    for (int k = 4 * t; k < K; k += 1024) {
-        const f32x4 v = *(const f32x4u *)(x + k);
-        mx = fmaxf(mx, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
-    }
-    mx = wave_max_dpp(mx);
-    if (lane == 0) red[wv] = mx;
-    __syncthreads();
-    const int sh = range_shift(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
-    const float p2 = __builtin_ldexpf(1.0f, sh);
-    for (int k = 4 * t; k < 64 * kc; k += 1024) {
+    for (int k0 = 256 * wv; k0 < 64 * kc; k0 += 1024) {
+        const int k = k0 + 4 * lane;
         f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
         if (k < K) v = *(const f32x4u *)(x + k);
-        emit(k, v, p2);
+        const float mx = wave_max_dpp(fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+        const int sh = range_shift(mx);
+        const float p2 = __builtin_ldexpf(1.0f, sh);
+        if (k < 64 * kc) {
+            uint32_t h0, l0, h1, l1;
+            split_f16_pair<true>(v.x * p2, v.y * p2, h0, l0);
+            split_f16_pair<true>(v.z * p2, v.w * p2, h1, l1);
+            uint8_t *p = o + (k >> 5) * 128 + (k & 31) * 2;
+            *(uint2 *)p = uint2{h0, h1};
+            *(uint2 *)(p + 64) = uint2{l0, l1};
+        }
+        if (lane == 0) rsc[(size_t)(k0 >> 8) * ldr + m] = __builtin_ldexpf(1.0f, -sh);
     }
-    if (t == 0) rsc[m] = __builtin_ldexpf(1.0f, -sh);
 }
 
 // ---------------------------------------------------------------------------
@@ -569,10 +550,10 @@ static hipError_t launch_mm(const RowsSplit &a, const Q4Frag &w, const MmOut &o,
     return hipGetLastError();
 }
 
-hipError_t enqueue_split_rows(const float *X, int ld, int M, int K, int seg, uint8_t *out, int kc, float *rsc,
-                              int ldr, hipStream_t s)
+hipError_t enqueue_split_rows(const float *X, int ld, int M, int K, uint8_t *out, int kc, float *rsc, int ldr,
+                              hipStream_t s)
 {
-    hipLaunchKernelGGL(k_split_rows, dim3(M), dim3(256), 0, s, X, ld, K, seg, out, kc, rsc, ldr);
+    hipLaunchKernelGGL(k_split_rows, dim3(M), dim3(256), 0, s, X, ld, K, out, kc, rsc, ldr);
     return hipGetLastError();
 }
 
@@ -664,8 +645,8 @@ static bool rows_by_segment(int rows, size_t ncols, int nseg)
 hipError_t enqueue_mm_rows(const Q4Frag &w, const float *X, int ld, int rows, const float *bias, bool silu, float *Y,
                            int ldy, float *ws, size_t ws_floats, hipStream_t s)
 {
-    const size_t per_row = (size_t)w.kc * 64 + 1, ncols = (size_t)w.ng * 32;
     const int nseg = mm_segments(w);
+    const size_t per_row = (size_t)w.kc * 64 + nseg, ncols = (size_t)w.ng * 32;
     const size_t cap_parts = ws_floats / (per_row + (size_t)nseg * ncols);
     const bool parts = bias || silu || ((size_t)rows <= cap_parts && rows_by_segment(rows, ncols, nseg));
     size_t cap = parts ? cap_parts : ws_floats / per_row;
@@ -681,8 +662,8 @@ hipError_t enqueue_mm_rows(const Q4Frag &w, const float *X, int ld, int rows, co
         uint8_t *sp = (uint8_t *)ws;
         float *part = ws + (size_t)M * w.kc * 64;
         float *rsc = part + (parts ? (size_t)nseg * M * ncols : 0);
-        GCHK(enqueue_split_rows(X + (size_t)r0 * ld, ld, M, w.k, 0, sp, w.kc, rsc, 0, s));
-        const RowsSplit a{sp, w.kc, M, rsc, 0, 1.0f};
+        GCHK(enqueue_split_rows(X + (size_t)r0 * ld, ld, M, w.k, sp, w.kc, rsc, M, s));
+        const RowsSplit a{sp, w.kc, M, rsc, M, 1.0f};
         float *y = Y + (size_t)r0 * ldy;
         if (parts) {
             MmParts p{part, (int)ncols, (size_t)M * ncols, nseg, nseg};
@@ -700,13 +681,13 @@ hipError_t enqueue_mm_rows(const Q4Frag &w, const float *X, int ld, int rows, co
 // plain rows take at once, up to a bound.
 size_t mm_rows_ws_floats(const Q4Frag &w, int M)
 {
-    return (size_t)M * (w.kc * 64 + 1 + (size_t)mm_segments(w) * w.ng * 32);
+    return (size_t)M * (w.kc * 64 + mm_segments(w) * (1 + (size_t)w.ng * 32));
 }
 
 size_t mm_plain_ws_floats(const Q4Frag &w, int64_t M, size_t most)
 {
     const size_t nseg = mm_segments(w), ncols = (size_t)w.ng * 32;
-    const size_t loop = (size_t)M * (w.kc * 64 + 1), seg = loop + (size_t)M * nseg * ncols;
+    const size_t loop = (size_t)M * (w.kc * 64 + nseg), seg = loop + (size_t)M * nseg * ncols;
     return std::min(most, seg <= most && rows_by_segment((int)M, ncols, (int)nseg) ? seg : loop);
 }
 

@@ -41,8 +41,8 @@ struct Q4Frag {
 };
 
 // GEMM rows split into f16 hi + lo (layout in qtts_gemm.hip), and what undoes
-// their staging: a factor per row (rseg 0), per row and 256 or 64 columns
-// (rseg floats between the column slots), or one for all (rsc null).
+// their staging: a factor per row and 256 or 64 columns (rseg floats between
+// the column slots), or one for all (rsc null).
 struct RowsSplit {
     const uint8_t *p;
     int32_t kc, M;
@@ -305,8 +305,8 @@ hipError_t enqueue_pred_qkv_tables(const PredictorDev &p, int n_tables, float *p
 bool frag_supported(const Q4Tiled &w);
 size_t frag_shape(const Q4Tiled &w, Q4Frag *f);
 hipError_t enqueue_frag_build(const Q4Tiled &w, const Q4Frag &f, uint8_t *out, hipStream_t s);
-hipError_t enqueue_split_rows(const float *X, int ld, int M, int K, int seg, uint8_t *out, int kc, float *rsc,
-                              int ldr, hipStream_t s);
+hipError_t enqueue_split_rows(const float *X, int ld, int M, int K, uint8_t *out, int kc, float *rsc, int ldr,
+                              hipStream_t s);
 size_t mm_part_floats(const Q4Frag &w, int M);
 size_t mm_swiglu_part_floats(const Q4Frag &w, int M);
 hipError_t enqueue_mm_parts(const RowsSplit &a, const Q4Frag &w, bool fp1, float *part, MmParts *p, hipStream_t s);

@@ -834,7 +834,7 @@ bool gemm_supported(const Q4Tiled &w)
 hipError_t enqueue_gemm_rows(const Q4Tiled &w, const Q4Frag &f, const float *X, int rows, float *Y, int ldy, float *ws,
                              size_t ws_floats, hipStream_t s)
 {
-    if (gemm_x3() && f.data && ws_floats >= (size_t)f.kc * 64 + 1)
+    if (gemm_x3() && f.data && ws_floats >= (size_t)f.kc * 64 + (f.kc + 3) / 4)
         return enqueue_mm_rows(f, X, w.k, rows, nullptr, false, Y, ldy, ws, ws_floats, s);
     return launch_gemm<GEMM_STORE>(GemmA{X, w.k, nullptr, nullptr, rows}, w,
                                    GemmOut{Y, ldy, std::min(ldy, w.G * 32), nullptr, 0}, 1, s);
@@ -1050,7 +1050,7 @@ hipError_t enqueue_talker_prefill(const TalkerDev &m, const PrefillWs &pw, int M
             hipLaunchKernelGGL(k_prefill_attn<PREFILL_ATTN_QB>, dim3((M + PREFILL_ATTN_QB - 1) / PREFILL_ATTN_QB, 8),
                                dim3(256), 0, s, pw.q, A, M, start, m.kv, l, out, A);
             PCHK(hipGetLastError());
-            if (sp) PCHK(enqueue_split_rows(out, A, M, A, 1, as, A / 64, pw.rsc, M, s));
+            if (sp) PCHK(enqueue_split_rows(out, A, M, A, as, A / 64, pw.rsc, M, s));
         }
         // o-proj, residual, post-attention norm
         if (sp)

@@ -1,14 +1,15 @@
 """The split-f16 Q4 GEMM (k_q4_gemm and the kernels around it) at the sizes
-where its tiles end: row blocks of 16, row tiles of up to 96, the rows where
+where its tiles end: row blocks of 16, row tiles of up to 80, the rows where
 the K runs change, half chunks of 64 rows of K, K segments of 256, partial
 column tiles, widths that leave stores unaligned.
 
-Each element is held to its own bound against 64 bits.  Every staged value is
-within 2^-22 of the f32 it stands for (hi + lo, and lo lo dropped), and an
-element is at most 24 accumulations a segment (8 chunks of 32, three
-products) plus one per segment, each rounded to f32: |error| <= 2 (2^-22 +
-(24 + segments) 2^-24) sum_k |x_k w_k|, the factor 2 for the sums inside one
-matrix instruction.
+Each element is held to its own bound against 64 bits.  A staged value is
+within 2^-22 of the f32 it stands for (hi + lo, and lo lo dropped) plus 2^-39
+of the largest of its row's 256 columns (lo's subnormal step), and an element
+is at most 24 accumulations a segment (8 chunks of 32, three products) plus
+one per segment, each rounded to f32: |error| <= 2 (2^-22 + (24 + segments)
+2^-24) sum_k |x_k w_k| + sum over segments 2^-39 max |x| sum_k |w_k|, the
+factor 2 for the sums inside one matrix instruction.
 """
 import numpy as np
 import pytest
@@ -32,6 +33,8 @@ def bits(a):
 def check(Y, X, w):
     W, X = w.dequant().astype(np.float64), X.astype(np.float64)
     bound = 2 * (2.0 ** -22 + (24 + -(-w.k // 256)) * 2.0 ** -24) * (np.abs(X) @ np.abs(W))
+    for k in range(0, w.k, 256):
+        bound += 2.0 ** -39 * np.abs(X[:, k:k + 256]).max(axis=1)[:, None] * np.abs(W[k:k + 256]).sum(axis=0)
     err = np.abs(Y.astype(np.float64) - X @ W)
     assert (err <= bound).all(), f"largest error {np.max(err / np.maximum(bound, 1e-300)):.3g} of its bound"
 
@@ -75,6 +78,20 @@ def test_rows_in_batches(ctx, k, n, rows):
     assert np.array_equal(bits(dy.get(whole.shape)), bits(whole))
     dx.free()
     dy.free()
+    dw.free()
+
+
+@pytest.mark.parametrize("rows", [5, 200])
+def test_small_values_beside_an_outlier(ctx, rows):
+    """A segment of 256 columns 2^30 times the others, with zero weights: the
+    others keep their bits (each segment has its own factor)."""
+    rng = np.random.Generator(np.random.PCG64(81))
+    w = synth.q4_random(rng, 1024, 96)
+    w.packed[256:512] = 0x88                      # nibbles of 8: zero
+    X = rng.standard_normal((rows, 1024)).astype(np.float32)
+    X[:, 256:512] *= np.float32(2.0 ** 30)
+    dw = ctx.upload(w)
+    check(ctx.gemm(dw, X), X, w)
     dw.free()
 
 
