@@ -60,7 +60,7 @@ struct qtts_ctx {
     float *leg_buf = nullptr;                        // side row + logits
     int *d_status = nullptr;
     int64_t lkv_len = 0;
-    // small host arguments and results go through pinned memory that a copy
+    // host arguments and results go through pinned memory that a copy
     // kernel reads and writes on the context stream (stage_in, finish)
     uint8_t *h_pin = nullptr;                        // PIN_BYTES
     size_t pin_top = 0;                              // taken since the last synchronisation
@@ -134,8 +134,12 @@ constexpr int64_t MFMA_MIN_ROWS = 3;
 constexpr int64_t F32_MIN_ROWS = 16;
 constexpr int PREFILL_MAX_ROWS = 2048;   // rows per prefill chunk, longer prompts in equal chunks
 constexpr int TIME_PREFILL_ROWS = 1024;  // rows qtts_time_prefill takes
-constexpr size_t PIN_BYTES = (size_t)1 << 20;    // pinned staging per context
-constexpr size_t PIN_MAX = (size_t)128 << 10;    // larger arguments are copied by the runtime
+// Pinned staging per context; what does not fit is copied by the runtime.  It
+// takes whole prompts (1,100 rows are 9 MB) and an utterance's samples: the
+// runtime sets up a copy engine for a stream's first large result, about 6 ms
+// of a process's first prompt (400 rows built and prefilled: 17.0 ms with 128
+// KB staged at most, 10.6 so; later ones 6.3 and 6.2).
+constexpr size_t PIN_BYTES = (size_t)16 << 20;
 constexpr size_t ARENA_BYTES = (size_t)64 << 20;
 constexpr int TEXT_BATCH_ROWS = 256;     // text rows whose partial sums are held at once
 
@@ -681,18 +685,19 @@ static bool prompt_mfma(const TalkerDev &m, int flags, int64_t rows, int64_t sta
     return one > 50 * split + 155 * f32 + 0.032 * start * m.n_layers;
 }
 
-// A slot of the pinned staging buffer, or null (full, or too large for it).
+// A slot of the pinned staging buffer, or null (it does not fit).
 static uint8_t *pin_take(qtts_ctx *c, size_t bytes)
 {
-    if (bytes > PIN_MAX || c->pin_top + bytes > PIN_BYTES) return nullptr;
+    if (c->pin_top + bytes > PIN_BYTES) return nullptr;
     uint8_t *p = c->h_pin + c->pin_top;
     c->pin_top += (bytes + 255) & ~(size_t)255;
     return p;
 }
 
-// Copy n floats in (host or device source) to a device buffer.  A small host
-// array goes through pinned memory and a copy kernel: 3 us on the stream and
-// no wait on the host, where a copy of pageable memory blocks it for about 8.
+// Copy n floats in (host or device source) to a device buffer.  A host array
+// goes through pinned memory and a copy kernel: 3 us on the stream and no wait
+// on the host, where a copy of pageable memory blocks it for about 8 (small
+// ones; 3 MB take 0.3 ms either way).
 static int stage_in(qtts_ctx *c, const float *src, int64_t n, float *dst, int flags)
 {
     const size_t bytes = (size_t)n * sizeof(float);
@@ -713,8 +718,8 @@ static int stage_ids(qtts_ctx *c, const uint32_t *src, int64_t n, uint32_t *dst)
     return stage_in(c, (const float *)src, n, (float *)dst, 0);
 }
 
-// n floats of a result to the caller's buffer.  A small host result is handed
-// over by the next finish(): src keeps its value until then.
+// n floats of a result to the caller's buffer.  A host result is handed over
+// by the next finish(): src keeps its value until then.
 static int stage_out(qtts_ctx *c, const float *src, int64_t n, float *dst, int flags)
 {
     if (!dst) return QTTS_OK;

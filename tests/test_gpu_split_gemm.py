@@ -160,3 +160,25 @@ def test_weight_uploaded_behind_queued_work(ctx_factory):
         dx.free()
         dy.free()
         d0.free()
+
+
+@pytest.mark.parametrize("rows", [1000, 1022, 1023, 1040])
+def test_host_arrays_around_the_staging_buffer(ctx, rows):
+    """Host rows of 0.25 MB and results of 16 MB, which fill the 16 MiB
+    staging buffer to within a slot, and more than it holds: the bits of the
+    call on device memory."""
+    rng = np.random.Generator(np.random.PCG64(82))
+    w = synth.q4_random(rng, 64, 4032)
+    X = rng.standard_normal((rows, 64)).astype(np.float32)
+    dw = ctx.upload(w)
+    h = hip()
+    dx, dy = DevBuf(h, X.nbytes), DevBuf(h, rows * 4032 * 4)
+    dx.put(X)
+    ctx.gemm_noalloc(dw, dx.ptr.value, rows, dy.ptr.value)
+    ctx.sync()
+    for _ in range(2):
+        assert np.array_equal(bits(ctx.gemm(dw, X)), bits(dy.get((rows, 4032))))
+        assert ctx.debug_query("staging") == 0
+    dx.free()
+    dy.free()
+    dw.free()
