@@ -1609,8 +1609,8 @@ static int text_rows(qtts_ctx *c, const uint32_t *d_ids, int n, float *out, floa
     return QTTS_OK;
 }
 
-// Device scratch for one prompt call, given back on every exit: from the context's arena, last in first out, or allocated
-// where it does not fit.
+// Device scratch for one prompt call, given back on every exit: from the
+// context's arena, last in first out, or allocated where it does not fit.
 struct DevScratch {
     void *p = nullptr;
     qtts_ctx *from = nullptr;
@@ -1625,8 +1625,12 @@ struct DevScratch {
 
 static int dev_scratch(qtts_ctx *c, DevScratch *b, size_t bytes)
 {
-    if (!c->arena) HIPCHK(c, hipMalloc(&c->arena, ARENA_BYTES));
-    if (c->arena_top + bytes <= ARENA_BYTES) {
+    // without room for the arena a call still gets the bytes it needs
+    if (!c->arena && hipMalloc(&c->arena, ARENA_BYTES) != hipSuccess) {
+        (void)hipGetLastError();
+        c->arena = nullptr;
+    }
+    if (c->arena && c->arena_top + bytes <= ARENA_BYTES) {
         b->p = c->arena + c->arena_top;
         b->from = c;
         b->top = c->arena_top;
