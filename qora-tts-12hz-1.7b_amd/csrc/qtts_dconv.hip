@@ -109,7 +109,7 @@ struct DcOut {
     const float *bias, *un;  // [M]; un: [phase][M]
     const float *snake;      // [2][M] e^alpha, e^-beta
     int M, os;               // channels; output row of (position n, phase ph): n os + ph
-    int32_t *flag;
+    float *rm;               // range check: a word a wave (range_note)
 };
 
 struct DcGeo {
@@ -123,12 +123,35 @@ struct DcFuse {
     DcOut o;
 };
 
-__device__ __forceinline__ float dc_snake(float v, float ea, float eb) { return v + eb * snake_sin2(ea * v); }
+// The split holds a value as f16 hi + lo: f32-accurate below the f16 maximum
+// and, through lo, to 2^-25 absolute.  So every wave that stores split rows
+// notes its largest |value| (a plain store: atomics on words of several waves
+// lengthened each launch by 2 us), and k_range_result judges them behind the
+// decode, over all channels of 64 positions (16 before a stride): a group that
+// reaches the maximum, or lies wholly below the normal f16 but is not zero, is
+// out, and the host repeats the decode on the f32 matrix path.  Quiet channels
+// beside loud ones of the same positions lose nothing that shows in the sums
+// over them.
+__global__ void __launch_bounds__(256)
+k_range_result(const int32_t *flag, RangeList l, int32_t *out)
+{
+    const RangeSignal g = l.s[blockIdx.y];
+    // 2^b lanes a group of `per` words
+    const int lane = threadIdx.x & 63, wv = blockIdx.x * 4 + (threadIdx.x >> 6), nw = gridDim.x * 4;
+    const int b = g.per >= 64 ? 6 : 32 - __clz(g.per - 1), lg = lane >> b, ll = lane & ((1 << b) - 1);
+    const uint32_t groups = (g.words + g.per - 1) / g.per;
+    bool bad = *flag != 0;
+    for (uint32_t g0 = (uint32_t)wv << (6 - b); g0 < groups; g0 += (uint32_t)nw << (6 - b)) {
+        const uint32_t w0 = (g0 + lg) * g.per;
+        float m = 0.0f;
+        for (uint32_t i = ll; i < g.per && w0 + i < g.words; i += 1u << b) m = fmaxf(m, g.p[w0 + i]);
+        for (int x = (1 << b) >> 1; x; x >>= 1) m = fmaxf(m, __shfl_xor(m, x));
+        bad |= !(m < 65504.0f) || (m > 0.0f && m < 0x1p-14f);
+    }
+    if (bad) *out = 1;
+}
 
-// out of the split's range: a value at the f16 maximum or above, or a tile
-// whose every value is below the normal f16 but not all zero (as lo alone
-// would carry it); NaN compares as out
-__device__ __forceinline__ bool dc_out_of_range(float mx) { return !(mx < 65504.0f) || (mx > 0.0f && mx < 0x1p-14f); }
+__device__ __forceinline__ float dc_snake(float v, float ea, float eb) { return v + eb * snake_sin2(ea * v); }
 
 // eight outputs of one position (two blocks' channels 4q..+3, record rec)
 __device__ __forceinline__ void dc_store8(const DcOut &o, size_t row, int rec, int q, const f32x4 &a, const f32x4 &b)
@@ -337,16 +360,12 @@ k_dconv(DcIn in, const uint8_t *wts, DcOut o, DcGeo g, DcFuse fz)
         }
         return;
     }
-    float *red = (float *)lds_all;                      // the loop ended with a barrier
-    const auto flag = [&](float mx) {
-        mx = wave_max_dpp(mx);
-        if (lane == 0) red[wv] = mx;
-        __syncthreads();
-        if (t == 0 && dc_out_of_range(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])))) *o.flag = 1;
-    };
+    const int n16 = n0 / 16 + PE * wv;               // for the range check's words
     if constexpr (EPI == DC_RAW) {
     } else if constexpr (!FUSE) {
-        float mx = 0.0f;
+        float mx[PE];
+#pragma unroll
+        for (int p = 0; p < PE; p++) mx[p] = 0.0f;
 #pragma unroll
         for (int b = 0; b < CB; b += 2) {
             const int ch = ct * 16 * CB + 16 * b + 4 * q;
@@ -376,12 +395,19 @@ k_dconv(DcIn in, const uint8_t *wts, DcOut o, DcGeo g, DcFuse fz)
                 for (int j = 0; j < 2; j++) {
                     y[j] = dc_epi<EPI>(o, acc[p][b + j], un[j], bi[j], ea[j], eb[j], ext[p][j],
                                        EPI == DC_X_SNAKE ? o.x + row * o.M + ch + 16 * j : nullptr);
-                    mx = max4(mx, y[j]);
+                    mx[p] = max4(mx[p], y[j]);
                 }
                 dc_store8(o, row, (ct * CB + b) / 2, q, y[0], y[1]);
             }
         }
-        if (o.ys) flag(mx);
+        if (o.ys && o.os > 1) {
+#pragma unroll
+            for (int p = 0; p < PE; p++) range_note(o.rm + ((size_t)(n16 + p) * g.tm + ct) * g.nph + ph, mx[p], lane);
+        } else if (o.ys) {
+#pragma unroll
+            for (int p = 1; p < PE; p++) mx[0] = fmaxf(mx[0], mx[p]);
+            range_note(o.rm + (size_t)(n16 / PE) * g.tm + ct, mx[0], lane);
+        }
     } else {
         // conv1's snake stays in registers as conv2's operand (the 16 CB
         // channels are all of conv2's input); the same values, products and
@@ -422,7 +448,7 @@ k_dconv(DcIn in, const uint8_t *wts, DcOut o, DcGeo g, DcFuse fz)
                 tl[p][b / 2] = __builtin_bit_cast(half8, uint4{l[0], l[1], l[2], l[3]});
             }
         }
-        flag(mx);
+        range_note(o.rm + n16 / PE, mx, lane);
         float mx2 = 0.0f;
 #pragma unroll
         for (int b = 0; b < CB; b += 2) {
@@ -468,10 +494,7 @@ k_dconv(DcIn in, const uint8_t *wts, DcOut o, DcGeo g, DcFuse fz)
                 dc_store8(o2, n, b / 2, q, y[0], y[1]);
             }
         }
-        if (o2.ys) {
-            __syncthreads();                         // red is read by the first check
-            flag(mx2);
-        }
+        if (o2.ys) range_note(o2.rm + n16 / PE, mx2, lane);
     }
 }
 
@@ -481,7 +504,6 @@ template <int EPI>
 __global__ void __launch_bounds__(256)
 k_dconv_reduce(const float *part, int ks, int64_t rows, int nph, DcOut o)
 {
-    __shared__ float red[4];
     const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x, n8 = o.M / 8;
     float mx = 0.0f;
     if (id < rows * n8) {
@@ -501,11 +523,7 @@ k_dconv_reduce(const float *part, int ks, int64_t rows, int nph, DcOut o)
         }
         dc_store8(o, row, rec, q, y[0], y[1]);
     }
-    if (!o.ys) return;
-    mx = wave_max_dpp(mx);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
-    __syncthreads();
-    if (threadIdx.x == 0 && dc_out_of_range(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])))) *o.flag = 1;
+    if (o.ys) range_note(o.rm + (id >> 6), mx, threadIdx.x & 63);
 }
 
 // ---------------------------------------------------------------------------
@@ -592,9 +610,8 @@ k_lin_cf(LinSum p, float *y)
 // silu(gate) up of interleaved rows (gate 2j, up 2j + 1) into split rows
 template <int KS>
 __global__ void __launch_bounds__(256)
-k_lin_swiglu(LinSum p, uint8_t *ys, int32_t *flag)
+k_lin_swiglu(LinSum p, uint8_t *ys, float *rm)
 {
-    __shared__ float red[4];
     const int C = p.M / 2, n8 = C / 8;
     const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
     float mx = 0.0f;
@@ -609,19 +626,15 @@ k_lin_swiglu(LinSum p, uint8_t *ys, int32_t *flag)
         }
         split_store8(ys, row, C, rec, q, y[0], y[1]);
     }
-    mx = wave_max_dpp(mx);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
-    __syncthreads();
-    if (threadIdx.x == 0 && dc_out_of_range(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])))) *flag = 1;
+    range_note(rm + (id >> 6), mx, threadIdx.x & 63);
 }
 
 // x (+)= scale * sum, then RMSNorm (eps 1e-5) into split rows; one wave a
 // row of at most 512 NV channels, in registers.  scale null: x = sum.
 template <int NV, int KS>
 __global__ void __launch_bounds__(256)
-k_lin_resid_rms(LinSum p, const float *scale, float *x, const float *gamma, uint8_t *ys, int32_t *flag)
+k_lin_resid_rms(LinSum p, const float *scale, float *x, const float *gamma, uint8_t *ys, float *rm)
 {
-    __shared__ float red[4];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, row = blockIdx.x * 4 + wv, H = p.M;
     float mx = 0.0f;
     if (row < p.rows) {
@@ -652,19 +665,15 @@ k_lin_resid_rms(LinSum p, const float *scale, float *x, const float *gamma, uint
             split_store8(ys, row, H, rec, q, a, b);
         }
     }
-    mx = wave_max_dpp(mx);
-    if (lane == 0) red[wv] = mx;
-    __syncthreads();
-    if (threadIdx.x == 0 && dc_out_of_range(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])))) *flag = 1;
+    range_note(rm + row, mx, lane);
 }
 
 // Channel-first f32 [C][L] -> split rows: 64 positions x 32 channels through
 // LDS; lane = position.
 __global__ void __launch_bounds__(256)
-k_cf_split(const float *x, int C, int L, uint8_t *ys, int32_t *flag)
+k_cf_split(const float *x, int C, int L, uint8_t *ys, float *rm)
 {
     __shared__ float tile[32][65];
-    __shared__ float red[4];
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6, p0 = blockIdx.x * 64, rec = blockIdx.y;
     for (int i = wv; i < 32; i += 4) tile[i][lane] = p0 + lane < L ? x[(size_t)(32 * rec + i) * L + p0 + lane] : 0.0f;
     __syncthreads();
@@ -682,10 +691,7 @@ k_cf_split(const float *x, int C, int L, uint8_t *ys, int32_t *flag)
         *(uint4 *)y = uint4{h[0], h[1], h[2], h[3]};
         *(uint4 *)(y + 64) = uint4{l[0], l[1], l[2], l[3]};
     }
-    mx = wave_max_dpp(mx);
-    if (lane == 0) red[wv] = mx;
-    __syncthreads();
-    if (t == 0 && dc_out_of_range(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])))) *flag = 1;
+    range_note(rm + ((size_t)blockIdx.x * gridDim.y + rec) * 4 + wv, mx, lane);
 }
 
 // One-channel output convolution over f32 rows [L][C], clamp to [-1, 1], the
@@ -759,6 +765,65 @@ hipError_t enqueue_snake_par(const float *alpha, const float *beta, int n, float
     return hipGetLastError();
 }
 
+// Words of the range check for T frames at most: of a stage's signal the
+// partial sums' kernel has the most waves (one per 64 rows and 8 channels).
+static size_t range_words(int64_t L, int M, int os) { return (size_t)(L / 16 + 16) * (M / (16 * DC_CB)) * 3 * os + 16; }
+
+size_t dec_range_words(const DecoderDev &d, int64_t T)
+{
+    size_t n = 0;
+    if (d.tf_rows) {
+        const size_t rms = T + 4, cf = (T / 64 + 1) * (d.latent / 8), att = (T / 16 + 1) * 4 * d.n_heads;
+        n += rms + cf + d.n_tf * (2 * rms + att + (size_t)T * d.inter / 512 + 4);
+    }
+    if (d.vocos_rows) {
+        int64_t L = T;
+        for (int u = 0; u < d.n_up; u++) L *= d.up[u].conv_t.stride;
+        n += (size_t)(L / 64 + 1) * (d.voc_init.ic / 8) + range_words(L, d.voc_init.oc, 1);
+        for (int b = 0; b < d.n_voc; b++) {
+            const DecVocos &B = d.voc[b];
+            n += range_words(L, B.up.oc, B.up.stride);
+            L *= B.up.stride;
+            n += 2 * B.n_res * range_words(L, B.up.oc, 1);
+        }
+    }
+    return n;
+}
+
+// `words` words for the next launch, `per` of them a group.
+static float *range_take(RangeLog &log, size_t words, int per)
+{
+    if (words > (size_t)(log.end - log.next)) {
+        log.full = true;
+        return log.next;
+    }
+    float *p = log.next;
+    log.next += words;
+    log.sig.push_back(RangeSignal{p, (uint32_t)words, (uint32_t)per});
+    return p;
+}
+
+// *out (host memory, 0 before) becomes 1 if `flag` is set or a signal left
+// the split's range.
+hipError_t enqueue_range_result(const RangeLog &log, const int32_t *flag, int32_t *out, hipStream_t s)
+{
+    RangeList l{};
+    size_t n = 0;
+    do {
+        const int k = (int)std::min<size_t>(log.sig.size() - n, RANGE_SIGNALS);
+        uint32_t most = 0;
+        for (int i = 0; i < k; i++) {
+            l.s[i] = log.sig[n + i];
+            most = std::max(most, l.s[i].words);
+        }
+        if (!k) l.s[0] = RangeSignal{nullptr, 0, 1};
+        hipLaunchKernelGGL(k_range_result, dim3(most < 4096 ? 1 : 8, std::max(k, 1)), dim3(256), 0, s, flag, l, out);
+        VCHK(hipGetLastError());
+        n += k;
+    } while (n < log.sig.size());
+    return hipSuccess;
+}
+
 // Tile form and slices of the contraction: the launch's rounds over the CUs
 // times a workgroup's matrix cycles, plus the partial sums' traffic.  Forms:
 // 256 positions; 128 (each wave's weights then outrun the L1 by a third); 64
@@ -816,8 +881,8 @@ static void dc_launch_form(int form, const DcIn &in, const uint8_t *w, const DcO
 }
 
 template <int KT, int EPI>
-static hipError_t dconv(const DcIn &in, const uint8_t *w, const DcOut &o, int nph, const DecoderWs &ws, hipStream_t s,
-                        const DcFuse *fz = nullptr, bool *fused = nullptr)
+static hipError_t dconv(const DcIn &in, const uint8_t *w, DcOut o, int nph, const DecoderWs &ws, RangeLog &log,
+                        hipStream_t s, DcFuse *fz = nullptr, bool *fused = nullptr)
 {
     int form = 0, ks = 1;
     DcGeo g{};
@@ -833,14 +898,23 @@ static hipError_t dconv(const DcIn &in, const uint8_t *w, const DcOut &o, int np
         if (fz && g.tm == 1 && ks == 1) {
             *fused = true;
             if (form == DC_P256) g.tn = (in.L + 64 * DC_FUSE_PB - 1) / (64 * DC_FUSE_PB);
+            const int per = form == DC_SK64 ? 4 : 2;
+            o.rm = range_take(log, 4 * (size_t)g.tn, per);
+            if (fz->o.ys) fz->o.rm = range_take(log, 4 * (size_t)g.tn, per);
+            if (log.full) return hipErrorInvalidValue;
             dc_launch_form<KT, EPI, true>(form, in, w, o, g, *fz, s);
             return hipGetLastError();
         }
     }
+    // a word a wave; with a stride one per 16 positions
+    const int64_t rows = (int64_t)in.L * nph, n = rows * (o.M / 8);
+    if (o.ys && ks > 1) o.rm = range_take(log, (size_t)(n + 255) / 256 * 4, o.M / 8);
+    else if (o.ys && o.os > 1) o.rm = range_take(log, (size_t)g.tn * (16 >> form) * g.tm * nph, g.tm * nph);
+    else if (o.ys) o.rm = range_take(log, 4 * (size_t)g.tn * g.tm, g.tm << form);
+    if (log.full) return hipErrorInvalidValue;
     dc_launch_form<KT, EPI, false>(form, in, w, o, g, DcFuse{}, s);
     VCHK(hipGetLastError());
     if (ks > 1) {
-        const int64_t rows = (int64_t)in.L * nph, n = rows * (o.M / 8);
         hipLaunchKernelGGL(k_dconv_reduce<EPI>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, ws.part, ks, rows, nph, o);
     }
     return hipGetLastError();
@@ -889,39 +963,49 @@ static hipError_t linear(const uint8_t *x, int nc, int rows, const DecLin &w, in
 #define K_RMS1(KS) k_lin_resid_rms<1, KS>
 #define K_RMS4(KS) k_lin_resid_rms<4, KS>
 
-static hipError_t resid_rms(const LinSum &p, const float *scale, float *x, const float *gamma, uint8_t *ys, int32_t *flag,
+static hipError_t resid_rms(const LinSum &p, const float *scale, float *x, const float *gamma, uint8_t *ys, RangeLog &log,
                             hipStream_t s)
 {
     const dim3 grid((p.rows + 3) / 4);
-    if (p.M <= 512) LIN_BY_KS(K_RMS1, grid, p, scale, x, gamma, ys, flag);
-    else LIN_BY_KS(K_RMS4, grid, p, scale, x, gamma, ys, flag);
+    float *rm = range_take(log, 4 * (size_t)grid.x, 64);
+    if (log.full) return hipErrorInvalidValue;
+    if (p.M <= 512) LIN_BY_KS(K_RMS1, grid, p, scale, x, gamma, ys, rm);
+    else LIN_BY_KS(K_RMS4, grid, p, scale, x, gamma, ys, rm);
     return hipSuccess;
 }
 
 // The transformer over T positions: in [latent][T] channel-first f32 to out
 // likewise.  bufs: four buffers of the workspace other than those two.
 hipError_t enqueue_dec_tf(const DecoderDev &d, const DecoderWs &ws, const float *in, float *out, float *const bufs[4], int T,
-                          hipStream_t s)
+                          RangeLog &log, hipStream_t s)
 {
     const int H = d.hidden, A = d.n_heads * d.head_dim, I = d.inter, LAT = d.latent;
     uint8_t *xs = (uint8_t *)bufs[0], *hs = (uint8_t *)bufs[1];
     float *x = bufs[2], *qkv = bufs[3];
     LinSum p{};
-    hipLaunchKernelGGL(k_cf_split, dim3((T + 63) / 64, LAT / 32), dim3(256), 0, s, in, LAT, T, hs, ws.range_flag);
+    float *rm = range_take(log, (size_t)((T + 63) / 64) * (LAT / 8), LAT / 8);
+    if (log.full) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_cf_split, dim3((T + 63) / 64, LAT / 32), dim3(256), 0, s, in, LAT, T, hs, rm);
     VCHK(hipGetLastError());
     VCHK(linear(hs, LAT / 32, T, d.tf_in, H, d.tf_in_b, ws, &p, s));
-    VCHK(resid_rms(p, nullptr, x, d.tf[0].in_norm, xs, ws.range_flag, s));
+    VCHK(resid_rms(p, nullptr, x, d.tf[0].in_norm, xs, log, s));
     for (int l = 0; l < d.n_tf; l++) {
         const DecLayer &L = d.tf[l];
         VCHK(linear(xs, H / 32, T, L.pqkv, 3 * A, nullptr, ws, &p, s));
         LIN_BY_KS(K_ROWS, dim3((unsigned)(((int64_t)T * 3 * A / 4 + 255) / 256)), p, qkv);
-        VCHK(enqueue_dec_attn_rows(d, qkv, T, hs, ws.range_flag, s));
+        // its blocks of 16 positions: four waves a head
+        rm = range_take(log, (size_t)((T + 15) / 16) * d.n_heads * 4, 16 * d.n_heads);
+        if (log.full) return hipErrorInvalidValue;
+        VCHK(enqueue_dec_attn_rows(d, qkv, T, hs, rm, s));
         VCHK(linear(hs, A / 32, T, L.po, H, nullptr, ws, &p, s));
-        VCHK(resid_rms(p, L.attn_scale, x, L.post_norm, xs, ws.range_flag, s));
+        VCHK(resid_rms(p, L.attn_scale, x, L.post_norm, xs, log, s));
         VCHK(linear(xs, H / 32, T, L.pgu, 2 * I, nullptr, ws, &p, s));
-        LIN_BY_KS(K_SWIGLU, dim3((unsigned)(((int64_t)T * I / 8 + 255) / 256)), p, hs, ws.range_flag);
+        const dim3 sg((unsigned)(((int64_t)T * I / 8 + 255) / 256));
+        rm = range_take(log, 4 * (size_t)sg.x, I / 8);
+        if (log.full) return hipErrorInvalidValue;
+        LIN_BY_KS(K_SWIGLU, sg, p, hs, rm);
         VCHK(linear(hs, I / 32, T, L.pdown, H, nullptr, ws, &p, s));
-        VCHK(resid_rms(p, L.mlp_scale, x, l + 1 < d.n_tf ? d.tf[l + 1].in_norm : d.tf_norm, xs, ws.range_flag, s));
+        VCHK(resid_rms(p, L.mlp_scale, x, l + 1 < d.n_tf ? d.tf[l + 1].in_norm : d.tf_norm, xs, log, s));
     }
     VCHK(linear(xs, H / 32, T, d.tf_out, LAT, d.tf_out_b, ws, &p, s));
     LIN_BY_KS(K_CF, dim3((T + 63) / 64, LAT / 32), p, out);
@@ -952,12 +1036,14 @@ int dec_tf_rows(const DecoderDev &d, size_t part_floats)
 // [voc_init.ic][L] (channel-first f32).  bufs: four buffers of the workspace
 // other than sig's.
 hipError_t enqueue_vocos(const DecoderDev &d, const DecoderWs &ws, const float *sig, float *const bufs[4], int L, int64_t cut,
-                         float *audio, bool fuse, hipStream_t s)
+                         float *audio, bool fuse, RangeLog &log, hipStream_t s)
 {
     uint8_t *sn = (uint8_t *)bufs[0], *t1 = (uint8_t *)bufs[1];
     float *x = bufs[2], *last = bufs[3];
     const int ic = d.voc_init.ic;
-    hipLaunchKernelGGL(k_cf_split, dim3((L + 63) / 64, ic / 32), dim3(256), 0, s, sig, ic, L, t1, ws.range_flag);
+    float *rm = range_take(log, (size_t)((L + 63) / 64) * (ic / 8), ic / 8);
+    if (log.full) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_cf_split, dim3((L + 63) / 64, ic / 32), dim3(256), 0, s, sig, ic, L, t1, rm);
     VCHK(hipGetLastError());
     // the snake that follows residual r of block b: the next residual's, the
     // next block's, or the last one, whose f32 rows the output conv reads
@@ -974,9 +1060,8 @@ hipError_t enqueue_vocos(const DecoderDev &d, const DecoderWs &ws, const float *
     o.os = 1;
     o.bias = d.voc_init.b;
     o.un = d.voc_init.un;
-    o.flag = ws.range_flag;
     next(-1, 0, &o);
-    VCHK((dconv<7, DC_SNAKE>(DcIn{t1, ic / 32, L, d.voc_init.dil}, d.voc_init.pw, o, 1, ws, s)));
+    VCHK((dconv<7, DC_SNAKE>(DcIn{t1, ic / 32, L, d.voc_init.dil}, d.voc_init.pw, o, 1, ws, log, s)));
     for (int b = 0; b < d.n_voc; b++) {
         const DecVocos &B = d.voc[b];
         DcOut u{};
@@ -986,11 +1071,10 @@ hipError_t enqueue_vocos(const DecoderDev &d, const DecoderWs &ws, const float *
         u.os = B.up.stride;
         u.bias = B.up.b;
         u.un = B.up.un;
-        u.flag = ws.range_flag;
         next(b, -1, &u);
         const DcIn ui{sn, B.up.ic / 32, L, 1};
-        if (B.up.taps == 2) VCHK((dconv<2, DC_X_SNAKE>(ui, B.up.pw, u, B.up.stride, ws, s)));
-        else VCHK((dconv<1, DC_X_SNAKE>(ui, B.up.pw, u, B.up.stride, ws, s)));
+        if (B.up.taps == 2) VCHK((dconv<2, DC_X_SNAKE>(ui, B.up.pw, u, B.up.stride, ws, log, s)));
+        else VCHK((dconv<1, DC_X_SNAKE>(ui, B.up.pw, u, B.up.stride, ws, log, s)));
         L *= B.up.stride;
         std::swap(sn, t1);
         for (int r = 0; r < B.n_res; r++) {
@@ -1002,7 +1086,6 @@ hipError_t enqueue_vocos(const DecoderDev &d, const DecoderWs &ws, const float *
             c1.bias = R.c1.b;
             c1.un = R.c1.un;
             c1.snake = R.a2_par;
-            c1.flag = ws.range_flag;
             DcOut c2 = c1;
             c2.ys = sn;
             c2.x = x;
@@ -1014,12 +1097,12 @@ hipError_t enqueue_vocos(const DecoderDev &d, const DecoderWs &ws, const float *
             if (fz.o.ys) fz.o.ys = t1;    // neighbouring tiles still read sn
             bool fused = false;
             const DcIn ci{sn, B.up.oc / 32, L, R.c1.dil};
-            VCHK((dconv<7, DC_SNAKE>(ci, R.c1.pw, c1, 1, ws, s, fuse ? &fz : nullptr, &fused)));
+            VCHK((dconv<7, DC_SNAKE>(ci, R.c1.pw, c1, 1, ws, log, s, fuse ? &fz : nullptr, &fused)));
             if (fused) {
                 std::swap(sn, t1);
                 continue;
             }
-            VCHK((dconv<1, DC_X_SNAKE>(DcIn{t1, B.up.oc / 32, L, 1}, R.c2.pw, c2, 1, ws, s)));
+            VCHK((dconv<1, DC_X_SNAKE>(DcIn{t1, B.up.oc / 32, L, 1}, R.c2.pw, c2, 1, ws, log, s)));
         }
     }
     const int ch = d.n_voc ? d.voc[d.n_voc - 1].up.oc : d.voc_init.oc;

@@ -813,7 +813,7 @@ static inline size_t attn_tile_lds(int hd, int W)
 template <int HD, bool ROWS>
 __global__ void __launch_bounds__(256)
 k_dec_attn_tile(const float *qkv, int heads, int T, int W, const float *cs, const float *sn, int64_t rope_rows,
-                float *out, int32_t *flag)
+                float *out, float *rm)
 {
     static_assert(HD % 4 == 0 && HD / 4 <= 16, "a lane's p.v takes 4 consecutive dims of 16 groups");
     extern __shared__ float sm[];
@@ -979,12 +979,7 @@ k_dec_attn_tile(const float *qkv, int heads, int T, int W, const float *cs, cons
             *(uint2 *)y = uint2{h0, h1};
             *(uint2 *)(y + 64) = uint2{l0, l1};
         }
-        float *red = Qs;                       // the queries are in registers
-        const float mx = wave_max_dpp(t < T ? fmaxf(fmaxf(fabsf(o.x), fabsf(o.y)), fmaxf(fabsf(o.z), fabsf(o.w))) : 0.0f);
-        if ((tid & 63) == 0) red[tid >> 6] = mx;
-        __syncthreads();
-        const float m4 = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-        if (tid == 0 && (!(m4 < 65504.0f) || (m4 > 0.0f && m4 < 0x1p-14f))) *flag = 1;
+        range_note(rm + ((size_t)blockIdx.x * gridDim.y + h) * 4 + (tid >> 6), t < T ? fmaxf(fmaxf(fabsf(o.x), fabsf(o.y)), fmaxf(fabsf(o.z), fabsf(o.w))) : 0.0f, tid & 63);
         return;
     }
     if (t >= T) return;
@@ -1369,11 +1364,11 @@ bool dec_attn_tiled(const DecoderDev &d)
     return d.window + ATT_QB - 1 <= 16 * ATT_SLOTS && attn_tile_lds(d.head_dim, d.window) <= 65536;
 }
 
-hipError_t enqueue_dec_attn_rows(const DecoderDev &d, const float *qkv, int T, uint8_t *ys, int32_t *flag, hipStream_t s)
+hipError_t enqueue_dec_attn_rows(const DecoderDev &d, const float *qkv, int T, uint8_t *ys, float *rm, hipStream_t s)
 {
     hipLaunchKernelGGL((k_dec_attn_tile<64, true>), dim3((T + ATT_QB - 1) / ATT_QB, d.n_heads), dim3(256),
                        attn_tile_lds(d.head_dim, d.window), s, qkv, d.n_heads, T, d.window, d.rope_cos, d.rope_sin,
-                       d.rope_rows, (float *)ys, flag);
+                       d.rope_rows, (float *)ys, rm);
     return hipGetLastError();
 }
 
@@ -1426,11 +1421,14 @@ static hipError_t enqueue_dec_tf_cf(const DecoderDev &d, const DecoderWs &ws, in
     return hipSuccess;
 }
 
+// out_of_range (host memory, 0 before; may be null): 1 behind it if an input
+// of the split convolutions left their range.
 hipError_t enqueue_decode(const DecoderDev &d, const DecoderWs &ws, const uint32_t *codes, int T, int64_t cut,
-                          float *audio, hipStream_t s)
+                          float *audio, int32_t *out_of_range, hipStream_t s)
 {
     if (T < 1 || T > ws.cap_frames) return hipErrorInvalidValue;
-    if (ws.range_flag) DCHK(hipMemsetAsync(ws.range_flag, 0, sizeof(int32_t), s));
+    DCHK(hipMemsetAsync(ws.range_flag, 0, sizeof(int32_t), s));
+    RangeLog log{ws.rmax, ws.rmax + ws.rmax_words, false, {}};
     const int D = d.codebook_dim, V = d.vq_dim;
     // 1. VQ -> [V][T]
     if (d.n_rest == 15)
@@ -1447,7 +1445,7 @@ hipError_t enqueue_decode(const DecoderDev &d, const DecoderWs &ws, const uint32
     // 3. transformer: [LAT][T] in ws.a, back to ws.a
     if (d.tf_rows && !ws.f32 && dec_x3() && T <= dec_tf_rows(d, ws.part_cap)) {
         float *const bufs[4] = {ws.b, ws.c, ws.d, ws.e};
-        DCHK(enqueue_dec_tf(d, ws, ws.a, ws.a, bufs, T, s));
+        DCHK(enqueue_dec_tf(d, ws, ws.a, ws.a, bufs, T, log, s));
     } else {
         DCHK(enqueue_dec_tf_cf(d, ws, T, s));
     }
@@ -1475,7 +1473,8 @@ hipError_t enqueue_decode(const DecoderDev &d, const DecoderWs &ws, const uint32
     }
     if (d.vocos_rows && !ws.f32 && dec_x3()) {
         float *const bufs[4] = {ws.c, ws.d, ws.e, other};
-        return enqueue_vocos(d, ws, sig, bufs, L, cut, audio, dec_fuse_voc(), s);
+        DCHK(enqueue_vocos(d, ws, sig, bufs, L, cut, audio, dec_fuse_voc(), log, s));
+        return out_of_range ? enqueue_range_result(log, ws.range_flag, out_of_range, s) : hipSuccess;
     }
     // 5. Vocos: init conv with the first block's pre-snake (or the final
     // snake) fused
@@ -1533,7 +1532,8 @@ hipError_t enqueue_decode(const DecoderDev &d, const DecoderWs &ws, const uint32
     // 6. output conv on snake(x) + clamp, first `cut` samples dropped
     hipLaunchKernelGGL(k_out_conv, dim3((L + 255) / 256), dim3(256), 0, s, sn, ch, L, d.out_w, d.out_b, d.out_k,
                        d.out_dil, cut, audio);
-    return hipGetLastError();
+    DCHK(hipGetLastError());
+    return out_of_range ? enqueue_range_result(log, ws.range_flag, out_of_range, s) : hipSuccess;
 }
 
 // Algorithmic floating-point operations of enqueue_decode over T frames:

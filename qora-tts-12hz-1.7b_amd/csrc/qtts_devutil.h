@@ -102,6 +102,14 @@ __device__ __forceinline__ float add_xor16_split(float lo, float hi)
     return swap_pair_sum(r[0], r[1]);
 }
 
+// Range check of a split signal (qtts_dconv.hip): the largest |value| that a
+// wave stored, into the wave's own word.
+__device__ __forceinline__ void range_note(float *at, float mx, int lane)
+{
+    mx = wave_max_dpp(mx);
+    if (lane == 0) *at = mx;
+}
+
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ f32x4 ld4(const float *p) { return *(const f32x4 *)p; }

@@ -4,6 +4,8 @@
 #pragma once
 #include "qtts_device.h"
 
+#include <vector>
+
 namespace qtts {
 
 constexpr int MAX_CHUNKS = 128;          // KV pages per sequence (8192 positions)
@@ -224,12 +226,28 @@ struct DecoderDev {
     bool vocos_rows;                      // the Vocos stages run position-major (qtts_dconv.hip)
     bool weights_f32;                     // a weight matrix outside the split-f16 range: f32 matrix path
 };
+// The range words of one signal: `per` words a group of positions.
+struct RangeSignal {
+    const float *p;
+    uint32_t words, per;
+};
+constexpr int RANGE_SIGNALS = 64;
+struct RangeList {
+    RangeSignal s[RANGE_SIGNALS];
+};
+struct RangeLog {
+    float *next, *end;
+    bool full;
+    std::vector<RangeSignal> sig;
+};
 struct DecoderWs {
     float *a, *b, *c, *d, *e;             // each floats_per_frame * cap_frames
     float *part;                          // split-K partial sums
     size_t part_cap;                      // floats in part
     uint32_t *codes;                      // [n_rest + 1][cap_frames]
-    int32_t *range_flag;                  // set by a split-f16 convolution whose inputs left its range
+    int32_t *range_flag;                  // set by a channel-first split-f16 convolution whose inputs left its range
+    float *rmax;                          // the position-major stages' range words, rmax_words of them
+    size_t rmax_words;
     int cap_frames;
     bool f32;                             // this decode on the f32 matrix path
 };
@@ -342,7 +360,7 @@ hipError_t enqueue_gemm_gateup(const TalkerDev &m, const PrefillWs &pw, int l, i
 hipError_t enqueue_talker_prefill(const TalkerDev &m, const PrefillWs &pw, int M, int64_t start,
                                   float *hidden_out, hipStream_t s);
 hipError_t enqueue_decode(const DecoderDev &d, const DecoderWs &ws, const uint32_t *codes, int T, int64_t cut,
-                          float *audio, hipStream_t s);
+                          float *audio, int32_t *out_of_range, hipStream_t s);
 bool vocos_fits(const DecoderDev &d);
 size_t dconv_weight_bytes(int rows, int ic, int kt);
 constexpr int DC_VOCOS_CB = 6, DC_TF_CB = 4;   // 16-channel blocks a tile
@@ -350,12 +368,14 @@ hipError_t enqueue_dconv_pack(const float *w, int rows, int ic, int kt, int cb, 
 bool dec_tf_fits(const DecoderDev &d);
 int dec_tf_rows(const DecoderDev &d, size_t part_floats);
 hipError_t enqueue_dec_tf(const DecoderDev &d, const DecoderWs &ws, const float *in, float *out, float *const bufs[4], int T,
-                          hipStream_t s);
+                          RangeLog &log, hipStream_t s);
+size_t dec_range_words(const DecoderDev &d, int64_t T);
+hipError_t enqueue_range_result(const RangeLog &log, const int32_t *flag, int32_t *out, hipStream_t s);
 bool dec_attn_tiled(const DecoderDev &d);
-hipError_t enqueue_dec_attn_rows(const DecoderDev &d, const float *qkv, int T, uint8_t *ys, int32_t *flag, hipStream_t s);
+hipError_t enqueue_dec_attn_rows(const DecoderDev &d, const float *qkv, int T, uint8_t *ys, float *rm, hipStream_t s);
 hipError_t enqueue_snake_par(const float *alpha, const float *beta, int n, float *out, hipStream_t s);
 hipError_t enqueue_vocos(const DecoderDev &d, const DecoderWs &ws, const float *sig, float *const bufs[4], int L, int64_t cut,
-                         float *audio, bool fuse, hipStream_t s);
+                         float *audio, bool fuse, RangeLog &log, hipStream_t s);
 double decode_flops(const DecoderDev &d, int T);
 hipError_t enqueue_gateup_timing(const TalkerDev &m, const Workspace &ws, int l, hipStream_t s);
 hipError_t enqueue_attn_timing(const TalkerDev &m, const Workspace &ws, int l, int slot, int64_t pos,

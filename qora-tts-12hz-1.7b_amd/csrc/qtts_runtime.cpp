@@ -2221,7 +2221,8 @@ static int ensure_dec_ws(qtts_ctx *c, int frames)
     const size_t per = (size_t)c->dec_floats_per_frame * frames;
     const size_t part = DEC_PART_FLOATS;
     void *m = nullptr;
-    HIPCHK(c, hipMalloc(&m, (5 * per + part) * sizeof(float) + (size_t)16 * frames * sizeof(uint32_t) + 256));
+    const size_t rw = dec_range_words(c->dec, frames);
+    HIPCHK(c, hipMalloc(&m, (5 * per + part + rw) * sizeof(float) + (size_t)16 * frames * sizeof(uint32_t) + 256));
     c->dws_mem = m;
     float *f = (float *)m;
     c->dws.a = f;
@@ -2231,7 +2232,9 @@ static int ensure_dec_ws(qtts_ctx *c, int frames)
     c->dws.e = f + 4 * per;
     c->dws.part = f + 5 * per;
     c->dws.part_cap = part;
-    c->dws.codes = (uint32_t *)(f + 5 * per + part);
+    c->dws.rmax = f + 5 * per + part;
+    c->dws.rmax_words = rw;
+    c->dws.codes = (uint32_t *)(c->dws.rmax + rw);
     c->dws.range_flag = (int32_t *)(c->dws.codes + (size_t)16 * frames);
     c->dws.cap_frames = frames;
     return QTTS_OK;
@@ -2285,8 +2288,8 @@ extern "C" int qtts_decode_to_audio(qtts_ctx *c, const uint32_t *codes, int64_t 
     // range; inputs outside it (flagged by the convolutions) repeat the
     // decode on the f32 matrix path
     c->dws.f32 = d.weights_f32;
-    HIPCHK(c, enqueue_decode(d, c->dws, c->dws.codes, (int)T, cut, out, c->stream));
-    HIPCHK(c, enqueue_move(MoveList{{{c->dws.range_flag, c->h_err, 1}}}, 1, c->stream));
+    *c->h_err = 0;
+    HIPCHK(c, enqueue_decode(d, c->dws, c->dws.codes, (int)T, cut, out, c->h_err, c->stream));
     // the samples come along with the flag; a decode that has to be repeated
     // sends them again
     if (out == dev && !(flags & QTTS_DEVICE_PTRS))
@@ -2294,7 +2297,7 @@ extern "C" int qtts_decode_to_audio(qtts_ctx *c, const uint32_t *codes, int64_t 
     HIPCHK(c, hipStreamSynchronize(c->stream));
     if (*c->h_err && !c->dws.f32) {
         c->dws.f32 = true;
-        const hipError_t e = enqueue_decode(d, c->dws, c->dws.codes, (int)T, cut, out, c->stream);
+        const hipError_t e = enqueue_decode(d, c->dws, c->dws.codes, (int)T, cut, out, nullptr, c->stream);
         c->dws.f32 = false;
         HIPCHK(c, e);
         if (out == dev && !(flags & QTTS_DEVICE_PTRS))
@@ -3048,7 +3051,7 @@ extern "C" int qtts_time_decode(qtts_ctx *c, int64_t n_frames, int32_t iters, do
     for (int b = 0; b < d.n_voc; b++) factor *= d.voc[b].up.stride;
     RCHK(ensure_io(c, (int64_t)T * factor));
     *flops = decode_flops(d, T);
-    return time_launches(c, iters, [&](int) { return enqueue_decode(d, c->dws, c->dws.codes, T, 0, c->d_io, c->stream); },
+    return time_launches(c, iters, [&](int) { return enqueue_decode(d, c->dws, c->dws.codes, T, 0, c->d_io, nullptr, c->stream); },
                          avg_us, false);
 }
 

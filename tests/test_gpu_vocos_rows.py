@@ -68,3 +68,34 @@ def test_stride_kernel(ctx):
     c = d.vocos_blocks[0].upsample
     c.weight, c.kernel_size = np.ascontiguousarray(c.weight[:, :, :4]), 4
     run(ctx, d, (1, 9, 130))
+
+
+def test_quiet_channels_beside_loud_ones(ctx, monkeypatch):
+    """One 96-channel tile of the first signal near 1e-7 (below what lo
+    carries) beside a loud one: the range check looks at all channels of the
+    positions, so the decode stays on the split path (other bits than the f32
+    one's), and is as accurate."""
+    d = decoder((192, 96), (3,))
+    c = d.vocos_init
+    c.weight[:96] *= np.float32(1e-7)
+    c.bias[:96] *= np.float32(1e-7)
+    run(ctx, d, (1, 40, 150))
+    codes = np.random.Generator(np.random.PCG64(5)).integers(0, 64, (16, 40)).astype(np.uint32)
+    got = ctx.decode_to_audio(codes)
+    monkeypatch.setenv("QTTS_DEC_F32", "1")
+    assert not np.array_equal(got.view(np.uint32), ctx.decode_to_audio(codes).view(np.uint32))
+
+
+def test_quiet_positions_repeat_the_decode(ctx, monkeypatch):
+    """A whole signal near 1e-7: out of the split's range, the decode is
+    repeated on the f32 path (its bits)."""
+    d = decoder((192, 96), (3,))
+    d.vocos_init.weight *= np.float32(1e-7)
+    d.vocos_init.bias *= np.float32(1e-7)
+    ctx.upload_decoder(d)
+    for T in (1, 40, 150):
+        codes = np.random.Generator(np.random.PCG64(T)).integers(0, 64, (16, T)).astype(np.uint32)
+        monkeypatch.delenv("QTTS_DEC_F32", raising=False)
+        got = ctx.decode_to_audio(codes)
+        monkeypatch.setenv("QTTS_DEC_F32", "1")
+        assert np.array_equal(got.view(np.uint32), ctx.decode_to_audio(codes).view(np.uint32)), f"{T} frames"
