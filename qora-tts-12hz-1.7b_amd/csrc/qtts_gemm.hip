@@ -625,15 +625,17 @@ size_t mm_swiglu_part_floats(const Q4Frag &w, int M)
 }
 
 // Whether plain rows run one workgroup per (tile, K segment) and add partial
-// sums, against one long K loop a tile: a segment saved is about 2.2 us while
-// the tiles alone do not fill the CUs, the second launch costs about 10, and
-// the partial sums go out and back at about 4.2 TB/s.  Loop / segments:
-// 6144 x 2048 16 rows 50 / 16 us, 400 rows 74 / 68, 500 rows 75 / 80;
-// 2048 x 4096 64 rows 21 / 18, 100 rows 22 / 24; 1024 deep 13 / 13 at 3 rows
-// (no gain at any count).
-static bool rows_by_segment(int rows, size_t ncols, int nseg)
+// sums, against one long K loop a tile: a segment saved is 2.2 us while the
+// tiles alone do not fill the CUs, the second launch costs 5, a second round
+// of workgroups 6 more, and the partial sums go out and back at about 4.2 TB/s.
+// Loop / segments, us, calls one behind the other: 6144 x 2048 16 rows 48 / 14,
+// 400 rows 72 / 67, 500 rows 72 / 82; 2048 x 4096 64 rows 19 / 16, 100 rows 20 /
+// 22; 1024 x 2048 16 rows 11.5 / 8.9, 130 rows 12.0 / 12.8; 512 x 2048 3 rows
+// 7.7 / 8.8 (never).
+static bool rows_by_segment(int64_t rows, size_t ncols, int nseg)
 {
-    return 8.0 * rows * ncols * nseg < 4.2e6 * (2.2 * (nseg - 1) - 10);
+    const bool rounds = (rows + 79) / 80 * ((int64_t)(ncols + 127) / 128) * nseg > 256;
+    return 8.0 * rows * ncols * nseg < 4.2e6 * (2.2 * (nseg - 1) - (rounds ? 11 : 5));
 }
 
 // Plain rows: Y[M][ldy] columns 0..ng*32-1 = (silu)(X W (+ bias)), the rows
@@ -688,7 +690,7 @@ size_t mm_plain_ws_floats(const Q4Frag &w, int64_t M, size_t most)
 {
     const size_t nseg = mm_segments(w), ncols = (size_t)w.ng * 32;
     const size_t loop = (size_t)M * (w.kc * 64 + nseg), seg = loop + (size_t)M * nseg * ncols;
-    return std::min(most, seg <= most && rows_by_segment((int)M, ncols, (int)nseg) ? seg : loop);
+    return std::min(most, seg <= most && rows_by_segment(M, ncols, (int)nseg) ? seg : loop);
 }
 
 }  // namespace qtts
