@@ -740,9 +740,6 @@ k_out_rows(const float *x, int C, int L, const float *w, float bias, int dil, in
 #define VCHK(x) do { hipError_t e_ = (x); if (e_ != hipSuccess) return e_; } while (0)
 
 constexpr int DC_CB = DC_VOCOS_CB, DC_LIN_CB = DC_TF_CB;
-// position blocks a wave of the fused residual unit: 4 spill (160 frames: 325
-// us a unit, with 2 242 us)
-constexpr int DC_FUSE_PB = 2;
 
 bool dconv_fits(int oc, int ic, int kt, int dil)
 {
@@ -830,11 +827,13 @@ hipError_t enqueue_range_result(const RangeLog &log, const int32_t *flag, int32_
 // positions with the records dealt to the four waves (SK), where the four
 // hold different weights: few positions take it (a k 7 convolution of 672
 // positions and 192 channels 45 us, on 64-position tiles whose waves share
-// the weights 118).
+// the weights 118).  A fused residual unit (one slice) does not run on 256
+// positions: its four position blocks a wave spill (160 frames: 325 us a unit,
+// with two blocks 242).
 constexpr double DC_WAIT = 2500;   // cycles, fitted at 1 to 400 frames (0 and 5000 are up to 2% slower at 160)
 enum { DC_P256 = 0, DC_P128 = 1, DC_SK64 = 2 };
 
-static void dc_plan(int L, int tm, int nph, int nc, int kt, int M, size_t part_cap, int *form, int *ks_out)
+static void dc_plan(int L, int tm, int nph, int nc, int kt, int M, size_t part_cap, bool fuse, int *form, int *ks_out)
 {
     double best = 1e300;
     for (int f = DC_P256; f <= DC_SK64; f++) {
@@ -842,6 +841,7 @@ static void dc_plan(int L, int tm, int nph, int nc, int kt, int M, size_t part_c
         for (int ks = 1; ks <= std::min(nc, 16); ks++) {
             const int cps = (nc + ks - 1) / ks;
             if ((nc + cps - 1) / cps != ks) continue;     // no empty slice
+            if (fuse && ks == 1 && f == DC_P256) continue;
             const double plane = (double)L * nph * M;
             if (ks > 1 && plane * ks > (double)part_cap) break;
             const int64_t wgs = (int64_t)tn * tm * nph * ks;
@@ -875,9 +875,17 @@ template <int KT, int EPI, bool FUSE>
 static void dc_launch_form(int form, const DcIn &in, const uint8_t *w, const DcOut &o, const DcGeo &g, const DcFuse &fz,
                            hipStream_t s)
 {
-    if (form == DC_P256) dc_launch<FUSE ? DC_FUSE_PB : 4, KT, EPI, FUSE, false>(in, w, o, g, fz, s);
-    else if (form == DC_P128) dc_launch<2, KT, EPI, FUSE, false>(in, w, o, g, fz, s);
-    else dc_launch<4, KT, EPI, FUSE, true>(in, w, o, g, fz, s);
+    if (form == DC_SK64) {
+        dc_launch<4, KT, EPI, FUSE, true>(in, w, o, g, fz, s);
+        return;
+    }
+    if constexpr (!FUSE) {
+        if (form == DC_P256) {
+            dc_launch<4, KT, EPI, FUSE, false>(in, w, o, g, fz, s);
+            return;
+        }
+    }
+    dc_launch<2, KT, EPI, FUSE, false>(in, w, o, g, fz, s);
 }
 
 template <int KT, int EPI>
@@ -888,16 +896,16 @@ static hipError_t dconv(const DcIn &in, const uint8_t *w, DcOut o, int nph, cons
     DcGeo g{};
     g.tm = o.M / (16 * DC_CB);
     g.nph = nph;
-    dc_plan(in.L, g.tm, nph, in.nc, KT, o.M, ws.part_cap, &form, &ks);
+    // one channel tile holds all of a fused conv2's input
+    const bool fuse = KT == 7 && fz && g.tm == 1;
+    dc_plan(in.L, g.tm, nph, in.nc, KT, o.M, ws.part_cap, fuse, &form, &ks);
     g.tn = (in.L + (256 >> form) - 1) / (256 >> form);
     g.cps = (in.nc + ks - 1) / ks;
     g.ks = ks;
     g.part = ws.part;
     if constexpr (KT == 7) {
-        // one channel tile holds all of conv2's input, no split sums
-        if (fz && g.tm == 1 && ks == 1) {
+        if (fuse && ks == 1) {
             *fused = true;
-            if (form == DC_P256) g.tn = (in.L + 64 * DC_FUSE_PB - 1) / (64 * DC_FUSE_PB);
             const int per = form == DC_SK64 ? 4 : 2;
             o.rm = range_take(log, 4 * (size_t)g.tn, per);
             if (fz->o.ys) fz->o.rm = range_take(log, 4 * (size_t)g.tn, per);
