@@ -261,20 +261,29 @@ def test_few_rows_without_a_split_copy(ctx_factory, rows, path):
     dw.free()
 
 
-def test_prefill_chunked(ctx_factory):
-    """More rows than one prefill chunk (1024): the second chunk attends to
-    the first through the cache."""
-    t = synth.make_talker(seed=411, n_layers=1, text_vocab=256, rope_max_pos=2048)
+@pytest.mark.parametrize("rows", [2049, 2085])
+def test_prefill_chunked(ctx_factory, rows):
+    """More rows than one prefill chunk (2048): two equal chunks (1025 + 1024
+    and 1043 + 1042 rows), the second attends to the first through the cache.
+    Against the oracle, and the bits of the two chunks prefilled by calls of
+    their own."""
+    t = synth.make_talker(seed=411, n_layers=1, text_vocab=256, rope_max_pos=2304)
     p = synth.make_predictor(seed=412, n_layers=5)
-    c = ctx_factory(2048)
+    c = ctx_factory(2304)
     c.upload_model(t, p)
-    om = O.Model(t, p, kv_cap=2048)
+    om = O.Model(t, p, kv_cap=2304)
     rng = np.random.Generator(np.random.PCG64(2500))
-    X = rng.standard_normal((1100, t.hidden)).astype(np.float32)
-    ok, e = close(c.prefill_talker_raw_from(X, 0), om.prefill(X, 0))
+    X = rng.standard_normal((rows, t.hidden)).astype(np.float32)
+    got = c.prefill_talker_raw_from(X, 0)
+    ok, e = close(got, om.prefill(X, 0))
     assert ok, f"rel err {e}"
-    check_kv(c, om, 1, 1100)
+    check_kv(c, om, 1, rows)
     om.close()
+    c.kv_reset()
+    first = (rows + 1) // 2
+    c.prefill_talker_raw_from(X[:first], 0)
+    again = c.prefill_talker_raw_from(X[first:], first)
+    assert np.array_equal(got.view(np.uint32), again.view(np.uint32))
     c.close()
 
 
