@@ -1,14 +1,14 @@
 """qtts_gemm_q4_noalloc: qtts_gemm_q4 on device rows with nothing allocated
-(split-K partial sums in the library's per-GPU scratch array).
+(split-K partial sums and split rows in the context's workspace).
 
 Checked through the C ABI against qtts_gemm_q4 on the same weight and rows:
 two calls in a row on the same device buffers, the second with fewer rows
-(the scratch keeps the first call's contents), on both paths (GEMV passes
+(the workspace keeps the first call's contents), on both paths (GEMV passes
 and the matrix-core GEMM) and on a ragged n; bit-identical, since both run
 the same kernels in the same order, and within 1e-3 of the oracle; rows far
-outside the f16 range on the matrix cores (their largest |x| staged in the
-same array).  A weight whose passes need more scratch than the array holds
-is refused.
+outside the f16 range on the matrix cores (the factors that
+undo their staging kept there too).  A weight whose passes need more than
+4 MiB of it is refused.
 The device buffers are the caller's, allocated here with hipMalloc.
 """
 import ctypes
@@ -93,8 +93,8 @@ def test_gemm_noalloc_matches_gemm(ctx_factory, k, n, rows, path):
 
 
 def test_gemm_noalloc_extreme_rows(ctx_factory):
-    """Rows far outside the f16 range on the matrix cores: the rows' largest
-    |x| (the staging range) go to the scratch array too; bit-identical to
+    """Rows far outside the f16 range on the matrix cores: the factors that
+    undo their staging go to the workspace too; bit-identical to
     qtts_gemm_q4 on two calls in a row, the second with fewer rows."""
     c = ctx_factory(256)
     h = hip()
@@ -129,7 +129,7 @@ def test_gemm_noalloc_extreme_rows(ctx_factory):
 
 def test_gemm_noalloc_refuses_oversized_scratch(ctx_factory, monkeypatch):
     """16 slices of 128 rows (tile G8_T128) x 33,792 columns need 1,081,344
-    floats of partial sums, beyond the 1,048,576 the array holds."""
+    floats of partial sums, beyond the 1,048,576 of their limit."""
     monkeypatch.setenv("QTTS_TILE_GEMV", "1")
     c = ctx_factory(256)
     h = hip()
