@@ -561,7 +561,9 @@ int qtts_debug_force_sync_err(qtts_ctx *ctx);
 
 /* Test hook, no reference counterpart: a figure of the context's state after
  * its last call.  QTTS_ERR_INVALID for another `what`. */
-#define QTTS_QUERY_STAGING 0    /* bytes of the host staging buffer still taken (0 between calls) */
+#define QTTS_QUERY_STAGING 0         /* bytes of the host staging buffer still taken (0 between calls) */
+#define QTTS_QUERY_DECODER_ROWS 1    /* the uploaded speech decoder's position-major stages: 1 transformer + 2 Vocos */
+#define QTTS_QUERY_DECODE_REPEATED 2 /* 1: the last decode left the split's range and ran again in f32 */
 int qtts_debug_query(qtts_ctx *ctx, int32_t what, int64_t *value);
 
 /* ---- measurement ------------------------------------------------------ */

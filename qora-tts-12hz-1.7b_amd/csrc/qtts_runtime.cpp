@@ -101,6 +101,7 @@ struct qtts_ctx {
     std::vector<void *> dec_allocs;
     int64_t dec_floats_per_frame = 0;                // largest stage, [channels][positions] per frame
     DecoderWs dws{};
+    bool dec_repeated = false;                       // the last decode ran again on the f32 path
     void *dws_mem = nullptr;
 
     // Talker KV page pool: 2 * kv_cap/64 physical pages shared by the running
@@ -2295,7 +2296,8 @@ extern "C" int qtts_decode_to_audio(qtts_ctx *c, const uint32_t *codes, int64_t 
     if (out == dev && !(flags & QTTS_DEVICE_PTRS))
         HIPCHK(c, hipMemcpyAsync(audio, out, (size_t)n * sizeof(float), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    if (*c->h_err && !c->dws.f32) {
+    c->dec_repeated = *c->h_err && !c->dws.f32;
+    if (c->dec_repeated) {
         c->dws.f32 = true;
         const hipError_t e = enqueue_decode(d, c->dws, c->dws.codes, (int)T, cut, out, nullptr, c->stream);
         c->dws.f32 = false;
@@ -2747,6 +2749,8 @@ extern "C" int qtts_debug_query(qtts_ctx *c, int32_t what, int64_t *value)
     if (!c || !value) return QTTS_ERR_INVALID;
     switch (what) {
     case QTTS_QUERY_STAGING: *value = (int64_t)c->pin_top; return QTTS_OK;
+    case QTTS_QUERY_DECODER_ROWS: *value = c->has_decoder ? c->dec.tf_rows + 2 * c->dec.vocos_rows : 0; return QTTS_OK;
+    case QTTS_QUERY_DECODE_REPEATED: *value = c->dec_repeated; return QTTS_OK;
     default: return QTTS_ERR_INVALID;
     }
 }

@@ -521,7 +521,7 @@ class Context:
         step / frame batch / chain call returns QTTS_ERR_HIP once."""
         self._check(self.lib.qtts_debug_force_sync_err(self.h))
 
-    QUERIES = ("staging",)
+    QUERIES = ("staging", "decoder_rows", "decode_repeated")
 
     def debug_query(self, what):
         """A figure of the context's state after its last call (QUERIES)."""

@@ -30,6 +30,7 @@ def test_tf_rows(ctx_factory, hidden, heads, inter, latent, frames):
                            rope_max_pos=1024)
     ctx = ctx_factory(64)
     ctx.upload_decoder(d)
+    assert ctx.debug_query("decoder_rows") == 3
     rng = np.random.Generator(np.random.PCG64(hidden))
     for T in frames:
         print(f"hidden {hidden} frames {T}", flush=True)
@@ -37,5 +38,6 @@ def test_tf_rows(ctx_factory, hidden, heads, inter, latent, frames):
         ref = F.decode(d, codes)
         got = ctx.decode_to_audio(codes)
         assert got.shape == ref.shape
+        assert ctx.debug_query("decode_repeated") == 0
         err = np.abs(got.astype(np.float64) - ref).max() / np.abs(ref).max()
         assert err <= TOL, f"{T} frames: {err:.3g} of the largest sample"

@@ -27,6 +27,7 @@ def decoder(vocos, rates, dilations=(1, 3, 9), latent=64, **kw):
 
 def run(ctx, d, frames):
     ctx.upload_decoder(d)
+    assert ctx.debug_query("decoder_rows") == 2      # (heads of 16: the transformer stays channel-first)
     rng = np.random.Generator(np.random.PCG64(frames))
     for T in frames if isinstance(frames, tuple) else (frames,):
         print(f"frames {T}", flush=True)
@@ -34,6 +35,7 @@ def run(ctx, d, frames):
         ref = F.decode(d, codes)
         got = ctx.decode_to_audio(codes)
         assert got.shape == ref.shape
+        assert ctx.debug_query("decode_repeated") == 0
         err = np.abs(got.astype(np.float64) - ref).max() / np.abs(ref).max()
         assert err <= TOL, f"{T} frames: {err:.3g} of the largest sample"
 
@@ -54,8 +56,10 @@ def test_several_channel_tiles(ctx):
 
 
 def test_wide_contraction(ctx):
-    """Many records and few positions: slices of the contraction."""
-    run(ctx, decoder((768, 384), (4,), latent=256), (1, 4, 33))
+    """Many records and few positions: slices of the contraction.  (192
+    channels at the end: the output convolution's tile holds no more than 208,
+    and a decoder beyond that stays channel-first.)"""
+    run(ctx, decoder((768, 384, 192), (4, 2), latent=256), (1, 4, 33))
 
 
 def test_no_residuals(ctx):
@@ -86,16 +90,30 @@ def test_quiet_channels_beside_loud_ones(ctx, monkeypatch):
     assert not np.array_equal(got.view(np.uint32), ctx.decode_to_audio(codes).view(np.uint32))
 
 
-def test_quiet_positions_repeat_the_decode(ctx, monkeypatch):
-    """A whole signal near 1e-7: out of the split's range, the decode is
-    repeated on the f32 path (its bits)."""
+def scaled(a, f):
+    a *= np.float32(f)
+
+
+@pytest.mark.parametrize("case", ["quiet", "loud"])
+def test_out_of_range_signal_repeats_the_decode(ctx, monkeypatch, case):
+    """The first Vocos signal wholly near 1e-6, or past the f16 maximum, behind
+    inputs and weights within the range: the decode is repeated on the f32 path
+    (its bits)."""
     d = decoder((192, 96), (3,))
-    d.vocos_init.weight *= np.float32(1e-7)
-    d.vocos_init.bias *= np.float32(1e-7)
+    if case == "quiet":
+        u = d.upsample[-1]                        # its signal near 1e-3 (and the weights above 2^-14)
+        scaled(u.conv_t.weight, 1e-3)
+        scaled(u.conv_t.bias, 1e-3)
+        scaled(u.gamma, 1e-4)
+        scaled(d.vocos_init.weight, 1e-3)
+        scaled(d.vocos_init.bias, 1e-7)
+    else:
+        scaled(d.vocos_init.weight, 6e4)
     ctx.upload_decoder(d)
     for T in (1, 40, 150):
         codes = np.random.Generator(np.random.PCG64(T)).integers(0, 64, (16, T)).astype(np.uint32)
         monkeypatch.delenv("QTTS_DEC_F32", raising=False)
         got = ctx.decode_to_audio(codes)
+        assert ctx.debug_query("decode_repeated") == 1, f"{T} frames"
         monkeypatch.setenv("QTTS_DEC_F32", "1")
         assert np.array_equal(got.view(np.uint32), ctx.decode_to_audio(codes).view(np.uint32)), f"{T} frames"
