@@ -234,7 +234,7 @@ int qtts_gemm_q4(qtts_ctx *ctx, const qtts_w *w, const float *X, int64_t rows,
  * allocates nothing: no reference counterpart.  For callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving
  * loops).  The GEMV passes' split-K partial sums and the matrix cores' staged
- * rows use 64 MiB of device memory that the context holds (rows that do not
+ * rows use 32 MiB of device memory that the context holds (rows that do not
  * fit go in batches).  A weight whose GEMV passes need more than 4 MiB (S * 2
  * * npad floats, S = ceil(k / 2048) for the default tile) is refused with
  * QTTS_ERR_CAPACITY below 16 rows unless QTTS_PATH_MFMA is asked for.  Only

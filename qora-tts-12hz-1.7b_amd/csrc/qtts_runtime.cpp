@@ -505,11 +505,13 @@ static void drop_graph(qtts_ctx *c)
 // split-K partial sums of its GEMV passes, the matrix cores' split rows,
 // factors and partial sums.  One per context, allocated with it, so that
 // calls of different contexts (threads, streams) do not share it.  The size
-// holds 2730 rows of 6144 columns: with 4 MiB (160 of them) 2000 rows x 6144 x
-// 2048 ran as thirteen launches of half the CUs or less and took 745 us, at
-// once 161.  The GEMV passes keep their limit of 4 MiB.
-constexpr size_t SCRATCH_FLOATS = (size_t)1 << 24;          // 64 MiB
+// holds 1365 rows of 6144 columns, whole rounds of tiles: with 4 MiB (160 of
+// them) 2000 rows x 6144 x 2048 ran as thirteen launches of half the CUs or less
+// and took 745 us.  The GEMV passes keep their limit of 4 MiB; qtts_gemm_q4
+// sizes its own for the call.
+constexpr size_t SCRATCH_FLOATS = (size_t)1 << 23;          // 32 MiB
 constexpr size_t GEMV_SCRATCH_FLOATS = (size_t)1 << 20;     // 4 MiB
+constexpr size_t MM_MOST_FLOATS = (size_t)1 << 24;          // 64 MiB
 
 extern "C" int qtts_ctx_create(int device, int64_t kv_capacity, qtts_ctx **out)
 {
@@ -830,7 +832,7 @@ extern "C" int qtts_gemm_q4(qtts_ctx *c, const qtts_w *w, const float *X, int64_
     RCHK(ensure_io(c, rows * std::max({w->t.k, w->t.n, w->t.npad})));
     RCHK(stage_in(c, X, rows * w->t.k, c->d_io, flags));
     if (gemm_mfma(w, flags, rows)) {
-        RCHK(ensure_mm(c, mm_plain_ws_floats(w->f, rows, SCRATCH_FLOATS)));
+        RCHK(ensure_mm(c, mm_plain_ws_floats(w->f, rows, MM_MOST_FLOATS)));
         HIPCHK(c, enqueue_gemm_rows(w->t, w->f, c->d_io, (int)rows, c->d_io2, w->t.n, c->d_mm, c->mm_floats, c->stream));
     }
     else

@@ -59,7 +59,7 @@ def test_rows_and_shapes(ctx, k, n):
 @pytest.mark.parametrize("k,n,rows", [(6144, 2048, 450), (2048, 12288, 600), (6144, 64, 2900)])
 def test_rows_in_batches(ctx, k, n, rows):
     """More rows than run one workgroup per K segment, and more (2900 x 6144)
-    than the workspace holds at once: the same bits as in batches of 100, with
+    than the workspaces hold at once: the same bits as in batches of 100, with
     and without the call's own allocations."""
     rng = np.random.Generator(np.random.PCG64(rows))
     w = synth.q4_random(rng, k, n)
