@@ -3057,7 +3057,7 @@ extern "C" int qtts_time_decode(qtts_ctx *c, int64_t n_frames, int32_t iters, do
     for (int b = 0; b < d.n_voc; b++) factor *= d.voc[b].up.stride;
     RCHK(ensure_io(c, (int64_t)T * factor));
     *flops = decode_flops(d, T);
-    return time_launches(c, iters, [&](int) { return enqueue_decode(d, c->dws, c->dws.codes, T, 0, c->d_io, nullptr, c->stream); },
+    return time_launches(c, iters, [&](int) { return enqueue_decode(d, c->dws, c->dws.codes, T, 0, c->d_io, c->h_err, c->stream); },
                          avg_us, false);
 }
 
