@@ -126,18 +126,18 @@ struct DcFuse {
 // The split holds a value as f16 hi + lo: f32-accurate below the f16 maximum
 // and, through lo, to 2^-25 absolute.  So every wave that stores split rows
 // notes its largest |value| (a plain store: atomics on words of several waves
-// lengthened each launch by 2 us), and k_range_result judges them behind the
-// decode, over all channels of 64 positions (16 before a stride): a group that
+// lengthened each launch by 2 us), and workgroups beside the output
+// convolution's judge them (a launch of their own took 10 us, 1% of a short
+// chunk), over all channels of 64 positions (16 before a stride): a group that
 // reaches the maximum, or lies wholly below the normal f16 but is not zero, is
 // out, and the host repeats the decode on the f32 matrix path.  Quiet channels
 // beside loud ones of the same positions lose nothing that shows in the sums
 // over them.
-__global__ void __launch_bounds__(256)
-k_range_result(const int32_t *flag, RangeList l, int32_t *out)
+__device__ __forceinline__ void range_judge(const int32_t *flag, const RangeList &l, int32_t *out, int block)
 {
-    const RangeSignal g = l.s[blockIdx.y];
+    const RangeSignal g = l.s[block / l.blocks];
     // 2^b lanes a group of `per` words
-    const int lane = threadIdx.x & 63, wv = blockIdx.x * 4 + (threadIdx.x >> 6), nw = gridDim.x * 4;
+    const int lane = threadIdx.x & 63, wv = block % l.blocks * 4 + (threadIdx.x >> 6), nw = l.blocks * 4;
     const int b = g.per >= 64 ? 6 : 32 - __clz(g.per - 1), lg = lane >> b, ll = lane & ((1 << b) - 1);
     const uint32_t groups = (g.words + g.per - 1) / g.per;
     bool bad = *flag != 0;
@@ -149,6 +149,12 @@ k_range_result(const int32_t *flag, RangeList l, int32_t *out)
         bad |= !(m < 65504.0f) || (m > 0.0f && m < 0x1p-14f);
     }
     if (bad) *out = 1;
+}
+
+__global__ void __launch_bounds__(256)
+k_range_result(const int32_t *flag, RangeList l, int32_t *out)
+{
+    range_judge(flag, l, out, blockIdx.x);
 }
 
 __device__ __forceinline__ float dc_snake(float v, float ea, float eb) { return v + eb * snake_sin2(ea * v); }
@@ -698,10 +704,16 @@ k_cf_split(const float *x, int C, int L, uint8_t *ys, float *rm)
 // first `cut` samples dropped.  Workgroup: 64 positions; thread (position,
 // quarter of the channels), four quarters added in order.  Bound: reading the
 // rows (118 MB at 160 frames, 41 us; 81 us a channel-first plane at a time).
+// Workgroups from nout on: the decode's range check.
 template <int K>
 __global__ void __launch_bounds__(256)
-k_out_rows(const float *x, int C, int L, const float *w, float bias, int dil, int64_t cut, float *out)
+k_out_rows(const float *x, int C, int L, const float *w, float bias, int dil, int64_t cut, float *out, int nout,
+           const int32_t *flag, RangeList l, int32_t *out_of_range)
 {
+    if ((int)blockIdx.x >= nout) {
+        range_judge(flag, l, out_of_range, blockIdx.x - nout);
+        return;
+    }
     extern __shared__ float sm[];
     const int t = threadIdx.x, n0 = blockIdx.x * 64, pad = (K - 1) * dil, R = 64 + pad, ld = C + 4;
     float *ws = sm, *xs = sm + ((K * C + 3) & ~3);   // ws [tap][C], xs [R][ld]
@@ -800,24 +812,31 @@ static float *range_take(RangeLog &log, size_t words, int per)
     return p;
 }
 
-// *out (host memory, 0 before) becomes 1 if `flag` is set or a signal left
-// the split's range.
-hipError_t enqueue_range_result(const RangeLog &log, const int32_t *flag, int32_t *out, hipStream_t s)
+// Signals from..+63 of the log, with one or several workgroups each.
+static int range_list(const RangeLog &log, size_t from, RangeList *l)
 {
-    RangeList l{};
-    size_t n = 0;
+    const int k = (int)std::min<size_t>(log.sig.size() - from, RANGE_SIGNALS);
+    uint32_t most = 0;
+    for (int i = 0; i < k; i++) {
+        l->s[i] = log.sig[from + i];
+        most = std::max(most, l->s[i].words);
+    }
+    if (!k) l->s[0] = RangeSignal{nullptr, 0, 1};
+    l->blocks = most < 4096 ? 1 : 8;
+    return std::max(k, 1) * l->blocks;
+}
+
+// *out (host memory, 0 before) becomes 1 if `flag` is set or a signal from
+// `from` on left the split's range.
+hipError_t enqueue_range_result(const RangeLog &log, size_t from, const int32_t *flag, int32_t *out, hipStream_t s)
+{
     do {
-        const int k = (int)std::min<size_t>(log.sig.size() - n, RANGE_SIGNALS);
-        uint32_t most = 0;
-        for (int i = 0; i < k; i++) {
-            l.s[i] = log.sig[n + i];
-            most = std::max(most, l.s[i].words);
-        }
-        if (!k) l.s[0] = RangeSignal{nullptr, 0, 1};
-        hipLaunchKernelGGL(k_range_result, dim3(most < 4096 ? 1 : 8, std::max(k, 1)), dim3(256), 0, s, flag, l, out);
+        RangeList l{};
+        const int n = range_list(log, from, &l);
+        hipLaunchKernelGGL(k_range_result, dim3(n), dim3(256), 0, s, flag, l, out);
         VCHK(hipGetLastError());
-        n += k;
-    } while (n < log.sig.size());
+        from += RANGE_SIGNALS;
+    } while (from < log.sig.size());
     return hipSuccess;
 }
 
@@ -1044,7 +1063,7 @@ int dec_tf_rows(const DecoderDev &d, size_t part_floats)
 // [voc_init.ic][L] (channel-first f32).  bufs: four buffers of the workspace
 // other than sig's.
 hipError_t enqueue_vocos(const DecoderDev &d, const DecoderWs &ws, const float *sig, float *const bufs[4], int L, int64_t cut,
-                         float *audio, bool fuse, RangeLog &log, hipStream_t s)
+                         float *audio, bool fuse, RangeLog &log, int32_t *out_of_range, hipStream_t s)
 {
     uint8_t *sn = (uint8_t *)bufs[0], *t1 = (uint8_t *)bufs[1];
     float *x = bufs[2], *last = bufs[3];
@@ -1115,9 +1134,13 @@ hipError_t enqueue_vocos(const DecoderDev &d, const DecoderWs &ws, const float *
     }
     const int ch = d.n_voc ? d.voc[d.n_voc - 1].up.oc : d.voc_init.oc;
     const size_t lds = (size_t)(((d.out_k * ch + 3) & ~3) + (64 + (d.out_k - 1) * d.out_dil) * (ch + 4)) * sizeof(float);
-    hipLaunchKernelGGL(k_out_rows<7>, dim3((L + 63) / 64), dim3(256), lds, s, last, ch, L, d.out_w, d.out_b, d.out_dil, cut,
-                       audio);
-    return hipGetLastError();
+    RangeList l{};
+    const int nout = (L + 63) / 64, nr = out_of_range ? range_list(log, 0, &l) : 0;
+    hipLaunchKernelGGL(k_out_rows<7>, dim3(nout + nr), dim3(256), lds, s, last, ch, L, d.out_w, d.out_b, d.out_dil, cut, audio,
+                       nout, ws.range_flag, l, out_of_range);
+    VCHK(hipGetLastError());
+    if (!out_of_range || log.sig.size() <= RANGE_SIGNALS) return hipSuccess;
+    return enqueue_range_result(log, RANGE_SIGNALS, ws.range_flag, out_of_range, s);
 }
 
 // Whether enqueue_vocos runs a decoder's shapes.

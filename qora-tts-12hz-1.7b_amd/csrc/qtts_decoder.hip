@@ -1473,8 +1473,7 @@ hipError_t enqueue_decode(const DecoderDev &d, const DecoderWs &ws, const uint32
     }
     if (d.vocos_rows && !ws.f32 && dec_x3()) {
         float *const bufs[4] = {ws.c, ws.d, ws.e, other};
-        DCHK(enqueue_vocos(d, ws, sig, bufs, L, cut, audio, dec_fuse_voc(), log, s));
-        return out_of_range ? enqueue_range_result(log, ws.range_flag, out_of_range, s) : hipSuccess;
+        return enqueue_vocos(d, ws, sig, bufs, L, cut, audio, dec_fuse_voc(), log, out_of_range, s);
     }
     // 5. Vocos: init conv with the first block's pre-snake (or the final
     // snake) fused
@@ -1533,7 +1532,7 @@ hipError_t enqueue_decode(const DecoderDev &d, const DecoderWs &ws, const uint32
     hipLaunchKernelGGL(k_out_conv, dim3((L + 255) / 256), dim3(256), 0, s, sn, ch, L, d.out_w, d.out_b, d.out_k,
                        d.out_dil, cut, audio);
     DCHK(hipGetLastError());
-    return out_of_range ? enqueue_range_result(log, ws.range_flag, out_of_range, s) : hipSuccess;
+    return out_of_range ? enqueue_range_result(log, 0, ws.range_flag, out_of_range, s) : hipSuccess;
 }
 
 // Algorithmic floating-point operations of enqueue_decode over T frames:

@@ -234,6 +234,7 @@ struct RangeSignal {
 constexpr int RANGE_SIGNALS = 64;
 struct RangeList {
     RangeSignal s[RANGE_SIGNALS];
+    int32_t blocks;                       // workgroups a signal
 };
 struct RangeLog {
     float *next, *end;
@@ -370,12 +371,12 @@ int dec_tf_rows(const DecoderDev &d, size_t part_floats);
 hipError_t enqueue_dec_tf(const DecoderDev &d, const DecoderWs &ws, const float *in, float *out, float *const bufs[4], int T,
                           RangeLog &log, hipStream_t s);
 size_t dec_range_words(const DecoderDev &d, int64_t T);
-hipError_t enqueue_range_result(const RangeLog &log, const int32_t *flag, int32_t *out, hipStream_t s);
+hipError_t enqueue_range_result(const RangeLog &log, size_t from, const int32_t *flag, int32_t *out, hipStream_t s);
 bool dec_attn_tiled(const DecoderDev &d);
 hipError_t enqueue_dec_attn_rows(const DecoderDev &d, const float *qkv, int T, uint8_t *ys, float *rm, hipStream_t s);
 hipError_t enqueue_snake_par(const float *alpha, const float *beta, int n, float *out, hipStream_t s);
 hipError_t enqueue_vocos(const DecoderDev &d, const DecoderWs &ws, const float *sig, float *const bufs[4], int L, int64_t cut,
-                         float *audio, bool fuse, RangeLog &log, hipStream_t s);
+                         float *audio, bool fuse, RangeLog &log, int32_t *out_of_range, hipStream_t s);
 double decode_flops(const DecoderDev &d, int T);
 hipError_t enqueue_gateup_timing(const TalkerDev &m, const Workspace &ws, int l, hipStream_t s);
 hipError_t enqueue_attn_timing(const TalkerDev &m, const Workspace &ws, int l, int slot, int64_t pos,
