@@ -127,13 +127,13 @@ struct DcFuse {
 // and, through lo, to 2^-25 absolute.  So every wave that stores split rows
 // notes its largest |value| (a plain store: atomics on words of several waves
 // lengthened each launch by 2 us), and workgroups beside the output
-// convolution's judge them (a launch of their own took 10 us, 1% of a short
+// convolution's test them (a launch of their own took 10 us, 1% of a short
 // chunk), over all channels of 64 positions (16 before a stride): a group that
 // reaches the maximum, or lies wholly below the normal f16 but is not zero, is
 // out, and the host repeats the decode on the f32 matrix path.  Quiet channels
 // beside loud ones of the same positions lose nothing that shows in the sums
 // over them.
-__device__ __forceinline__ void range_judge(const int32_t *flag, const RangeList &l, int32_t *out, int block)
+__device__ __forceinline__ void range_test(const int32_t *flag, const RangeList &l, int32_t *out, int block)
 {
     const RangeSignal g = l.s[block / l.blocks];
     // 2^b lanes a group of `per` words
@@ -154,7 +154,7 @@ __device__ __forceinline__ void range_judge(const int32_t *flag, const RangeList
 __global__ void __launch_bounds__(256)
 k_range_result(const int32_t *flag, RangeList l, int32_t *out)
 {
-    range_judge(flag, l, out, blockIdx.x);
+    range_test(flag, l, out, blockIdx.x);
 }
 
 __device__ __forceinline__ float dc_snake(float v, float ea, float eb) { return v + eb * snake_sin2(ea * v); }
@@ -711,7 +711,7 @@ k_out_rows(const float *x, int C, int L, const float *w, float bias, int dil, in
            const int32_t *flag, RangeList l, int32_t *out_of_range)
 {
     if ((int)blockIdx.x >= nout) {
-        range_judge(flag, l, out_of_range, blockIdx.x - nout);
+        range_test(flag, l, out_of_range, blockIdx.x - nout);
         return;
     }
     extern __shared__ float sm[];
